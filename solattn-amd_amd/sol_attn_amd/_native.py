@@ -251,6 +251,18 @@ PAIRING = True
 # paired: the three pairing kernels cost ~27 us, more than the union they
 # save on a short attention launch.
 PAIR_MIN_QUERY_BLOCKS = 8192
+# Nor are launches whose keys keep one query block per workgroup
+# (one_block_launch in csrc/sol_internal.h): K and V bytes per head up to this.
+ONE_BLOCK_KEY_BYTES = 16 << 20
+
+
+def _pairs(b, nq, nk, h, d):
+    """Whether a call's attention launch pairs query blocks (a forced
+    WORKGROUP_FORM or ROUTE_PREPASS "always" leaves the size rule aside)."""
+    if not PAIRING or b * h * -(-nq // BLOCK) < PAIR_MIN_QUERY_BLOCKS:
+        return False
+    return (WORKGROUP_FORM != 0 or ROUTE_PREPASS == "always"
+            or -(-nk // BLOCK) * BLOCK * d * 4 > ONE_BLOCK_KEY_BYTES)
 
 
 def _pair_buffers(q, rows, min_blocks):
@@ -528,8 +540,10 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
     plain = (rows is None and keys is None and key_lengths is None and not debug and qk_precision == "bf16"
              and threshold_estimator == "diagonal_covariance" and WORKGROUP_FORM == 0
              and ROUTE_PREPASS != "always")
-    if (ALL_IN and plain and protection is None and out is None and SELF_POOLING and SPLIT_SINKS
-            and (not PAIRING or q.shape[0] * q.shape[2] * -(-q.shape[1] // BLOCK) < PAIR_MIN_QUERY_BLOCKS)):
+    b, nq = rows.shape if rows is not None else q.shape[:2]
+    nk = keys.shape[1] if keys is not None else k.shape[1]
+    pairs = _pairs(b, nq, nk, *q.shape[-2:])
+    if ALL_IN and plain and protection is None and out is None and SELF_POOLING and SPLIT_SINKS and not pairs:
         # No pairing pass: pooling and attention in one C-ABI call.
         return _all_in(q, k, v, float(scale), float(beta), int(local), int(kv_sink), int(q_sink), stats)
     stream = _stream(q.device)
@@ -539,8 +553,8 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
         out, counts, _ = attend(q, _self_pooled(k, v), scale, beta, local, kv_sink, q_sink, protection,
                                 out=out, stats=stats, stream=stream, strides=None)
         return out, counts
-    strides, pairing, means = _UNSET, None, None
-    if PAIRING and OVERLAP_PAIRING:
+    strides, pairing, means = _UNSET if pairs else None, None, None
+    if pairs and OVERLAP_PAIRING:
         # Buffers come from the caller's stream and stay referenced until the
         # join below, so no other allocation can reuse them while the side
         # stream still works on them.

@@ -28,31 +28,123 @@
 // The dense control streams every exact tile, 128 queries per workgroup
 // (4 waves x 32 queries, full 64-key tiles per wave).
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_common.h"
 
 namespace sol {
 
 namespace {
+// How a tile meets its LDS slots (tile_attend's Step).
+// RingStep: the tile's slot stays untouched while it is attended; the DMA of
+// a later tile goes to another slot, its rounds spread over the score
+// products.
+template <typename Refill>
+struct RingStep {
+  static constexpr bool kOneSlot = false;
+  const Refill& refill;
+};
+
+template <typename Refill>
+__device__ __forceinline__ RingStep<Refill> ring_step(const Refill& refill) {
+  return {refill};
+}
+
+// SlotStep: one K slot and one V slot (slot_stream).  The next tile's K rows
+// are DMA'd into the K slot once every wave holds its last K fragments (after
+// half 0's score products), its V rows into the V slot once every wave holds
+// its last V fragments (after half 0's P V products): each DMA has about half
+// a tile's time to arrive, and a workgroup holds 32 KB of LDS at head_dim 128
+// instead of 64.  k0: half 0's K fragments, read at the end of the previous
+// step.  frag(t, ks): this lane's K fragment from global memory (the uncommon
+// second look at a half's raw scores, after its slot may have been refilled).
+template <int D, typename Refill, typename Frag>
+struct SlotStep {
+  static constexpr bool kOneSlot = true;
+  const Refill& refill;  // the next tile's
+  Frag frag;
+  u32x4 (&k0)[Shape<D>::KT];
+  // Part k of N of the K (V) rounds.
+  template <int N>
+  __device__ __forceinline__ void k_rounds(int k) const {
+    constexpr int H = Refill::kRounds / 2;
+#pragma unroll
+    for (int r = k * H / N; r < (k + 1) * H / N; ++r) refill.round(r);
+  }
+  template <int N>
+  __device__ __forceinline__ void v_rounds(int k) const {
+    constexpr int H = Refill::kRounds / 2;
+#pragma unroll
+    for (int r = k * H / N; r < (k + 1) * H / N; ++r) refill.round(H + r);
+  }
+};
+
+template <int D, typename Refill, typename Frag>
+__device__ __forceinline__ SlotStep<D, Refill, Frag> slot_step(const Refill& refill, Frag frag,
+                                                               u32x4 (&k0)[Shape<D>::KT]) {
+  return {refill, frag, k0};
+}
+
+// For steps with the max-pass softmax, which never look again.
+struct NoFrag {
+  __device__ __forceinline__ u32x4 operator()(int, int) const { return zero_u32x4(); }
+};
+
+// K fragments of key block j of (entry b, head h) from global memory, as
+// FragLane::k reads them from the LDS tile: k_fragments(...)(j)(t, ks).
+template <int D, bool KT>
+__device__ __forceinline__ auto k_fragments(const AttnParams& p, int b, int h, int col, int hh) {
+  const uint16_t* base = KT ? p.tiles + (int64_t(b) * p.H + h) * p.NKB * Shape<D>::TILE
+                            : p.k.base + int64_t(b) * p.k.sb + int64_t(h) * p.k.sh;
+  const int64_t st = p.k.st;
+  const int tk = p.Tk;
+  return [=](int j) {
+    return [=](int t, int ks) {
+      const int c = fresh(col), x = fresh(hh);
+      if constexpr (KT) {
+        return load16(base + int64_t(j) * Shape<D>::TILE + (c + 32 * t) * D +
+                      (TileLayout<D>::k_lane_xor(c, x) ^ (16 * ks)));
+      } else {
+        const int row = ((j + 1) * kBlock <= tk ? j * kBlock : tk - kBlock) + 32 * t + c;
+        return load16(base + int64_t(row) * st + 16 * ks + 8 * x);
+      }
+    };
+  };
+}
+
+// Every DMA of this wave has landed and its LDS reads have returned, in every
+// wave of the workgroup.
+__device__ __forceinline__ void slot_barrier() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // One 64-key tile, software-pipelined over its two 32-key halves inside the
 // wave so that the VALU softmax work overlaps the MFMAs:
-//   chunk 0        half 0's K reads
+//   chunk 0        half 0's K reads (RingStep; a SlotStep has them already)
 //   chunks 1..KT   half 0's score MFMAs; half 1's K reads
+//   [SlotStep: the K slot is free, V has landed]
 //   next KT        half 1's score MFMAs; half 0's softmax; half 0's V^T reads
 //   [rescale]
 //   next 2 DT      half 0's P V MFMAs; half 1's softmax; half 1's V^T reads
+//   [SlotStep: the V slot is free, the next K has landed: its half 0's reads]
 //   [rescale]      half 1's P V MFMAs
-// The refill's DMA rounds are spread over the 2 KT score chunks.  Scores
+// A RingStep spreads its refill's DMA rounds over the 2 KT score chunks, a
+// SlotStep its K rounds over half 1's score chunks and its V rounds over half
+// 1's P V chunks.  FULL: the max-pass softmax from the start (HalfSoftmax, the
+// same results), for a SlotStep that may have to look at the raw scores again:
+// a state without any key yet.  Scores
 // start from bias(t) when BIASED (-inf drops a key, log2(len) / c adds a
 // centroid's ln(len) logit term), else from 0.  LATE: the bias (0 or -inf
 // only) is added once a half's products are done instead, which keeps it out
 // of the registers live across the score chain; the same values (x + 0 is x
 // for the nonzero-signed sums a chain from +0 gives, and -inf either way).
-template <int D, bool BIASED, typename Bias, typename Refill, bool LATE = false>
+template <int D, bool BIASED, typename Bias, typename Step, bool LATE = false, bool FULL = false>
 __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
                                             const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
-                                            Bias bias, const Refill& refill) {
+                                            Bias bias, const Step& step) {
   constexpr bool EARLY = BIASED && !LATE;
+  constexpr bool ONE = Step::kOneSlot;
+  static_assert(ONE || !FULL, "a ring's tile stays in LDS");
   auto late = [&](f32x16& x, int t) {
     if constexpr (LATE) {
       const f32x16 b = bias(t);
@@ -66,27 +158,39 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
   const uint32_t vbase = fl.v_base(buf);
   u32x4 k0[KT], k1[KT];
 #pragma unroll
-  for (int ks = 0; ks < KT; ++ks) k0[ks] = fl.k(buf, 0, ks);
-  // The raw scores of half t again (FastHalf::resolve), from the tile still in LDS.
+  for (int ks = 0; ks < KT; ++ks) {
+    if constexpr (ONE)
+      k0[ks] = step.k0[ks];
+    else
+      k0[ks] = fl.k(buf, 0, ks);
+  }
+  // The raw scores of half t again (FastHalf::resolve): from the tile still
+  // in LDS, or (SlotStep) from global memory.
   auto raw = [&](int t) {
-    const FragLane<D> fr(fresh(col), fresh(hh));
     f32x16 s = EARLY ? bias(t) : zero16();
+    if constexpr (ONE) {
 #pragma unroll
-    for (int ks = 0; ks < KT; ++ks) s = mfma32x32x16(as_bf16x8(fr.k(buf, t, ks)), qf[ks], s);
+      for (int ks = 0; ks < KT; ++ks) s = mfma32x32x16(as_bf16x8(step.frag(t, ks)), qf[ks], s);
+    } else {
+      const FragLane<D> fr(fresh(col), fresh(hh));
+#pragma unroll
+      for (int ks = 0; ks < KT; ++ks) s = mfma32x32x16(as_bf16x8(fr.k(buf, t, ks)), qf[ks], s);
+    }
     late(s, t);
     return s;
   };
-  FastHalf<D> h0, h1;
+  std::conditional_t<FULL, HalfSoftmax<D>, FastHalf<D>> h0, h1;
   h0.s = EARLY ? bias(0) : zero16();
   chunk_end();
 #pragma unroll
   for (int ks = 0; ks < KT; ++ks) {
     h0.s = mfma32x32x16(as_bf16x8(k0[ks]), qf[ks], h0.s);
     k1[ks] = fl.k(buf, 1, ks);
-    refill.template after_step<2 * KT>(ks);
+    if constexpr (!ONE) step.refill.template after_step<2 * KT>(ks);
     chunk_end();
   }
   late(h0.s, 0);
+  if constexpr (ONE) slot_barrier();
   u32x4 va[2][DT];
 #pragma unroll
   for (int ks = 0; ks < KT; ++ks) {
@@ -98,7 +202,10 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
       for (int f = 2 * (ks - KT / 2); f < 2 * (ks - KT / 2) + 2; ++f)
         va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT);
     }
-    refill.template after_step<2 * KT>(KT + ks);
+    if constexpr (ONE)
+      step.template k_rounds<KT>(ks);
+    else
+      step.refill.template after_step<2 * KT>(KT + ks);
     chunk_end();
   }
   h0.resolve(st, c, [&] { return raw(0); });
@@ -112,11 +219,17 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
     h1.template part<2 * DT>(f, st, c);
     chunk_end();
   }
+  if constexpr (ONE) slot_barrier();
   h1.resolve(st, c, [&] { return raw(1); });
 #pragma unroll
   for (int f = 0; f < 2 * DT; ++f) {
     const int c4 = f / DT, dt = f % DT;
     st.acc[dt] = mfma32x32x16(as_bf16x8(vb[c4][dt]), h1.pb(c4), st.acc[dt]);
+    if constexpr (ONE) {
+      step.k0[f] = fl.k(buf, 0, f);  // KT = 2 DT fragments
+      step.template v_rounds<2 * DT>(f);
+      chunk_end();
+    }
   }
 }
 
@@ -125,45 +238,53 @@ struct NoBias {
 };
 
 // A full exact block (every key present).
-template <int D, typename Refill>
+template <int D, bool FULL = false, typename Step>
 __device__ __forceinline__ void full_tile(State<D>& st, const uint16_t* buf,
                                           const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
-                                          const Refill& refill) {
-  tile_attend<D, false>(st, buf, qf, col, hh, c, NoBias{}, refill);
+                                          const Step& step) {
+  tile_attend<D, false, NoBias, Step, false, FULL>(st, buf, qf, col, hh, c, NoBias{}, step);
 }
 
 // The rows of the sequence's partial last block j that hold its tk - 64 j
 // keys: [64 - len, 64) when the block was DMA'd from rows shifted back to the
 // sequence's last 64 rows (SHIFTED), else [0, len) (zero-padded tiles).
-// Returned relative to this lane's rows, as the bounds a <= tile_row(t, e, 0)
+// A whole block's are all 64.  Returned relative to this lane's rows, as the bounds a <= tile_row(t, e, 0)
 // < z of the present keys.
 template <bool SHIFTED>
 __device__ __forceinline__ int2 tail_rows(int j, int tk, int hh) {
-  const int len = tk - j * kBlock;
+  const int len = min(kBlock, tk - j * kBlock);
   const int lo = SHIFTED ? kBlock - len : 0;
   return make_int2(fresh(lo - 4 * hh), fresh(lo + len - 4 * hh));
 }
 
-// Exact block j: a full block, or the partial last block, whose absent keys
-// start at -inf.  Only a stream's last exact tile can be that block.
-template <int D, bool SHIFTED, typename Refill>
+// The partial last block j, whose absent keys start at -inf.
+template <int D, bool SHIFTED, bool FULL = false, typename Step>
+__device__ __forceinline__ void tail_tile(State<D>& st, const uint16_t* buf, int j, int tk,
+                                          const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
+                                          const Step& step) {
+  const int2 present = tail_rows<SHIFTED>(j, tk, hh);
+  const auto absent = [&](int t) {
+    f32x16 bias;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = tile_row(t, e, 0);
+      bias[e] = row >= present.x && row < present.y ? 0.f : kNegInf;
+    }
+    return bias;
+  };
+  tile_attend<D, true, decltype(absent), Step, true, FULL>(st, buf, qf, col, hh, c, absent, step);
+}
+
+// Exact block j: a full block, or the partial last block.  Only a stream's
+// last exact tile can be that block.
+template <int D, bool SHIFTED, bool FULL = false, typename Step>
 __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, int j, int tk,
                                            const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
-                                           const Refill& refill) {
+                                           const Step& step) {
   if ((j + 1) * kBlock <= tk) {
-    full_tile<D>(st, buf, qf, col, hh, c, refill);
+    full_tile<D, FULL>(st, buf, qf, col, hh, c, step);
   } else {
-    const int2 present = tail_rows<SHIFTED>(j, tk, hh);
-    const auto absent = [&](int t) {
-      f32x16 bias;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = tile_row(t, e, 0);
-        bias[e] = row >= present.x && row < present.y ? 0.f : kNegInf;
-      }
-      return bias;
-    };
-    tile_attend<D, true, decltype(absent), Refill, true>(st, buf, qf, col, hh, c, absent, refill);
+    tail_tile<D, SHIFTED, FULL>(st, buf, j, tk, qf, col, hh, c, step);
   }
 }
 
@@ -171,10 +292,10 @@ __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, in
 // `approx` contribute logit q . Kc_j + ln(len_j) and value Vc_j: their scores
 // start at log2(len_j) / c (c = scale * log2(e)), the others at -inf.  Only
 // the lane's share of the row index is formed at run time.
-template <int D, typename Refill>
+template <int D, bool FULL = false, typename Step>
 __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf, int ct, uint64_t approx,
                                               int tk, const bf16x8 (&qf)[Shape<D>::KT], int col, int hh,
-                                              float c, const Refill& refill) {
+                                              float c, const Step& step) {
   const uint64_t lane_approx = approx >> (4 * hh);
   const float inv_c = 1.f / c;
   // Every block of the tile is whole unless it holds the sequence's partial
@@ -183,25 +304,22 @@ __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf,
   const bool whole_tile = kBlock * kBlock * (ct + 1) <= tk;
   const float whole = __builtin_amdgcn_logf(float(kBlock)) * inv_c;
   const int lane_tokens = tk - kBlock * (kBlock * ct + 4 * hh);  // keys from the lane's first block on
-  tile_attend<D, true>(st, buf, qf, col, hh, c,
-                       [&](int t) {
-                         f32x16 bias;
-                         if (whole_tile) {
+  const auto lengths = [&](int t) {
+    f32x16 bias;
+    if (whole_tile) {
 #pragma unroll
-                           for (int e = 0; e < 16; ++e)
-                             bias[e] = ((lane_approx >> tile_row(t, e, 0)) & 1u) ? whole : kNegInf;
-                         } else {
+      for (int e = 0; e < 16; ++e) bias[e] = ((lane_approx >> tile_row(t, e, 0)) & 1u) ? whole : kNegInf;
+    } else {
 #pragma unroll
-                           for (int e = 0; e < 16; ++e) {
-                             const int row = tile_row(t, e, 0);
-                             const int len = min(kBlock, lane_tokens - kBlock * row);
-                             bias[e] = ((lane_approx >> row) & 1u)
-                                           ? __builtin_amdgcn_logf(float(len)) * inv_c : kNegInf;
-                           }
-                         }
-                         return bias;
-                       },
-                       refill);
+      for (int e = 0; e < 16; ++e) {
+        const int row = tile_row(t, e, 0);
+        const int len = min(kBlock, lane_tokens - kBlock * row);
+        bias[e] = ((lane_approx >> row) & 1u) ? __builtin_amdgcn_logf(float(len)) * inv_c : kNegInf;
+      }
+    }
+    return bias;
+  };
+  tile_attend<D, true, decltype(lengths), Step, false, FULL>(st, buf, qf, col, hh, c, lengths, step);
 }
 
 // The quantised-QK experiment's exact tile: S^T = K8 Q8^T on the INT8 matrix
@@ -321,8 +439,7 @@ __device__ __forceinline__ void wait_ahead(int ahead) {
 // id) in order; the tile each reference names is the same for every thread,
 // while selected(ref) may differ between waves.  make(ref, lds) returns the
 // refill (TileRefill, Q8Refill) that DMAs tile ref into the LDS slot at lds.
-// R = 1: one slot, refilled after a barrier (latency
-// hidden by the other workgroups of the CU).  Two streams over the same ring
+// Two streams over the same ring
 // are separated by a barrier.  prologue() runs once the first tiles' DMA is
 // issued (or, for an empty stream, at once), before the first wait.
 // Selection predicate and the two tile consumers of a stream.
@@ -369,33 +486,14 @@ __device__ __forceinline__ void tile_stream(uint16_t* ring, int count, Next next
                                             Prologue prologue = {}) {
   using S = Shape<D>;
   constexpr int kRounds = decltype(make(0, 0u))::kRounds;
-  static_assert(R >= 1 && R <= 4 && (R & (R - 1)) == 0, "ring depth 1, 2 or 4");
-  static_assert(R < 2 || (R - 2) * kRounds <= 63, "vmcnt range");
+  static_assert(R == 2 || R == 4, "ring depth 2 or 4");
+  static_assert((R - 2) * kRounds <= 63, "vmcnt range");
   if (count <= 0) {
     prologue();
     return;
   }
   const uint32_t ring_lds = lds_address(ring);
-  if constexpr (R == 1) {
-    for (int i = 0; i < count; ++i) {
-      const int id = next();
-      make(id, ring_lds).all();
-      wait_vmcnt<0>();
-      ring_barrier();
-      if (i + 1 < count) {
-        if (runs.selected(id)) {
-          runs.hit(ring, id, NoRefill{});
-        } else {
-          runs.miss(ring, id, NoRefill{});
-        }
-      } else {
-        last(ring, id, NoRefill{});
-      }
-      lds_barrier();
-    }
-    return;
-  }
-  int ids[R > 1 ? R - 1 : 1];  // tiles i .. i+R-2 (uniform); shifted each iteration
+  int ids[R - 1];  // tiles i .. i+R-2 (uniform); shifted each iteration
 #pragma unroll
   for (int s = 0; s < R - 1; ++s) {
     ids[s] = s < count ? next() : 0;
@@ -434,6 +532,44 @@ __device__ __forceinline__ void tile_stream(uint16_t* ring, int count, Next next
   step(count - 1, last);
   // The last refills were issued after the last wait: drain them before the
   // ring is reused or the workgroup exits.
+  wait_vmcnt<0>();
+}
+
+// Streams `count` tiles through one K slot and one V slot (SlotStep).  The
+// tile at hand's K has landed when its step begins, and each step leaves the
+// next tile's K in the slot with half 0's fragments read.  While `first()`
+// holds a tile goes to full(id, refill, k0), then every tile to
+// fast(id, refill, k0), the last one to last(id, refill, k0); past the last
+// tile the refill names that tile again, into slots nobody reads.  first()
+// must be wave-uniform and, once false, stay false.
+template <int D, typename Next, typename Make, typename First, typename Full, typename Fast, typename Last>
+__device__ __forceinline__ void slot_stream(uint16_t* slot, int count, Next next, Make make, First first, Full full,
+                                            Fast fast, Last last, int col, int hh) {
+  constexpr int KT = Shape<D>::KT;
+  constexpr int kRounds = decltype(make(0, 0u))::kRounds;
+  if (count <= 0) return;
+  const uint32_t lds = lds_address(slot);
+  int id = next();
+  make(id, lds).all();
+  wait_vmcnt<kRounds / 2>();  // its K
+  lds_barrier();
+  u32x4 k0[KT];
+  {
+    const FragLane<D> fl(fresh(col), fresh(hh));
+#pragma unroll
+    for (int ks = 0; ks < KT; ++ks) k0[ks] = fl.k(slot, 0, ks);
+  }
+  int i = 0;
+  auto step = [&](auto&& fn) {
+    const int cur = id;
+    if (++i < count) id = next();
+    fn(cur, make(id, lds), k0);
+  };
+  while (i < count - 1 && first()) step(full);
+  while (i < count - 1) step(fast);
+  step(last);
+  // The last refills were issued after the last wait: drain them before the
+  // slots are reused or the workgroup exits.
   wait_vmcnt<0>();
 }
 
@@ -656,7 +792,7 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
   const int ntiles = (p.NQB + G - 1) / G;
   const int front = min(p.q_sink_blocks, ntiles);
   const int split_tiles = sink_split_tiles(p.splits, p.q_sink_blocks, G, front);
-  TileTask task = sol_task(blockIdx.x, ntiles, front, split_tiles, p.B * p.H, p.splits);
+  TileTask task = sol_task(blockIdx.x, ntiles, front, split_tiles, p.B * p.H, p.splits, p.flat);
   if (task.bh < 0) return;
   if (G == 2 && p.order && task.tile >= front)  // the order_kernel's deal of the regular tiles
     task.tile = front + p.order[int64_t(task.bh) * p.NQB + task.tile - front];
@@ -828,22 +964,30 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
           s_mask[g][w] = qbg < p.NQB ? p.mask[((head * p.NQB) + qbg) * p.NW + seg / 32 + w] : 0u;
         }
         __syncthreads();
-        auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
-          // Branch-free: a tile with no approximated block for this query
-          // block (or a query block past the end) has every score at -inf and
-          // adds nothing.
-          const uint64_t approx = live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
-          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, refill);
-        };
-        tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
-                              wave, lane);
+        // Branch-free: a tile with no approximated block for this query
+        // block (or a query block past the end) has every score at -inf and
+        // adds nothing.
+        if constexpr (R == 1) {
+          auto process = [&](int ct, const auto& refill, u32x4 (&k0)[S::KT]) {
+            centroid_tile<D, true>(st, ring, ct, tile_approx(s_mask[0], ct - ct0, r0, r1), tk, qf, col, hh, scale_log2,
+                                   slot_step<D>(refill, NoFrag{}, k0));
+          };
+          slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
+        } else {
+          auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
+            const uint64_t approx = live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
+            centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
+          };
+          tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
+                                wave, lane);
+        }
       } else {
         // Per tile: routing of the tile's 64 blocks for every query block of
         // the group -- wave w scores blocks 32 (w & 1) + (lane & 31) of query
         // block w >> 1 over feature half lane >> 5, the halves summed across
         // the lane pair -- into the LDS bitmask; a barrier publishes the mask;
         // then the approximated blocks' contributions.
-        auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
+        auto route = [&](const uint16_t* buf, int ct) {
           const int r = fresh(32 * qh + col);  // centroid row inside the tile
           const int j = kBlock * ct + r;
           bool sel = false;
@@ -855,11 +999,23 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
           // Branch-free: a tile with no approximated block for this query block
           // (or a query block past the end) has every score at -inf and adds
           // nothing.
-          const uint64_t approx = live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
-          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, refill);
+          return live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
         };
-        tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
-                              wave, lane);
+        if constexpr (R == 1) {
+          auto process = [&](int ct, const auto& refill, u32x4 (&k0)[S::KT]) {
+            const uint64_t approx = route(ring, ct);
+            centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
+                                   slot_step<D>(refill, NoFrag{}, k0));
+          };
+          slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
+        } else {
+          auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
+            const uint64_t approx = route(buf, ct);
+            centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
+          };
+          tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
+                                wave, lane);
+        }
       }
       lds_barrier();  // every wave is done with the ring's centroid tiles
     }
@@ -875,16 +1031,34 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
     const auto kv = kv_refills<D, NT, KT>(p, b, h, wave, lane);
     auto selected = [](int tag) { return (tag & 1) != 0; };
     auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
-    if constexpr (!Q8) {
+    if constexpr (R == 1) {
+      // One query block: every streamed tile is its own.  The last tile may be
+      // the partial block, and may be the only one.
+      static_assert(G == 1 && !Q8, "one-slot streams hold one query block's tiles");
+      auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
+      const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
+      slot_stream<D>(
+          ring, count, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
+          [&](int, const auto& refill, u32x4 (&k0)[S::KT]) {
+            full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k0));
+          },
+          [&](int tag, const auto& refill, u32x4 (&k0)[S::KT]) {
+            full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k0));
+          },
+          [&](int tag, const auto& refill, u32x4 (&k0)[S::KT]) {
+            tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k0));
+          },
+          col, hh);
+    } else if constexpr (!Q8) {
       auto hit = [&](const uint16_t* buf, int, const auto& refill) {
-        full_tile<D>(st, buf, qf, col, hh, scale_log2, refill);
+        full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
       };
       tile_stream<D, NT, R>(
           ring, count, cursor, [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); },
           tile_runs(selected, hit, miss),
           [&](const uint16_t* buf, int tag, const auto& refill) {
             if (tag & 1) {
-              exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, refill);
+              exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
             } else {
               refill.all();
             }
@@ -1245,7 +1419,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
         // without approximated blocks (a query-sink block's) is skipped.
         const uint64_t approx = tile_approx(s_mask, ct, 0, nkb);
         if (grp == 0 && approx != 0ull) {
-          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, refill);
+          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
         } else {
           refill.all();
         }
@@ -1270,7 +1444,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
     const auto kv = kv_refills<D, 128, KT>(p, b, h, wg, lane);
     auto selected = [](int tag) { return (tag & 1) != 0; };
     auto hit = [&](const uint16_t* buf, int, const auto& refill) {
-      full_tile<D>(st, buf, qf, col, hh, scale_log2, refill);
+      full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
     };
     auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
     tile_stream<D, 128, 2>(
@@ -1278,7 +1452,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
         [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); }, tile_runs(selected, hit, miss),
         [&](const uint16_t* buf, int tag, const auto& refill) {
           if (tag & 1) {
-            exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, refill);
+            exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
           } else {
             refill.all();
           }
@@ -1287,7 +1461,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
           if constexpr (POOL) {
             const uint64_t approx = tile_approx(s_mask, 0, 0, nkb);
             if (grp == 0 && approx != 0ull)
-              centroid_tile<D>(st, ctile, 0, approx, tk, qf, col, hh, scale_log2, NoRefill{});
+              centroid_tile<D>(st, ctile, 0, approx, tk, qf, col, hh, scale_log2, ring_step(NoRefill{}));
           }
         });
   }
@@ -1391,12 +1565,12 @@ __global__ __launch_bounds__(256, 2) void dense_attention_kernel(AttnParams p) {
   const float scale_log2 = p.scale_log2;
   auto always = [](int) { return true; };
   auto hit = [&](const uint16_t* buf, int, const auto& refill) {
-    full_tile<D>(st, buf, qf, col, hh, scale_log2, refill);
+    full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
   };
   tile_stream<D, NT, 2>(
       ring, p.NKB, RangeCursor{0}, kv_refills<D, NT, KT>(p, b, h, wave, lane), tile_runs(always, hit, hit),
       [&](const uint16_t* buf, int j, const auto& refill) {
-        exact_tile<D, !KT>(st, buf, j, tk, qf, col, hh, scale_log2, refill);
+        exact_tile<D, !KT>(st, buf, j, tk, qf, col, hh, scale_log2, ring_step(refill));
       },
       wave, lane);
   store_output<D>(p, b, h, q0 + myq, hh, st);
@@ -1534,35 +1708,30 @@ __global__ __launch_bounds__(kOrderThreads) void order_kernel(AttnParams p, int 
 
 // LDS ring depth of the SOL kernel.
 constexpr int kSolRing = 2;
-// Below this many two-block workgroups the launch leaves CUs idle (256 CUs x
-// 2 workgroups): such launches run one query block per workgroup instead,
-// which doubles the workgroups and has no union to stream.  Both forms give
-// bit-identical results (a wave's tiles, their order and its softmax state
-// do not depend on its partner).  AttnParams::workgroup_form 1 or 2 forces
-// one form (tests run both).
-constexpr int64_t kSmallLaunchGroups = 512;
-
+// One-block workgroups hold one K and one V slot (slot_stream).
+constexpr int kSlots1 = 1;
 template <int D, int G, bool SEG>
 void launch_sol_variant(const AttnParams& p, hipStream_t stream) {
   // Grid of sol_task: the sink-holding tiles of every head (p.splits
   // workgroups each), then balanced_task's.
   const int ntiles = (p.NQB + G - 1) / G, front = std::min(p.q_sink_blocks, ntiles);
   const int split_tiles = sink_split_tiles(p.splits, p.q_sink_blocks, G, front);
-  const unsigned grid = balanced_grid((split_tiles * (p.splits - 1) + front) * (p.B * p.H), p.B * p.H, ntiles - front);
+  const int F = (split_tiles * (p.splits - 1) + front) * (p.B * p.H);
+  const unsigned grid = p.flat ? flat_grid(F, p.B * p.H, ntiles - front) : balanced_grid(F, p.B * p.H, ntiles - front);
   // Key blocks from pooled tile pairs (p.tiles) or straight from K / V rows.
   if (p.tiles) {
     if (p.k8)
       hipLaunchKernelGGL((sol_attention_kernel<D, G, kSolRing, true, true, SEG>), dim3(grid), dim3(128 * G), 0,
                          stream, p);
     else
-      hipLaunchKernelGGL((sol_attention_kernel<D, G, kSolRing, false, true, SEG>), dim3(grid), dim3(128 * G), 0,
+      hipLaunchKernelGGL((sol_attention_kernel<D, G, G == 1 ? kSlots1 : kSolRing, false, true, SEG>), dim3(grid), dim3(128 * G), 0,
                          stream, p);
   } else {
     if (p.k8)
       hipLaunchKernelGGL((sol_attention_kernel<D, G, kSolRing, true, false, SEG>), dim3(grid), dim3(128 * G), 0,
                          stream, p);
     else
-      hipLaunchKernelGGL((sol_attention_kernel<D, G, kSolRing, false, false, SEG>), dim3(grid), dim3(128 * G), 0,
+      hipLaunchKernelGGL((sol_attention_kernel<D, G, G == 1 ? kSlots1 : kSolRing, false, false, SEG>), dim3(grid), dim3(128 * G), 0,
                          stream, p);
   }
 }
@@ -1616,9 +1785,12 @@ hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
       launch_small<64, 4>(p, stream);
     return hipGetLastError();
   }
-  int g = int64_t(p.B) * p.H * ((p.NQB + 1) / 2) < kSmallLaunchGroups ? 1 : 2;
+  // AttnParams::workgroup_form 1 or 2 forces one form (tests run both: results are bit-identical -- a wave's
+  // tiles, their order and its softmax state do not depend on its partner).
+  int g = one_block_launch(int64_t(p.B) * p.H, p.NQB, p.NKB, D) ? 1 : 2;
   if (p.workgroup_form == 1 || p.workgroup_form == 2) g = p.workgroup_form;
   AttnParams q = p;
+  q.flat = head_key_bytes(p.NKB, D) <= kFlatKeyBytes ? 1 : 0;
   q.order = nullptr;
   if (g == 2 && p.order && p.mask && p.force != 1 && p.splits == 1) {
     const int ntiles = (p.NQB + 1) / 2, front = std::min(p.q_sink_blocks, ntiles);

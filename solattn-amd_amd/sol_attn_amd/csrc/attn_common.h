@@ -66,6 +66,17 @@ __host__ __device__ inline unsigned balanced_grid(int F, int heads, int R) {
   return unsigned(kXcds * ((total + kXcds - 1) / kXcds));
 }
 
+// The other map (`flat`): XCD x takes one contiguous eighth of the list of
+// all heads' tiles, so its workgroups stay on one head (or few) from end to
+// end and that head's keys stay in its L2.
+__host__ __device__ inline int64_t flat_start(int64_t n, int x) { return n * x / kXcds; }
+
+// Workgroups of a flat launch of F front ids and `heads` x R regular tiles.
+__host__ __device__ inline unsigned flat_grid(int64_t F, int heads, int R) {
+  const int64_t T = int64_t(heads) * R;
+  return unsigned(kXcds * ((F + kXcds - 1) / kXcds + (T + kXcds - 1) / kXcds));
+}
+
 // SOL launches dispatch the first `front` query tiles of every (entry, head)
 // ahead of the rest, head-interleaved.  With query sinks those tiles hold the
 // sink query blocks, whose workgroups stream every key block and run several
@@ -74,9 +85,24 @@ __host__ __device__ inline unsigned balanced_grid(int F, int heads, int R) {
 // 128-token sinks: 251 -> 163 us).  The first `split_tiles` of them (<=
 // front) are `splits` workgroups each, one per key range (split_range), whose
 // partial states sol_merge_kernel combines.  The remaining tiles follow
-// balanced_task.
+// balanced_task, or with `flat` each XCD's eighth of the list.
 __device__ __forceinline__ TileTask sol_task(int i, int ntiles, int front, int split_tiles, int heads,
-                                             int splits) {
+                                             int splits, int flat) {
+  if (flat) {
+    const int x = i % kXcds, k = i / kXcds;
+    const int per = split_tiles * splits + (front - split_tiles);  // front ids per head
+    const int64_t F = int64_t(per) * heads, T = int64_t(ntiles - front) * heads;
+    const int nf = int(flat_start(F, x + 1) - flat_start(F, x));
+    if (k < nf) {
+      const int64_t j = flat_start(F, x) + k;
+      const int h = int(j / per), e = int(j % per);
+      if (e < split_tiles * splits) return TileTask{h, e / splits, e % splits};
+      return TileTask{h, split_tiles + e - split_tiles * splits};
+    }
+    const int64_t j = flat_start(T, x) + (k - nf);
+    if (j >= flat_start(T, x + 1)) return TileTask{-1, 0};
+    return TileTask{int(j / (ntiles - front)), front + int(j % (ntiles - front))};
+  }
   const int nsplit = split_tiles * heads * splits;
   if (i < nsplit) {
     const int j = i / heads;
@@ -474,6 +500,11 @@ struct HalfSoftmax {
   }
   // The B operand of the P V product for keys 16 c4 .. 16 c4 + 15 of the half.
   __device__ __forceinline__ bf16x8 pb(int c4) const { return pw[c4]; }
+  // After the last stage: acc follows the max if this half moved it.
+  template <typename Raw>
+  __device__ __forceinline__ void resolve(State<D>& st, float, Raw) {
+    if (rescale) rescale_acc<D>(st, alpha);
+  }
   // Part k of n (n = 4 or 8) of the stages.
   template <int N>
   __device__ __forceinline__ void part(int k, State<D>& st, float c) {

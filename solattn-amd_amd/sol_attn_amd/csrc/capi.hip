@@ -100,16 +100,16 @@ int64_t route_mask_bytes(int64_t batch, int64_t query_tokens, int64_t key_tokens
 // Key-range parts per query-sink tile of the SOL kernel (sol_task).  A
 // query-sink block selects every key block, so its workgroup streams all of
 // them and, in a launch of few workgroups, ends long after the rest.  Split:
-// launches of one-block workgroups (fewer than 512 query-block pairs over all
-// (entry, head) pairs, the default schedule's threshold) at finite beta, and
-// at beta = +inf (every other workgroup streams its protected blocks only)
+// launches of fewer than 512 query-block pairs over all (entry, head) pairs,
+// and one-block launches of at most 2,048 query blocks over at least 128 key
+// blocks (8,192 tokens x 16 heads 210 -> 188), at finite beta, and at beta = +inf (every other workgroup streams its protected blocks only)
 // launches of up to 8,192 query blocks (8 rounds of 512 two-block
 // workgroups).  Parts hold at least 16 key blocks, at most 8 parts, while
 // their partial states fit kSplitBytesMax.  Measured (us per call, 4 heads,
 // beta 1): 4,096 tokens 97 -> 60, 8,192 tokens 172 -> 108; at 2 x 4,096 x 16
-// heads beta +inf 109 -> 91, while beta 0 or 1 there gains nothing (the
-// launch is bound by its two rounds of workgroups, and the extra
-// workgroups and the merge cost 1-4%).  beta = -inf (every block exact),
+// heads beta +inf 109 -> 91, while beta 0 or 1 there (128 -> 137) and more
+// rounds of workgroups (8,192 x 24 heads 257 -> 270) lose: the other
+// workgroups fill the time, and the merge comes on top.  beta = -inf (every block exact),
 // fewer than two sink blocks and sinks over a quarter of the query blocks
 // are not split.
 constexpr int64_t kSplitBytesMax = int64_t(64) << 20;
@@ -120,12 +120,13 @@ int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t h
 }
 
 int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, int64_t head_dim) {
-  const bool one_block_groups = bh * ((nqb + 1) / 2) < 512;
+  const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
+                          (bh * nqb <= 2048 && nkb >= 128 && sol::one_block_launch(bh, nqb, nkb, head_dim));
   // Launches of the small kernel split every query block's chain inside its
   // workgroup instead.
   if (sol::small_key_split(bh * nqb, nkb, head_dim)) return 1;
   if (force == 1 || q_sink_blocks < 2 || 4 * q_sink_blocks > nqb || nkb > sol::kMaxKeyBlocks ||
-      !(one_block_groups || (force == 2 && bh * nqb <= 8192)))
+      !(few_groups || (force == 2 && bh * nqb <= 8192)))
     return 1;
   int64_t s = std::min<int64_t>(8, nkb / 16);
   while (s > 1 && split_bytes(bh, q_sink_blocks, s, head_dim) > kSplitBytesMax) --s;

@@ -103,6 +103,7 @@ struct AttnParams {
                        // null: the attention kernel routes tile by tile
   int NW;              // ceil(NKB / 32)
   const float* qc;     // [B, H, NQB, D] FP32 query-block means for route_kernel, or null (formed from Q)
+  int flat;            // workgroup map: 1 = one eighth of all heads' tiles per XCD (sol_task)
   int32_t* order;      // [B H, NQB] with mask: the regular query tiles of a two-block launch in
                        // the order order_kernel deals them to the XCDs, or null: tile order
 };
@@ -142,6 +143,37 @@ inline int small_key_split(int64_t blocks, int64_t nkb, int64_t head_dim) {
   const int ks = head_dim == 64 ? 4 : 2;
   return blocks <= kSmallBlocks && nkb <= kSmallChain * ks ? ks : 0;
 }
+
+// K and V bytes of one head's key blocks.
+inline int64_t head_key_bytes(int64_t nkb, int64_t head_dim) { return nkb * kBlock * head_dim * 4; }
+
+// One query block per workgroup (a K and a V slot each, four workgroups per
+// CU at head_dim 128) or two (a ring of two slots, the union of the pair's
+// blocks, two workgroups per CU); AttnParams::workgroup_form 0.  Two blocks
+// stream fewer bytes, but a wave idles on the tiles only its partner selected.
+// While the keys come from the L2s the idle waves cost more; past about 16 MB
+// of K and V per head the bytes do (more than the 4 MB L2s hold, at about 7
+// TB/s from beyond them).  Attention launches, one box, us, two blocks -> one,
+// flat map: 4,096 x 10,000 keys x 24 heads x D128 170 -> 138; 2 x 4,096 x 16
+// 103 -> 94; 16,384 x 8 x D64 200 -> 160; 24,576 x 8 x D128 565 -> 531 (video
+// field), 618 -> 541 (random); 32,768 x 8 945 -> 927, 1075 -> 982, x 24 heads
+// 2896 -> 2902; 40,960 x 8 1505 -> 1573, 1713 -> 1648; 65,536 x 8 3705 ->
+// 4585, at D64 (16 MB) 2077 -> 1995.  Launches of fewer than 512 pairs (256
+// CUs x 2 workgroups) would leave CUs idle with two.
+constexpr int64_t kOneBlockKeyBytes = int64_t(16) << 20;
+constexpr int64_t kSmallLaunchGroups = 512;
+inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_dim) {
+  return head_key_bytes(nkb, head_dim) <= kOneBlockKeyBytes || bh * ((nqb + 1) / 2) < kSmallLaunchGroups;
+}
+
+// The flat workgroup map (sol_task) keeps an XCD on its own heads, so a head's
+// keys are read into one or two L2s instead of eight: 4,096 x 10,000 keys x 24
+// heads 185 -> 138 us, 19,003 x 16 708 -> 632 (one block per workgroup).  With
+// K and V per head far beyond the L2 it gains nothing, and eight heads at a
+// time no longer fit the 256 MB memory-side cache: 40,960 x 8 heads (20 MB)
+// 1544 -> 1505, 49,152 (24 MB) 2264 -> 2258, 65,536 (32 MB) 3662 -> 3705,
+// 84,672 x 24 (43 MB) 17056 -> 18243 (two blocks).
+constexpr int64_t kFlatKeyBytes = int64_t(24) << 20;
 
 hipError_t launch_pool(const PoolParams& p, int D, hipStream_t stream);
 hipError_t launch_quantize_keys(const QuantParams& p, int D, hipStream_t stream);
