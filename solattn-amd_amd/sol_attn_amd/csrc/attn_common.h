@@ -451,10 +451,14 @@ __device__ __forceinline__ void rescale_acc(State<D>& st, float alpha) {
 // when some query's max exceeds it by more than kRescaleSlack.  Otherwise the
 // probabilities exp2(s c - m) may exceed 1 by up to 2^kRescaleSlack, which
 // FP32 sums and BF16 products carry at unchanged relative precision; acc and
-// den always share m, so O = acc / den is unaffected.  The common case has
+// den always share m, so O = acc / den is unaffected.  (A slack of 8 made a
+// half's sum, not its max, send it the long way round: 16 keys that score
+// alike, as those of one block do, pass 255 at p = 16.  At 16, block-smooth
+// inputs: 2 x 4,096 tokens x 16 heads 159 -> 131 us a call, the dense kernel
+// 271 -> 252, the same error against 64 bits.)  The common case has
 // no data-dependent branch, so a half's softmax can be spread between
 // matrix-core instructions.
-constexpr float kRescaleSlack = 8.f;
+constexpr float kRescaleSlack = 16.f;
 
 // Softmax of one 32-key half of raw scores s (absent keys -inf; c = scale *
 // log2(e)), in 8 stages that a caller places between MFMAs: max; the
@@ -516,14 +520,14 @@ struct HalfSoftmax {
 // Common case of HalfSoftmax without its max pass: the probabilities
 // p = exp2(s c - m) are formed against the running max m as it stands, and
 // the row sum tells whether that was what HalfSoftmax would have done.  If
-// no lane's sum exceeds 255 (or, before any key, 0), every p is below 2^8,
-// i.e. every s c - m < log2(255) < kRescaleSlack, so HalfSoftmax would not
+// no lane's sum exceeds 65,535 (or, before any key, 0), every p is below
+// 2^16, i.e. every s c - m < log2(65,535) < kRescaleSlack, so HalfSoftmax would not
 // have moved m and would have formed these same p, den += lsum, with acc
 // untouched: the results are bit-identical.  Otherwise `redo` is set (a
 // wave-uniform ballot) and the caller re-forms the half's raw scores and
 // runs HalfSoftmax on them (resolve).  The stages are:
 // 4 x 4 probabilities and the row sum; the redo ballot; BF16 packing; den.
-constexpr float kFastSumMax = 255.f;
+constexpr float kFastSumMax = 65535.f;
 
 template <int D>
 struct FastHalf {
