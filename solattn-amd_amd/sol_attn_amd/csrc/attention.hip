@@ -50,39 +50,40 @@ __device__ __forceinline__ RingStep<Refill> ring_step(const Refill& refill) {
   return {refill};
 }
 
-// SlotStep: one K slot and one V slot (slot_stream).  The next tile's K rows
-// are DMA'd into the K slot once every wave holds its last K fragments (after
-// half 0's score products), its V rows into the V slot once every wave holds
-// its last V fragments (after half 0's P V products): each DMA has about half
-// a tile's time to arrive, and a workgroup holds 32 KB of LDS at head_dim 128
-// instead of 64.  k0: half 0's K fragments, read at the end of the previous
-// step.  frag(t, ks): this lane's K fragment from global memory (the uncommon
-// second look at a half's raw scores, after its slot may have been refilled).
+// SlotStep: one K slot and one V slot (slot_stream).  A tile passes through
+// them into registers: all its K fragments are read while the previous tile's
+// half 1 P V products run, all its V fragments with half 1's score products,
+// and each slot's next DMA starts once every wave's reads have returned.  Each
+// DMA then has about three quarters of a tile's time to arrive (with the
+// fragments read only as they are used it had half, and a tile took twice the
+// DMA latency), and a workgroup holds 32 KB of LDS at head_dim 128 instead of
+// 64.  k: this tile's K fragments (half t at [t]), on return the next one's.
+// frag(t, ks): this lane's K fragment from global memory (the uncommon second
+// look at a half's raw scores, after its slot may have been refilled).
 template <int D, typename Refill, typename Frag>
 struct SlotStep {
   static constexpr bool kOneSlot = true;
+  static constexpr int kHalfRounds = Refill::kRounds / 2;  // K rounds, V rounds
   const Refill& refill;  // the next tile's
   Frag frag;
-  u32x4 (&k0)[Shape<D>::KT];
-  // Part k of N of the K (V) rounds.
+  u32x4 (&k)[2][Shape<D>::KT];
+  // Part i of N of the K (V) rounds.
   template <int N>
-  __device__ __forceinline__ void k_rounds(int k) const {
-    constexpr int H = Refill::kRounds / 2;
+  __device__ __forceinline__ void k_rounds(int i) const {
 #pragma unroll
-    for (int r = k * H / N; r < (k + 1) * H / N; ++r) refill.round(r);
+    for (int r = i * kHalfRounds / N; r < (i + 1) * kHalfRounds / N; ++r) refill.round(r);
   }
   template <int N>
-  __device__ __forceinline__ void v_rounds(int k) const {
-    constexpr int H = Refill::kRounds / 2;
+  __device__ __forceinline__ void v_rounds(int i) const {
 #pragma unroll
-    for (int r = k * H / N; r < (k + 1) * H / N; ++r) refill.round(H + r);
+    for (int r = i * kHalfRounds / N; r < (i + 1) * kHalfRounds / N; ++r) refill.round(kHalfRounds + r);
   }
 };
 
 template <int D, typename Refill, typename Frag>
 __device__ __forceinline__ SlotStep<D, Refill, Frag> slot_step(const Refill& refill, Frag frag,
-                                                               u32x4 (&k0)[Shape<D>::KT]) {
-  return {refill, frag, k0};
+                                                               u32x4 (&k)[2][Shape<D>::KT]) {
+  return {refill, frag, k};
 }
 
 // For steps with the max-pass softmax, which never look again.
@@ -112,25 +113,27 @@ __device__ __forceinline__ auto k_fragments(const AttnParams& p, int b, int h, i
   };
 }
 
-// Every DMA of this wave has landed and its LDS reads have returned, in every
-// wave of the workgroup.
-__device__ __forceinline__ void slot_barrier() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+// All but the newest N DMAs of every wave of the workgroup have landed.
+template <int N>
+__device__ __forceinline__ void landed_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // One 64-key tile, software-pipelined over its two 32-key halves inside the
 // wave so that the VALU softmax work overlaps the MFMAs:
-//   chunk 0        half 0's K reads (RingStep; a SlotStep has them already)
+//   chunk 0        half 0's K reads
 //   chunks 1..KT   half 0's score MFMAs; half 1's K reads
-//   [SlotStep: the K slot is free, V has landed]
 //   next KT        half 1's score MFMAs; half 0's softmax; half 0's V^T reads
 //   [rescale]
 //   next 2 DT      half 0's P V MFMAs; half 1's softmax; half 1's V^T reads
-//   [SlotStep: the V slot is free, the next K has landed: its half 0's reads]
 //   [rescale]      half 1's P V MFMAs
-// A RingStep spreads its refill's DMA rounds over the 2 KT score chunks, a
-// SlotStep its K rounds over half 1's score chunks and its V rounds over half
-// 1's P V chunks.  FULL: the max-pass softmax from the start (HalfSoftmax, the
+// A RingStep spreads its refill's DMA rounds over the 2 KT score chunks.  A
+// SlotStep has the K fragments already and reads all V^T fragments beside half
+// 1's score MFMAs; around it, four barriers:
+//   [every wave holds its K fragments]  half 0's scores; the next K's DMA
+//   [V has landed]                      half 1's scores; V^T reads
+//   [every wave holds its V fragments]  half 0's P V; the next V's DMA
+//   [the next K has landed]             half 1's P V; its K reads  FULL: the max-pass softmax from the start (HalfSoftmax, the
 // same results), for a SlotStep that may have to look at the raw scores again:
 // a state without any key yet.  Scores
 // start from bias(t) when BIASED (-inf drops a key, log2(len) / c adds a
@@ -159,10 +162,12 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
   u32x4 k0[KT], k1[KT];
 #pragma unroll
   for (int ks = 0; ks < KT; ++ks) {
-    if constexpr (ONE)
-      k0[ks] = step.k0[ks];
-    else
+    if constexpr (ONE) {
+      k0[ks] = step.k[0][ks];
+      k1[ks] = step.k[1][ks];
+    } else {
       k0[ks] = fl.k(buf, 0, ks);
+    }
   }
   // The raw scores of half t again (FastHalf::resolve): from the tile still
   // in LDS, or (SlotStep) from global memory.
@@ -181,53 +186,68 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
   };
   std::conditional_t<FULL, HalfSoftmax<D>, FastHalf<D>> h0, h1;
   h0.s = EARLY ? bias(0) : zero16();
+  if constexpr (ONE) lds_barrier();
   chunk_end();
 #pragma unroll
   for (int ks = 0; ks < KT; ++ks) {
     h0.s = mfma32x32x16(as_bf16x8(k0[ks]), qf[ks], h0.s);
-    k1[ks] = fl.k(buf, 1, ks);
-    if constexpr (!ONE) step.refill.template after_step<2 * KT>(ks);
+    if constexpr (ONE) {
+      step.template k_rounds<KT>(ks);
+    } else {
+      k1[ks] = fl.k(buf, 1, ks);
+      step.refill.template after_step<2 * KT>(ks);
+    }
     chunk_end();
   }
   late(h0.s, 0);
-  if constexpr (ONE) slot_barrier();
-  u32x4 va[2][DT];
+  if constexpr (ONE) landed_barrier<Step::kHalfRounds>();
+  u32x4 va[2][DT], vb[2][DT];
 #pragma unroll
   for (int ks = 0; ks < KT; ++ks) {
     if (ks == 0) h1.s = EARLY ? bias(1) : zero16();
     h1.s = mfma32x32x16(as_bf16x8(k1[ks]), qf[ks], h1.s);
     h0.template part<KT>(ks, st, c);
-    if (ks >= KT / 2) {  // two of half 0's 2 DT = KT V^T fragments per chunk
+    if constexpr (ONE) {  // fragments 2 ks, 2 ks + 1 of the two halves' 2 KT
 #pragma unroll
-      for (int f = 2 * (ks - KT / 2); f < 2 * (ks - KT / 2) + 2; ++f)
-        va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT);
-    }
-    if constexpr (ONE)
-      step.template k_rounds<KT>(ks);
-    else
+      for (int f = 2 * ks; f < 2 * ks + 2; ++f) {
+        if (f < KT)
+          va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT);
+        else
+          vb[(f - KT) / DT][f % DT] = fl.v(vbase, 1, (f - KT) / DT, f % DT);
+      }
+    } else {
+      if (ks >= KT / 2) {  // two of half 0's 2 DT = KT V^T fragments per chunk
+#pragma unroll
+        for (int f = 2 * (ks - KT / 2); f < 2 * (ks - KT / 2) + 2; ++f)
+          va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT);
+      }
       step.refill.template after_step<2 * KT>(KT + ks);
+    }
     chunk_end();
   }
   h0.resolve(st, c, [&] { return raw(0); });
   late(h1.s, 1);
-  u32x4 vb[2][DT];
+  if constexpr (ONE) lds_barrier();
 #pragma unroll
   for (int f = 0; f < 2 * DT; ++f) {
     const int c4 = f / DT, dt = f % DT;
     st.acc[dt] = mfma32x32x16(as_bf16x8(va[c4][dt]), h0.pb(c4), st.acc[dt]);
-    vb[c4][dt] = fl.v(vbase, 1, c4, dt);
+    if constexpr (ONE)
+      step.template v_rounds<2 * DT>(f);
+    else
+      vb[c4][dt] = fl.v(vbase, 1, c4, dt);
     h1.template part<2 * DT>(f, st, c);
     chunk_end();
   }
-  if constexpr (ONE) slot_barrier();
   h1.resolve(st, c, [&] { return raw(1); });
+  if constexpr (ONE) landed_barrier<Step::kHalfRounds>();
 #pragma unroll
   for (int f = 0; f < 2 * DT; ++f) {
     const int c4 = f / DT, dt = f % DT;
     st.acc[dt] = mfma32x32x16(as_bf16x8(vb[c4][dt]), h1.pb(c4), st.acc[dt]);
     if constexpr (ONE) {
-      step.k0[f] = fl.k(buf, 0, f);  // KT = 2 DT fragments
-      step.template v_rounds<2 * DT>(f);
+      step.k[0][f] = fl.k(buf, 0, f);  // KT = 2 DT fragments per half
+      step.k[1][f] = fl.k(buf, 1, f);
       chunk_end();
     }
   }
@@ -536,12 +556,11 @@ __device__ __forceinline__ void tile_stream(uint16_t* ring, int count, Next next
 }
 
 // Streams `count` tiles through one K slot and one V slot (SlotStep).  The
-// tile at hand's K has landed when its step begins, and each step leaves the
-// next tile's K in the slot with half 0's fragments read.  While `first()`
-// holds a tile goes to full(id, refill, k0), then every tile to
-// fast(id, refill, k0), the last one to last(id, refill, k0); past the last
-// tile the refill names that tile again, into slots nobody reads.  first()
-// must be wave-uniform and, once false, stay false.
+// tile at hand's K fragments are read (or in flight) when its step begins, its
+// V's DMA may still be.  While `first()` holds a tile goes to full(id, refill,
+// k), then every tile to fast(id, refill, k), the last one to last(id, refill,
+// k); past the last tile the refill names that tile again, into slots nobody
+// reads.  first() must be wave-uniform and, once false, stay false.
 template <int D, typename Next, typename Make, typename First, typename Full, typename Fast, typename Last>
 __device__ __forceinline__ void slot_stream(uint16_t* slot, int count, Next next, Make make, First first, Full full,
                                             Fast fast, Last last, int col, int hh) {
@@ -553,17 +572,19 @@ __device__ __forceinline__ void slot_stream(uint16_t* slot, int count, Next next
   make(id, lds).all();
   wait_vmcnt<kRounds / 2>();  // its K
   lds_barrier();
-  u32x4 k0[KT];
+  u32x4 k[2][KT];
   {
     const FragLane<D> fl(fresh(col), fresh(hh));
 #pragma unroll
-    for (int ks = 0; ks < KT; ++ks) k0[ks] = fl.k(slot, 0, ks);
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KT; ++ks) k[t][ks] = fl.k(slot, t, ks);
   }
   int i = 0;
   auto step = [&](auto&& fn) {
     const int cur = id;
     if (++i < count) id = next();
-    fn(cur, make(id, lds), k0);
+    fn(cur, make(id, lds), k);
   };
   while (i < count - 1 && first()) step(full);
   while (i < count - 1) step(fast);
@@ -818,11 +839,25 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
   const float scale_log2 = p.scale_log2;
 
   // 1. Q tiles -> LDS -> fragments.
-  for (int idx = tid; idx < G * kBlock * S::DC; idx += NT) {
-    const int r = idx / S::DC, c = idx % S::DC;
-    const int t = slot_block(qb0 + r / kBlock, p.NQB, stride) * kBlock + r % kBlock;
-    const u32x4 x = t < p.Tq ? load16(p.q.row(b, t, h) + 8 * c) : zero_u32x4();
-    *reinterpret_cast<u32x4*>(ring + r * S::KS + 8 * c) = x;
+  {
+    // Every load is issued (unconditionally, rows past the end re-reading the
+    // last one) before the first store that waits on one.
+    constexpr int QPT = G * kBlock * S::DC / NT;
+    static_assert(QPT * NT == G * kBlock * S::DC, "Q rows split evenly over the workgroup");
+    u32x4 x[QPT];
+    int t[QPT];
+#pragma unroll
+    for (int i = 0; i < QPT; ++i) {
+      const int r = (tid + i * NT) / S::DC;
+      t[i] = slot_block(qb0 + r / kBlock, p.NQB, stride) * kBlock + r % kBlock;
+    }
+#pragma unroll
+    for (int i = 0; i < QPT; ++i) x[i] = load16(p.q.row(b, min(t[i], p.Tq - 1), h) + 8 * ((tid + i * NT) % S::DC));
+#pragma unroll
+    for (int i = 0; i < QPT; ++i) {
+      const int r = (tid + i * NT) / S::DC, c = (tid + i * NT) % S::DC;
+      *reinterpret_cast<u32x4*>(ring + r * S::KS + 8 * c) = t[i] < p.Tq ? x[i] : zero_u32x4();
+    }
   }
   __syncthreads();
   bf16x8 qf[S::KT];
@@ -968,9 +1003,9 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
         // block (or a query block past the end) has every score at -inf and
         // adds nothing.
         if constexpr (R == 1) {
-          auto process = [&](int ct, const auto& refill, u32x4 (&k0)[S::KT]) {
+          auto process = [&](int ct, const auto& refill, u32x4 (&k)[2][S::KT]) {
             centroid_tile<D, true>(st, ring, ct, tile_approx(s_mask[0], ct - ct0, r0, r1), tk, qf, col, hh, scale_log2,
-                                   slot_step<D>(refill, NoFrag{}, k0));
+                                   slot_step<D>(refill, NoFrag{}, k));
           };
           slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
         } else {
@@ -1002,10 +1037,10 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
           return live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
         };
         if constexpr (R == 1) {
-          auto process = [&](int ct, const auto& refill, u32x4 (&k0)[S::KT]) {
+          auto process = [&](int ct, const auto& refill, u32x4 (&k)[2][S::KT]) {
             const uint64_t approx = route(ring, ct);
             centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
-                                   slot_step<D>(refill, NoFrag{}, k0));
+                                   slot_step<D>(refill, NoFrag{}, k));
           };
           slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
         } else {
@@ -1039,14 +1074,14 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
       const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
       slot_stream<D>(
           ring, count, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
-          [&](int, const auto& refill, u32x4 (&k0)[S::KT]) {
-            full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k0));
+          [&](int, const auto& refill, u32x4 (&k)[2][S::KT]) {
+            full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
           },
-          [&](int tag, const auto& refill, u32x4 (&k0)[S::KT]) {
-            full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k0));
+          [&](int tag, const auto& refill, u32x4 (&k)[2][S::KT]) {
+            full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k));
           },
-          [&](int tag, const auto& refill, u32x4 (&k0)[S::KT]) {
-            tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k0));
+          [&](int tag, const auto& refill, u32x4 (&k)[2][S::KT]) {
+            tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
           },
           col, hh);
     } else if constexpr (!Q8) {
