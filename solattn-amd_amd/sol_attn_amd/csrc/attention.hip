@@ -752,39 +752,88 @@ __device__ __forceinline__ float cutoff_value(const AttnParams& p, float lin0, f
   return (lin0 + lin1) + p.beta * sqrtf(p.cov ? fmaxf(quad, 0.f) : quad);
 }
 
-// Routing decision for key block j (row r of the centroid tile in LDS at
-// buf) of query block qb in entry b: the proxy Qc . Kc_j over this lane's
-// feature half (qm: the block's FP32 query mean), summed across the lane
-// pair, above the cutoff -- or a key sink, local or plan-protected block
-// (kernels.py:129-143).  Writes the diagnostics of row dbg_row.
+// The FP32 query mean of one feature as an exact sum of three BF16 terms (hi,
+// mid, lo: 8 significant bits each) in the routing operand rows qb [4][QB]:
+// row k the k-th term, row 3 zero.
 template <int D>
-__device__ __forceinline__ bool route_block(const AttnParams& p, const uint16_t* buf, const float* qm, float cut,
-                                            int r, int j, int b, int qb, int hh, int64_t dbg_row) {
-  using S = Shape<D>;
-  using TL = TileLayout<D>;
-  bool sel = false;
+constexpr int kRouteRow = D + 8;  // padded: rows on different banks
+
+template <int D>
+__device__ __forceinline__ void split_query_mean(uint16_t* qb, int f, float x) {
+  const uint16_t hi = f32_to_bf16_bits(x);
+  const float r1 = __fsub_rn(x, bf16_bits_to_f32(hi));
+  const uint16_t mid = f32_to_bf16_bits(r1);
+  qb[f] = hi;
+  qb[kRouteRow<D> + f] = mid;
+  qb[2 * kRouteRow<D> + f] = f32_to_bf16_bits(__fsub_rn(r1, bf16_bits_to_f32(mid)));
+  qb[3 * kRouteRow<D> + f] = 0;
+}
+
+// Lane 0 (and 4, 8, ...) of x from lane K of its quad.
+template <int K>
+__device__ __forceinline__ float quad_lane(float x) {
+  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), K * 0x55, 0xf, 0xf, true));
+}
+
+// Routing decisions of key blocks j0 .. j0 + 31 (rows 32 t .. of the centroid
+// tile in LDS at buf) for query block qb of entry b, as one bit each, on the
+// matrix cores: the proxies Qc . Kc_j against the three terms of Qc as three
+// columns of the B operand (the other columns are zero), exact BF16 products
+// summed in FP32, the three sums added up; above the cutoff -- or a key sink,
+// local or plan-protected block (kernels.py:129-143).  Only blocks of [lo, hi)
+// are kept.  Writes the diagnostics of row dbg_row.  A wave's 32 decisions
+// take 8 MFMAs and about 100 VALU operations at head_dim 128 (an FP32 dot
+// product per lane pair took 64 multiply-adds, as many unpackings and 24 LDS
+// reads; a centroid tile's step @@ROUTE@@).
+template <int D>
+__device__ __forceinline__ uint32_t route_word(const AttnParams& p, const uint16_t* buf, const uint16_t* qterms,
+                                               float cut, int t, int j0, int lo, int hi, int b, int qb, int lane,
+                                               int64_t dbg_row) {
+  constexpr int KT = Shape<D>::KT;
+  const int col = fresh(lane & 31), hh = fresh(lane >> 5);
+  uint32_t word = 0;
+  const uint32_t valid = uint32_t(bit_range64(lo - j0, min(hi - j0, 32)));
   if (p.force == 0) {
-    const int c0 = fresh(hh) * (S::DC / 2);  // first 16-byte chunk of this lane's feature half
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    const FragLane<D> fl(col, hh);
+    const uint16_t* qrow = qterms + min(col, 3) * kRouteRow<D> + 8 * hh;
+    f32x16 x = zero16();
 #pragma unroll
-    for (int c = 0; c < S::DC / 2; ++c) {
-      const int cc = c0 + c;
-      const u32x4 x = *reinterpret_cast<const u32x4*>(buf + TL::k_offset(r, cc));
+    for (int k0 = 0; k0 < KT; k0 += 4) {  // four steps' operands at a time
+      u32x4 kf[4], qf[4];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t w = x[e >> 1];
-        part[e & 3] = fmaf(qm[8 * cc + e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)), part[e & 3]);
+      for (int i = 0; i < 4; ++i) {
+        kf[i] = fl.k(buf, t, k0 + i);
+        qf[i] = *reinterpret_cast<const u32x4*>(qrow + 16 * (k0 + i));
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x = mfma32x32x16(as_bf16x8(kf[i]), as_bf16x8(qf[i]), x);
+      chunk_end();
     }
-    const float proxy = pair_sum((part[0] + part[1]) + (part[2] + part[3]));
-    sel = proxy > cut;
-    if (p.dbg_proxy && hh == 0) p.dbg_proxy[dbg_row + j] = proxy * p.scale;
+    uint32_t bits = 0;  // lanes 0 and 32: rows 8 (e / 4) + 4 hh + e % 4
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      x[e] = (x[e] + quad_lane<1>(x[e])) + quad_lane<2>(x[e]);
+      bits |= x[e] > cut ? 1u << (8 * (e >> 2) + (e & 3)) : 0u;
+    }
+    word = uint32_t(__builtin_amdgcn_readlane(bits, 0)) | (uint32_t(__builtin_amdgcn_readlane(bits, 32)) << 4);
+    if (p.dbg_proxy && col == 0)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = tile_row(0, e, hh);
+        if ((valid >> row) & 1u) p.dbg_proxy[dbg_row + j0 + row] = x[e] * p.scale;
+      }
   }
-  sel = sel || (p.local_blocks >= 0 && abs(j - qb) <= p.local_blocks) || j < p.kv_sink_blocks ||
-        qb < p.q_sink_blocks;
-  if (p.protection) sel = sel || p.protection[(int64_t(b) * p.NQB + qb) * p.NKB + j] != 0;
-  if (p.dbg_selected && hh == 0) p.dbg_selected[dbg_row + j] = sel ? 1 : 0;
-  return sel;
+  if (p.local_blocks >= 0) word |= uint32_t(bit_range64(qb - p.local_blocks - j0, min(qb + p.local_blocks + 1 - j0, 32)));
+  word |= uint32_t(bit_range64(0, min(p.kv_sink_blocks - j0, 32)));
+  if (qb < p.q_sink_blocks) word = ~0u;
+  const bool here = lane < 32 && ((valid >> (lane & 31)) & 1u);
+  if (p.protection) {
+    const bool on = here && p.protection[(int64_t(b) * p.NQB + qb) * p.NKB + j0 + lane] != 0;
+    word |= uint32_t(__builtin_amdgcn_ballot_w64(on));
+  }
+  word &= valid;
+  if (p.dbg_selected && here) p.dbg_selected[dbg_row + j0 + lane] = uint8_t((word >> lane) & 1u);
+  return word;
 }
 
 }  // namespace
@@ -797,8 +846,9 @@ __device__ __forceinline__ bool route_block(const AttnParams& p, const uint16_t*
 // The bound names 256 threads for both workgroup forms, so the one-block form
 // (128 threads) is held to the same budget (with its own 128-thread bound the
 // compiler moves values through AGPRs instead).
+// (Three at head_dim 64, whose registers allow it.)
 template <int D, int G, int R, bool Q8, bool KT, bool SEG>
-__global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
+__global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_attention_kernel(AttnParams p) {
   using S = Shape<D>;
   using TL = TileLayout<D>;
   constexpr int NT = 128 * G;
@@ -806,6 +856,7 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
   static_assert(R * S::TILE >= G * kBlock * S::KS, "Q staging must fit in the ring");
   __shared__ __align__(256) uint16_t ring[R * S::TILE];  // Q staging, then the tile ring
   __shared__ float s_qm[G][D];  // in-kernel routing: query means, partial sums, cutoffs
+  __shared__ __align__(16) uint16_t s_qb[G][4 * kRouteRow<D>];  // and the means' BF16 terms
   __shared__ float s_red[G][4];
   __shared__ float s_cut[G];
   __shared__ uint32_t s_mask[G][kMaskWords];
@@ -921,6 +972,7 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
     if (lt < D) {
       km.finish(p);
       const float qm = s_qm[qg][lt];
+      split_query_mean<D>(s_qb[qg], lt, qm);
       a = qm * km.mu;
       if (p.cov) {
         // Full covariance: this feature's term of Qc^T cov Qc.  cov is
@@ -1018,18 +1070,17 @@ __global__ __launch_bounds__(256, 2) void sol_attention_kernel(AttnParams p) {
         }
       } else {
         // Per tile: routing of the tile's 64 blocks for every query block of
-        // the group -- wave w scores blocks 32 (w & 1) + (lane & 31) of query
-        // block w >> 1 over feature half lane >> 5, the halves summed across
-        // the lane pair -- into the LDS bitmask; a barrier publishes the mask;
-        // then the approximated blocks' contributions.
+        // the group (wave w: rows 32 (w & 1) .. +31 for query block w >> 1)
+        // into the LDS bitmask; a barrier publishes the mask; then the
+        // approximated blocks' contributions.
         auto route = [&](const uint16_t* buf, int ct) {
-          const int r = fresh(32 * qh + col);  // centroid row inside the tile
-          const int j = kBlock * ct + r;
-          bool sel = false;
-          if (live && j >= seg + r0 && j < seg + r1)
-            sel = route_block<D>(p, buf, s_qm[qg], s_cut[qg], r, j, b, qb, hh, dbg_row);
-          const uint64_t bal = __ballot(sel);
-          if (lane == 0) s_mask[qg][2 * (ct - ct0) + qh] = uint32_t(bal);
+          if (live) {
+            const uint32_t word = route_word<D>(p, buf, s_qb[qg], s_cut[qg], qh, kBlock * ct + 32 * qh, seg + r0,
+                                                seg + r1, b, qb, lane, dbg_row);
+            if (lane == 0) s_mask[qg][2 * (ct - ct0) + qh] = word;
+          } else if (lane == 0) {
+            s_mask[qg][2 * (ct - ct0) + qh] = 0u;
+          }
           lds_barrier();  // publishes the mask words
           // Branch-free: a tile with no approximated block for this query block
           // (or a query block past the end) has every score at -inf and adds
@@ -1219,6 +1270,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
   // first two); Q staging and the pooled centroid tile alias them early on.
   __shared__ __align__(256) uint16_t ring[2 * KS * S::TILE];
   __shared__ float s_qm[D];
+  __shared__ __align__(16) uint16_t s_qb[4 * kRouteRow<D>];  // its BF16 terms (route_word)
   __shared__ float s_red[4];
   __shared__ float s_mom[2][POOL ? D : 1];  // pooled key mean, variance
   __shared__ uint32_t s_mask[kMaskWords];
@@ -1380,6 +1432,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
     float a = 0.f, g = 0.f;
     if (tid < D) {
       const float qm = s_qm[tid];
+      split_query_mean<D>(s_qb, tid, qm);
       float mu;
       if (POOL) {
         mu = s_mom[0][tid];
@@ -1431,10 +1484,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       // its V rows); its contributions run in the exact stream's prologue,
       // over the first exact tiles' DMA (group 0's first slot is slot 0).
       if (!routed && grp == 0) {
-        const int j = fresh(myq);
-        const bool sel = j < nkb && route_block<D>(p, ctile, s_qm, cut, j, j, b, qb, hh, dbg_row);
-        const uint64_t bal = __ballot(sel);
-        if (lane == 0) s_mask[qh] = uint32_t(bal);
+        const uint32_t word = route_word<D>(p, ctile, s_qb, cut, qh, 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+        if (lane == 0) s_mask[qh] = word;
       }
       if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
       lds_barrier();  // publishes the mask words and the V centroids
@@ -1442,11 +1493,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
         if (!routed) {
           if (grp == 0) {
-            const int r = fresh(myq);  // centroid row inside the tile
-            const int j = kBlock * ct + r;
-            const bool sel = j < nkb && route_block<D>(p, buf, s_qm, cut, r, j, b, qb, hh, dbg_row);
-            const uint64_t bal = __ballot(sel);
-            if (lane == 0) s_mask[2 * ct + qh] = uint32_t(bal);
+            const uint32_t word = route_word<D>(p, buf, s_qb, cut, qh, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+            if (lane == 0) s_mask[2 * ct + qh] = word;
           }
           lds_barrier();  // publishes the mask words
         }
