@@ -555,40 +555,43 @@ __device__ __forceinline__ void tile_stream(uint16_t* ring, int count, Next next
   wait_vmcnt<0>();
 }
 
-// Streams `count` tiles through one K slot and one V slot (SlotStep).  The
-// tile at hand's K fragments are read (or in flight) when its step begins, its
-// V's DMA may still be.  While `first()` holds a tile goes to full(id, refill,
-// k), then every tile to fast(id, refill, k), the last one to last(id, refill,
-// k); past the last tile the refill names that tile again, into slots nobody
-// reads.  first() must be wave-uniform and, once false, stay false.
-template <int D, typename Next, typename Make, typename First, typename Full, typename Fast, typename Last>
-__device__ __forceinline__ void slot_stream(uint16_t* slot, int count, Next next, Make make, First first, Full full,
-                                            Fast fast, Last last, int col, int hh) {
-  constexpr int KT = Shape<D>::KT;
-  constexpr int kRounds = decltype(make(0, 0u))::kRounds;
-  if (count <= 0) return;
-  const uint32_t lds = lds_address(slot);
-  int id = next();
-  make(id, lds).all();
-  wait_vmcnt<kRounds / 2>();  // its K
+// K fragments of the tile in the K slot.
+template <int D>
+__device__ __forceinline__ void slot_fragments(const uint16_t* slot, u32x4 (&k)[2][Shape<D>::KT], int col, int hh) {
+  const FragLane<D> fl(fresh(col), fresh(hh));
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < Shape<D>::KT; ++ks) k[t][ks] = fl.k(slot, t, ks);
+}
+
+// Waits for the K of a whole tile's DMA (its V may still be in flight) and
+// reads its fragments.
+template <int D, int kRounds>
+__device__ __forceinline__ void slot_prime(const uint16_t* slot, u32x4 (&k)[2][Shape<D>::KT], int col, int hh) {
+  wait_vmcnt<kRounds / 2>();
   lds_barrier();
-  u32x4 k[2][KT];
-  {
-    const FragLane<D> fl(fresh(col), fresh(hh));
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int ks = 0; ks < KT; ++ks) k[t][ks] = fl.k(slot, t, ks);
-  }
+  slot_fragments<D>(slot, k, col, hh);
+}
+
+// Streams `count` tiles through one K slot and one V slot (SlotStep).  The
+// first tile `id` is primed: its K fragments are in k (or in flight), its V's
+// DMA is issued.  While `first()` holds a tile goes to full(id, refill), then
+// every tile to fast(id, refill), the last one to last(id, refill); past the
+// last tile the refill names that tile again, into slots nobody reads.
+// first() must be wave-uniform and, once false, stay false.
+template <typename Next, typename Make, typename First, typename Full, typename Fast, typename Last>
+__device__ __forceinline__ void slot_stream(uint32_t lds, int id, int count, Next& next, Make make, First first,
+                                            Full full, Fast fast, Last last) {
   int i = 0;
   auto step = [&](auto&& fn) {
     const int cur = id;
     if (++i < count) id = next();
-    fn(cur, make(id, lds), k);
+    fn(cur, make(id, lds));
   };
   while (i < count - 1 && first()) step(full);
   while (i < count - 1) step(fast);
-  step(last);
+  if (count > 0) step(last);
   // The last refills were issued after the last wait: drain them before the
   // slots are reused or the workgroup exits.
   wait_vmcnt<0>();
@@ -782,9 +785,9 @@ __device__ __forceinline__ float quad_lane(float x) {
 // summed in FP32, the three sums added up; above the cutoff -- or a key sink,
 // local or plan-protected block (kernels.py:129-143).  Only blocks of [lo, hi)
 // are kept.  Writes the diagnostics of row dbg_row.  A wave's 32 decisions
-// take 8 MFMAs and about 100 VALU operations at head_dim 128 (an FP32 dot
+// take 8 MFMAs and about 100 VALU operations at head_dim 128; an FP32 dot
 // product per lane pair took 64 multiply-adds, as many unpackings and 24 LDS
-// reads; a centroid tile's step @@ROUTE@@).
+// reads.
 template <int D>
 __device__ __forceinline__ uint32_t route_word(const AttnParams& p, const uint16_t* buf, const uint16_t* qterms,
                                                float cut, int t, int j0, int lo, int hi, int b, int qb, int lane,
@@ -853,8 +856,13 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
   using TL = TileLayout<D>;
   constexpr int NT = 128 * G;
   constexpr int kMaskWords = kMaxKeyBlocks / 32;
-  static_assert(R * S::TILE >= G * kBlock * S::KS, "Q staging must fit in the ring");
-  __shared__ __align__(256) uint16_t ring[R * S::TILE];  // Q staging, then the tile ring
+  // The tile ring; before it, Q staging.  R = 1 (one K and one V slot): the
+  // staging starts behind the K slot, where centroid tile 0's K rows arrive
+  // meanwhile.
+  constexpr int kStage = R == 1 ? TL::kElems : 0;
+  constexpr int kRing = R * S::TILE > kStage + G * kBlock * S::KS ? R * S::TILE : kStage + G * kBlock * S::KS;
+  __shared__ __align__(256) uint16_t ring[kRing];
+  uint16_t* const stage = ring + kStage;
   __shared__ float s_qm[G][D];  // in-kernel routing: query means, partial sums, cutoffs
   __shared__ __align__(16) uint16_t s_qb[G][4 * kRouteRow<D>];  // and the means' BF16 terms
   __shared__ float s_red[G][4];
@@ -888,6 +896,17 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
   const int nsplit = task.tile < split_tiles ? p.splits : 1;
   const int2 range = split_range(task.split, nsplit, nkb);
   const float scale_log2 = p.scale_log2;
+  const uint16_t* ctiles = p.ctiles + head * p.NCT * S::TILE;
+  const auto crefill = bf16_refills<D, NT>([=](int ct) { return ctiles + int64_t(ct) * S::TILE; }, wave, lane);
+  constexpr int kHalfRounds = TileRefill<D, NT>::kRounds / 2;
+  const uint32_t ring_lds = lds_address(ring);
+  if (R == 1 && p.force != 1 && range.y > range.x) {
+    // The first centroid tile's K rows travel while Q is staged and the
+    // cutoff formed (its V rows follow once the staging is dead).
+    const auto first = crefill(range.x / kBlock, ring_lds);
+#pragma unroll
+    for (int r = 0; r < kHalfRounds; ++r) first.round(r);
+  }
 
   // 1. Q tiles -> LDS -> fragments.
   {
@@ -907,14 +926,14 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
 #pragma unroll
     for (int i = 0; i < QPT; ++i) {
       const int r = (tid + i * NT) / S::DC, c = (tid + i * NT) % S::DC;
-      *reinterpret_cast<u32x4*>(ring + r * S::KS + 8 * c) = t[i] < p.Tq ? x[i] : zero_u32x4();
+      *reinterpret_cast<u32x4*>(stage + r * S::KS + 8 * c) = t[i] < p.Tq ? x[i] : zero_u32x4();
     }
   }
   __syncthreads();
   bf16x8 qf[S::KT];
   const int myq = 32 * qh + col;  // query inside the block
   {
-    const uint16_t* qrow = ring + (qg * kBlock + myq) * S::KS;
+    const uint16_t* qrow = stage + (qg * kBlock + myq) * S::KS;
 #pragma unroll
     for (int ks = 0; ks < S::KT; ++ks)
       qf[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(qrow + ks * 16 + 8 * hh));
@@ -925,7 +944,7 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
   i32x4 q8[Q8 ? D / 32 : 1];
   float csq = 0.f;  // c s_q
   if constexpr (Q8) {
-    const uint16_t* qrow = ring + (qg * kBlock + myq) * S::KS;
+    const uint16_t* qrow = stage + (qg * kBlock + myq) * S::KS;
     u32x4 raw[D / 32][2];
     float amax = 0.f;
 #pragma unroll
@@ -966,7 +985,7 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
     const int qlen = live ? min(kBlock, p.Tq - qb * kBlock) : 1;
     KeyMoments<D> km;  // this thread's feature of the key moments, loads issued first
     if (lt < D) km.load(p, head, lt);
-    if (lt < D) s_qm[qg][lt] = query_mean<D>(ring + qg * kBlock * S::KS, qlen, lt);
+    if (lt < D) s_qm[qg][lt] = query_mean<D>(stage + qg * kBlock * S::KS, qlen, lt);
     __syncthreads();
     float a = 0.f, g = 0.f;
     if (lt < D) {
@@ -985,11 +1004,8 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
         g = qm * qm * km.var;
       }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      a += __shfl_xor(a, off);
-      g += __shfl_xor(g, off);
-    }
+    a = wave_sum(a);
+    g = wave_sum(g);
     if (lane == 0) {
       s_red[qg][qh] = a;
       s_red[qg][2 + qh] = g;
@@ -1023,8 +1039,8 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
     // This workgroup's blocks of the segment, as bits of its masks.
     const int r0 = max(seg, range.x) - seg, r1 = min(seg + snkb, range.y) - seg;
     if (seg > 0) lds_barrier();  // every wave is done with the last segment's mask and ring slots
-    if (p.force == 1) {
-      // 3'. beta = -inf: every block exact, no centroid pass.
+    // Every block of the segment selected (beta = -inf), as masks.
+    auto select_all = [&] {
       const int nwords = (snkb + 31) / 32;
       for (int i = tid; i < G * nwords; i += NT) {
         const int g = i / nwords, w = i % nwords;
@@ -1033,153 +1049,162 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
                            ? (nvalid == 32 ? ~0u : ((1u << nvalid) - 1u)) : 0u;
       }
       __syncthreads();
-    } else {
-      // 3. Centroid pass over the segment's centroid tiles (the tiles holding
-      // blocks [r0, r1)).  Routing decisions come from route_kernel's masks
-      // (loaded into the LDS bitmask, bit j - seg, before the stream) or are
-      // formed here, tile by tile.
-      const uint16_t* ctiles = p.ctiles + head * p.NCT * S::TILE;
-      auto always = [](int) { return true; };
-      const int ct_lo = ct0 + r0 / kBlock;
-      const int nct = r1 > r0 ? ct0 + (r1 - 1) / kBlock - ct_lo + 1 : 0;
-      const auto crefill = bf16_refills<D, NT>([=](int ct) { return ctiles + int64_t(ct) * S::TILE; }, wave, lane);
-      if (routed) {
-        const int nwords = (snkb + 31) / 32;
-        for (int i = tid; i < G * nwords; i += NT) {
-          const int g = i / nwords, w = i % nwords;
-          const int qbg = slot_block(qb0 + g, p.NQB, stride);
-          s_mask[g][w] = qbg < p.NQB ? p.mask[((head * p.NQB) + qbg) * p.NW + seg / 32 + w] : 0u;
-        }
-        __syncthreads();
-        // Branch-free: a tile with no approximated block for this query
-        // block (or a query block past the end) has every score at -inf and
-        // adds nothing.
-        if constexpr (R == 1) {
-          auto process = [&](int ct, const auto& refill, u32x4 (&k)[2][S::KT]) {
-            centroid_tile<D, true>(st, ring, ct, tile_approx(s_mask[0], ct - ct0, r0, r1), tk, qf, col, hh, scale_log2,
-                                   slot_step<D>(refill, NoFrag{}, k));
-          };
-          slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
-        } else {
-          auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
-            const uint64_t approx = live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
-            centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
-          };
-          tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
-                                wave, lane);
-        }
-      } else {
-        // Per tile: routing of the tile's 64 blocks for every query block of
-        // the group (wave w: rows 32 (w & 1) .. +31 for query block w >> 1)
-        // into the LDS bitmask; a barrier publishes the mask; then the
-        // approximated blocks' contributions.
-        auto route = [&](const uint16_t* buf, int ct) {
-          if (live) {
-            const uint32_t word = route_word<D>(p, buf, s_qb[qg], s_cut[qg], qh, kBlock * ct + 32 * qh, seg + r0,
-                                                seg + r1, b, qb, lane, dbg_row);
-            if (lane == 0) s_mask[qg][2 * (ct - ct0) + qh] = word;
-          } else if (lane == 0) {
-            s_mask[qg][2 * (ct - ct0) + qh] = 0u;
-          }
-          lds_barrier();  // publishes the mask words
-          // Branch-free: a tile with no approximated block for this query block
-          // (or a query block past the end) has every score at -inf and adds
-          // nothing.
-          return live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
-        };
-        if constexpr (R == 1) {
-          auto process = [&](int ct, const auto& refill, u32x4 (&k)[2][S::KT]) {
-            const uint64_t approx = route(ring, ct);
-            centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
-                                   slot_step<D>(refill, NoFrag{}, k));
-          };
-          slot_stream<D>(ring, nct, RangeCursor{ct_lo}, crefill, [] { return true; }, process, process, process, col, hh);
-        } else {
-          auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
-            const uint64_t approx = route(buf, ct);
-            centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
-          };
-          tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill, tile_runs(always, process, process), process,
-                                wave, lane);
-        }
+    };
+    // route_kernel's masks of the segment, into the LDS bitmask (bit j - seg).
+    auto load_masks = [&] {
+      const int nwords = (snkb + 31) / 32;
+      for (int i = tid; i < G * nwords; i += NT) {
+        const int g = i / nwords, w = i % nwords;
+        const int qbg = slot_block(qb0 + g, p.NQB, stride);
+        s_mask[g][w] = qbg < p.NQB ? p.mask[((head * p.NQB) + qbg) * p.NW + seg / 32 + w] : 0u;
       }
-      lds_barrier();  // every wave is done with the ring's centroid tiles
-    }
-    if (live && p.counts && lt == 0)
-      for (int w = r0 / 32; w < (r1 + 31) / 32; ++w)
-        nsel += __builtin_popcount(s_mask[qg][w] & uint32_t(bit_range64(r0 - 32 * w, r1 - 32 * w)));
-
-    // 4. Exact pass over the union of the group's selected blocks of the
-    // segment.  Only the last segment's last tile can be the partial tail
-    // block.  Tile ids travel as tags 2 j + own-selection bit (UnionCursor).
+      __syncthreads();
+    };
+    // Approximated blocks of centroid tile ct (in LDS at buf) for the wave's
+    // query block: from the masks, or routed here -- the tile's 64 blocks for
+    // every query block of the group (wave w: rows 32 (w & 1) .. +31 for query
+    // block w >> 1) into the LDS bitmask, a barrier publishing it.  A tile
+    // with none (or a query block past the end) has every score at -inf and
+    // adds nothing.
+    auto approximated = [&](const uint16_t* buf, int ct) {
+      if (!routed) {
+        if (live) {
+          const uint32_t word = route_word<D>(p, buf, s_qb[qg], s_cut[qg], qh, kBlock * ct + 32 * qh, seg + r0,
+                                              seg + r1, b, qb, lane, dbg_row);
+          if (lane == 0) s_mask[qg][2 * (ct - ct0) + qh] = word;
+        } else if (lane == 0) {
+          s_mask[qg][2 * (ct - ct0) + qh] = 0u;
+        }
+        lds_barrier();  // publishes the mask words
+      }
+      return live ? tile_approx(s_mask[qg], ct - ct0, r0, r1) : 0ull;
+    };
+    auto count_selected = [&] {
+      if (live && p.counts && lt == 0)
+        for (int w = r0 / 32; w < (r1 + 31) / 32; ++w)
+          nsel += __builtin_popcount(s_mask[qg][w] & uint32_t(bit_range64(r0 - 32 * w, r1 - 32 * w)));
+    };
+    // The segment's centroid tiles (those holding blocks [r0, r1)).
+    const int ct_lo = ct0 + r0 / kBlock;
+    const int nct = p.force != 1 && r1 > r0 ? ct0 + (r1 - 1) / kBlock - ct_lo + 1 : 0;
+    // Exact pass: the union of the group's selected blocks of the segment.
+    // Only the last segment's last tile can be the partial tail block.  Tile
+    // ids travel as tags 2 j + own-selection bit (UnionCursor).
     UnionCursor<G> cursor{&s_mask[0][0], s_mask[qg], kMaskWords, r0, r1, seg};
-    const int count = cursor.count();
     const auto kv = kv_refills<D, NT, KT>(p, b, h, wave, lane);
-    auto selected = [](int tag) { return (tag & 1) != 0; };
-    auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
     if constexpr (R == 1) {
-      // One query block: every streamed tile is its own.  The last tile may be
-      // the partial block, and may be the only one.
+      // One query block: every streamed tile is its own, and the centroid
+      // tiles and the exact tiles are one stream (the last centroid tile's
+      // refill is the first exact tile).
       static_assert(G == 1 && !Q8, "one-slot streams hold one query block's tiles");
+      if (r1 <= r0) continue;
+      u32x4 k[2][S::KT];
       auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
+      int count, id;
+      if (p.force == 1) {
+        select_all();
+        count = cursor.count();
+        id = cursor();
+        make(id, ring_lds).all();
+        slot_prime<D, 2 * kHalfRounds>(ring, k, col, hh);
+      } else {
+        if (routed) load_masks();
+        const auto first = crefill(ct_lo, ring_lds);
+        if (si > 0) {
+          first.all();
+        } else {
+#pragma unroll
+          for (int r = kHalfRounds; r < 2 * kHalfRounds; ++r) first.round(r);
+        }
+        slot_prime<D, 2 * kHalfRounds>(ring, k, col, hh);
+        for (int ct = ct_lo; ct < ct_lo + nct - 1; ++ct)
+          centroid_tile<D, true>(st, ring, ct, approximated(ring, ct), tk, qf, col, hh, scale_log2,
+                                 slot_step<D>(crefill(ct + 1, ring_lds), NoFrag{}, k));
+        const int ct = ct_lo + nct - 1;
+        const uint64_t approx = approximated(ring, ct);
+        count = cursor.count();
+        id = cursor();  // with no selected block, a valid one that nobody attends
+        centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
+                               slot_step<D>(make(id, ring_lds), NoFrag{}, k));
+      }
+      count_selected();
       const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
-      slot_stream<D>(
-          ring, count, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
-          [&](int, const auto& refill, u32x4 (&k)[2][S::KT]) {
+      slot_stream(
+          ring_lds, id, count, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
+          [&](int, const auto& refill) {
             full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
           },
-          [&](int tag, const auto& refill, u32x4 (&k)[2][S::KT]) {
+          [&](int tag, const auto& refill) {
             full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k));
           },
-          [&](int tag, const auto& refill, u32x4 (&k)[2][S::KT]) {
+          [&](int tag, const auto& refill) {
             tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
-          },
-          col, hh);
-    } else if constexpr (!Q8) {
-      auto hit = [&](const uint16_t* buf, int, const auto& refill) {
-        full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
-      };
-      tile_stream<D, NT, R>(
-          ring, count, cursor, [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); },
-          tile_runs(selected, hit, miss),
-          [&](const uint16_t* buf, int tag, const auto& refill) {
-            if (tag & 1) {
-              exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
-            } else {
-              refill.all();
-            }
-          },
-          wave, lane);
+          });
     } else {
-      // Quantised QK: INT8 K tiles and their scales (the V tiles as in the
-      // BF16 stream).
-      const int8_t* k8 = p.k8 + head * p.NKB * K8Layout<D>::kBytes;
-      const float* k8s = p.k8_scale + head * p.NKB;
-      auto make = [=](int tag, uint32_t lds) {
-        const int j = tag >> 1;
-        return Q8Refill<D, NT, decltype(kv(0, 0u))>(k8 + int64_t(j) * K8Layout<D>::kBytes, lds, wave, lane,
-                                                    kv(j, lds));
-      };
-      auto hit = [&](const uint16_t* buf, int tag, const auto& refill) {
-        tile_attend_i8<D, false>(st, buf, q8, col, hh, csq * k8s[tag >> 1], int2{}, refill);
-      };
-      tile_stream<D, NT, R>(
-          ring, count, cursor, make, tile_runs(selected, hit, miss),
-          [&](const uint16_t* buf, int tag, const auto& refill) {
-            if (tag & 1) {
-              const int j = tag >> 1;
-              const float c8 = csq * k8s[j];
-              if ((j + 1) * kBlock <= tk)
-                tile_attend_i8<D, false>(st, buf, q8, col, hh, c8, int2{}, refill);
-              else
-                tile_attend_i8<D, true>(st, buf, q8, col, hh, c8, tail_rows<!KT>(j, tk, hh), refill);
-            } else {
-              refill.all();
-            }
-          },
-          wave, lane);
+      if (p.force == 1) {
+        // 3'. beta = -inf: every block exact, no centroid pass.
+        select_all();
+      } else {
+        // 3. Centroid pass.
+        if (routed) load_masks();
+        auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
+          const uint64_t approx = approximated(buf, ct);
+          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
+        };
+        tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill,
+                              tile_runs([](int) { return true; }, process, process), process, wave, lane);
+        lds_barrier();  // every wave is done with the ring's centroid tiles
+      }
+      count_selected();
+      // 4. Exact pass.
+      const int count = cursor.count();
+      auto selected = [](int tag) { return (tag & 1) != 0; };
+      auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
+      if constexpr (!Q8) {
+        auto hit = [&](const uint16_t* buf, int, const auto& refill) {
+          full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
+        };
+        tile_stream<D, NT, R>(
+            ring, count, cursor, [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); },
+            tile_runs(selected, hit, miss),
+            [&](const uint16_t* buf, int tag, const auto& refill) {
+              if (tag & 1) {
+                exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
+              } else {
+                refill.all();
+              }
+            },
+            wave, lane);
+      } else {
+        // Quantised QK: INT8 K tiles and their scales (the V tiles as in the
+        // BF16 stream).
+        const int8_t* k8 = p.k8 + head * p.NKB * K8Layout<D>::kBytes;
+        const float* k8s = p.k8_scale + head * p.NKB;
+        auto make = [=](int tag, uint32_t lds) {
+          const int j = tag >> 1;
+          return Q8Refill<D, NT, decltype(kv(0, 0u))>(k8 + int64_t(j) * K8Layout<D>::kBytes, lds, wave, lane,
+                                                      kv(j, lds));
+        };
+        auto hit = [&](const uint16_t* buf, int tag, const auto& refill) {
+          tile_attend_i8<D, false>(st, buf, q8, col, hh, csq * k8s[tag >> 1], int2{}, refill);
+        };
+        tile_stream<D, NT, R>(
+            ring, count, cursor, make, tile_runs(selected, hit, miss),
+            [&](const uint16_t* buf, int tag, const auto& refill) {
+              if (tag & 1) {
+                const int j = tag >> 1;
+                const float c8 = csq * k8s[j];
+                if ((j + 1) * kBlock <= tk)
+                  tile_attend_i8<D, false>(st, buf, q8, col, hh, c8, int2{}, refill);
+                else
+                  tile_attend_i8<D, true>(st, buf, q8, col, hh, c8, tail_rows<!KT>(j, tk, hh), refill);
+              } else {
+                refill.all();
+              }
+            },
+            wave, lane);
+      }
     }
-
   }  // segments
   if (nsplit > 1) {
     // Partial state of this key range: the record of row (tile, part,
@@ -1450,11 +1475,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
         g = qm * qm * (POOL ? s_mom[1][tid] : km.var);
       }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      a += __shfl_xor(a, off);
-      g += __shfl_xor(g, off);
-    }
+    a = wave_sum(a);
+    g = wave_sum(g);
     if (wave < 2 && lane == 0) {
       s_red[wave] = a;
       s_red[2 + wave] = g;

@@ -173,6 +173,22 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
 }
 
+// x plus x of the lane `N` back in its row of 16 lanes.
+template <int N>
+__device__ __forceinline__ float row_ror_sum(float x) {
+  return x + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x120 + N, 0xf, 0xf, true));
+}
+
+// Sum over the wave's 64 lanes, in every lane: the tree of xor shuffles 32, 16,
+// .. 1 (after step n the values repeat every n lanes, so a rotation inside the
+// row is the xor), in cross-lane moves instead of LDS permutes.
+__device__ __forceinline__ float wave_sum(float x) {
+  x = pair_sum(x);
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  return row_ror_sum<1>(row_ror_sum<2>(row_ror_sum<4>(row_ror_sum<8>(x))));
+}
+
 __device__ __forceinline__ bf16x8 pack8(const f32x16& s, int base) {
   u32x4 pb;
 #pragma unroll
