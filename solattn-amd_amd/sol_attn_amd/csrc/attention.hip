@@ -310,32 +310,31 @@ __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, in
 
 // Centroid tile ct: the block centroids 64 ct + r whose bit r is set in
 // `approx` contribute logit q . Kc_j + ln(len_j) and value Vc_j: their scores
-// start at log2(len_j) / c (c = scale * log2(e)), the others at -inf.  Only
-// the lane's share of the row index is formed at run time.
+// start at log2(len_j) / c (c = scale * log2(e)), the others at -inf.
 template <int D, bool FULL = false, typename Step>
 __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf, int ct, uint64_t approx,
                                               int tk, const bf16x8 (&qf)[Shape<D>::KT], int col, int hh,
                                               float c, const Step& step) {
-  const uint64_t lane_approx = approx >> (4 * hh);
   const float inv_c = 1.f / c;
-  // Every block of the tile is whole unless it holds the sequence's partial
-  // last block; whole blocks share one offset, log2(64) / c, computed as the
-  // per-block formula computes it at len 64.
-  const bool whole_tile = kBlock * kBlock * (ct + 1) <= tk;
+  // Every block is whole but the sequence's last one: whole blocks share one
+  // offset, log2(64) / c.  The approximated blocks are wave-uniform, so each
+  // element's choice is a lane mask formed on the scalar unit: rows r (lanes
+  // 0 .. 31) and r + 4 (lanes 32 .. 63).
+  const uint64_t bits = uniform64(approx);
   const float whole = __builtin_amdgcn_logf(float(kBlock)) * inv_c;
-  const int lane_tokens = tk - kBlock * (kBlock * ct + 4 * hh);  // keys from the lane's first block on
+  const int last = (tk - 1) / kBlock - kBlock * ct;           // the last block's row, if in this tile
+  const int len = tk - kBlock * (kBlock * ct + last);         // and its keys
   const auto lengths = [&](int t) {
     f32x16 bias;
-    if (whole_tile) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) bias[e] = ((lane_approx >> tile_row(t, e, 0)) & 1u) ? whole : kNegInf;
-    } else {
+    for (int e = 0; e < 16; ++e)
+      bias[e] = mask_select(row_mask(bits, tile_row(t, e, 0)), kNegInf, whole);
+    if (last < kBlock && len < kBlock) {
+      const int lr = fresh(last - 4 * hh);
+      const float part = __builtin_amdgcn_logf(float(len)) * inv_c;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = tile_row(t, e, 0);
-        const int len = min(kBlock, lane_tokens - kBlock * row);
-        bias[e] = ((lane_approx >> row) & 1u) ? __builtin_amdgcn_logf(float(len)) * inv_c : kNegInf;
-      }
+      for (int e = 0; e < 16; ++e)
+        if (tile_row(t, e, 0) == lr) bias[e] = bias[e] == kNegInf ? kNegInf : part;
     }
     return bias;
   };
@@ -772,71 +771,52 @@ __device__ __forceinline__ void split_query_mean(uint16_t* qb, int f, float x) {
   qb[3 * kRouteRow<D> + f] = 0;
 }
 
-// Lane 0 (and 4, 8, ...) of x from lane K of its quad.
-template <int K>
-__device__ __forceinline__ float quad_lane(float x) {
-  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), K * 0x55, 0xf, 0xf, true));
-}
-
-// Routing decisions of key blocks j0 .. j0 + 31 (rows 32 t .. of the centroid
-// tile in LDS at buf) for query block qb of entry b, as one bit each, on the
-// matrix cores: the proxies Qc . Kc_j against the three terms of Qc as three
-// columns of the B operand (the other columns are zero), exact BF16 products
-// summed in FP32, the three sums added up; above the cutoff -- or a key sink,
-// local or plan-protected block (kernels.py:129-143).  Only blocks of [lo, hi)
-// are kept.  Writes the diagnostics of row dbg_row.  A wave's 32 decisions
-// take 8 MFMAs and about 100 VALU operations at head_dim 128; an FP32 dot
-// product per lane pair took 64 multiply-adds, as many unpackings and 24 LDS
-// reads.
-template <int D>
-__device__ __forceinline__ uint32_t route_word(const AttnParams& p, const uint16_t* buf, const uint16_t* qterms,
-                                               float cut, int t, int j0, int lo, int hi, int b, int qb, int lane,
-                                               int64_t dbg_row) {
+// Routing decisions of key blocks j0 .. j0 + 31 for query block qb of entry b,
+// as one bit each, on the matrix cores: the three BF16 terms of Qc are rows 0,
+// 1, 2 of the A operand (the others are zero), the centroids the columns
+// (kfrag(ks): this lane's centroid j0 + lane % 32, features 16 ks + 8 (lane /
+// 32) .. + 7), so lane l < 32 ends with the three sums of centroid j0 + l --
+// exact BF16 products summed in FP32 -- in its first three elements.  Selected:
+// their sum above the cutoff -- or a key sink, local or plan-protected block
+// (kernels.py:129-143).  Only blocks of [lo, hi) are kept.  Writes the
+// diagnostics of row dbg_row.  At head_dim 128 a wave's 32 decisions are 8
+// MFMAs and a handful of VALU operations; as an FP32 dot product per lane pair
+// they were 64 multiply-adds, as many unpackings and 24 LDS reads.
+template <int D, typename KFrag>
+__device__ __forceinline__ uint32_t route_word(const AttnParams& p, KFrag kfrag, const uint16_t* qterms, float cut,
+                                               int j0, int lo, int hi, int b, int qb, int lane, int64_t dbg_row) {
   constexpr int KT = Shape<D>::KT;
-  const int col = fresh(lane & 31), hh = fresh(lane >> 5);
+  const int l = fresh(lane);
   uint32_t word = 0;
   const uint32_t valid = uint32_t(bit_range64(lo - j0, min(hi - j0, 32)));
+  const bool here = l < 32 && ((valid >> (l & 31)) & 1u);
   if (p.force == 0) {
-    const FragLane<D> fl(col, hh);
-    const uint16_t* qrow = qterms + min(col, 3) * kRouteRow<D> + 8 * hh;
+    const uint16_t* qrow = qterms + min(l & 31, 3) * kRouteRow<D> + 8 * (l >> 5);
     f32x16 x = zero16();
 #pragma unroll
-    for (int k0 = 0; k0 < KT; k0 += 4) {  // four steps' operands at a time
-      u32x4 kf[4], qf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kf[i] = fl.k(buf, t, k0 + i);
-        qf[i] = *reinterpret_cast<const u32x4*>(qrow + 16 * (k0 + i));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x = mfma32x32x16(as_bf16x8(kf[i]), as_bf16x8(qf[i]), x);
-      chunk_end();
-    }
-    uint32_t bits = 0;  // lanes 0 and 32: rows 8 (e / 4) + 4 hh + e % 4
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      x[e] = (x[e] + quad_lane<1>(x[e])) + quad_lane<2>(x[e]);
-      bits |= x[e] > cut ? 1u << (8 * (e >> 2) + (e & 3)) : 0u;
-    }
-    word = uint32_t(__builtin_amdgcn_readlane(bits, 0)) | (uint32_t(__builtin_amdgcn_readlane(bits, 32)) << 4);
-    if (p.dbg_proxy && col == 0)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = tile_row(0, e, hh);
-        if ((valid >> row) & 1u) p.dbg_proxy[dbg_row + j0 + row] = x[e] * p.scale;
-      }
+    for (int ks = 0; ks < KT; ++ks)
+      x = mfma32x32x16(as_bf16x8(*reinterpret_cast<const u32x4*>(qrow + 16 * ks)), as_bf16x8(kfrag(ks)), x);
+    const float proxy = (x[0] + x[1]) + x[2];
+    word = uint32_t(__builtin_amdgcn_ballot_w64(proxy > cut));
+    if (p.dbg_proxy && here) p.dbg_proxy[dbg_row + j0 + l] = proxy * p.scale;
   }
   if (p.local_blocks >= 0) word |= uint32_t(bit_range64(qb - p.local_blocks - j0, min(qb + p.local_blocks + 1 - j0, 32)));
   word |= uint32_t(bit_range64(0, min(p.kv_sink_blocks - j0, 32)));
   if (qb < p.q_sink_blocks) word = ~0u;
-  const bool here = lane < 32 && ((valid >> (lane & 31)) & 1u);
   if (p.protection) {
-    const bool on = here && p.protection[(int64_t(b) * p.NQB + qb) * p.NKB + j0 + lane] != 0;
+    const bool on = here && p.protection[(int64_t(b) * p.NQB + qb) * p.NKB + j0 + l] != 0;
     word |= uint32_t(__builtin_amdgcn_ballot_w64(on));
   }
   word &= valid;
-  if (p.dbg_selected && here) p.dbg_selected[dbg_row + j0 + lane] = uint8_t((word >> lane) & 1u);
+  if (p.dbg_selected && here) p.dbg_selected[dbg_row + j0 + l] = uint8_t((word >> l) & 1u);
   return word;
+}
+
+// kfrag of rows 32 t .. of the centroid tile in LDS at buf.
+template <int D>
+__device__ __forceinline__ auto lds_centroids(const uint16_t* buf, int t, int lane) {
+  const FragLane<D> fl(fresh(lane & 31), fresh(lane >> 5));
+  return [=](int ks) { return fl.k(buf, t, ks); };
 }
 
 }  // namespace
@@ -907,6 +887,11 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
 #pragma unroll
     for (int r = 0; r < kHalfRounds; ++r) first.round(r);
   }
+
+  // This thread's feature of the key moments: its loads travel with Q's.
+  const bool routed = p.mask != nullptr;  // decisions precomputed by route_kernel
+  KeyMoments<D> km;
+  if (p.force == 0 && !routed && lt < D) km.load(p, head, lt);
 
   // 1. Q tiles -> LDS -> fragments.
   {
@@ -980,11 +965,8 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
 
   // 2. In-kernel routing (no routing masks given): query mean and cutoff per
   // query block (sums in torch's cascade order).
-  const bool routed = p.mask != nullptr;  // decisions precomputed by route_kernel
   if (p.force == 0 && !routed) {
     const int qlen = live ? min(kBlock, p.Tq - qb * kBlock) : 1;
-    KeyMoments<D> km;  // this thread's feature of the key moments, loads issued first
-    if (lt < D) km.load(p, head, lt);
     if (lt < D) s_qm[qg][lt] = query_mean<D>(stage + qg * kBlock * S::KS, qlen, lt);
     __syncthreads();
     float a = 0.f, g = 0.f;
@@ -1060,17 +1042,20 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
       }
       __syncthreads();
     };
-    // Approximated blocks of centroid tile ct (in LDS at buf) for the wave's
-    // query block: from the masks, or routed here -- the tile's 64 blocks for
+    // Approximated blocks of centroid tile ct for the wave's query block: from
+    // the masks, or routed here (centroids(fn) calls fn with the tile's K
+    // fragments of rows 32 (w & 1) .. +31) -- the tile's 64 blocks for
     // every query block of the group (wave w: rows 32 (w & 1) .. +31 for query
     // block w >> 1) into the LDS bitmask, a barrier publishing it.  A tile
     // with none (or a query block past the end) has every score at -inf and
     // adds nothing.
-    auto approximated = [&](const uint16_t* buf, int ct) {
+    auto approximated = [&](auto&& centroids, int ct) {
       if (!routed) {
         if (live) {
-          const uint32_t word = route_word<D>(p, buf, s_qb[qg], s_cut[qg], qh, kBlock * ct + 32 * qh, seg + r0,
-                                              seg + r1, b, qb, lane, dbg_row);
+          const uint32_t word = centroids([&](const auto& kfrag) {
+            return route_word<D>(p, kfrag, s_qb[qg], s_cut[qg], kBlock * ct + 32 * qh, seg + r0, seg + r1, b, qb,
+                                 lane, dbg_row);
+          });
           if (lane == 0) s_mask[qg][2 * (ct - ct0) + qh] = word;
         } else if (lane == 0) {
           s_mask[qg][2 * (ct - ct0) + qh] = 0u;
@@ -1099,6 +1084,9 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
       static_assert(G == 1 && !Q8, "one-slot streams hold one query block's tiles");
       if (r1 <= r0) continue;
       u32x4 k[2][S::KT];
+      auto centroids = [&](auto&& fn) {  // in registers
+        return qh ? fn([&](int ks) { return k[1][ks]; }) : fn([&](int ks) { return k[0][ks]; });
+      };
       auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
       int count, id;
       if (p.force == 1) {
@@ -1118,10 +1106,10 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
         }
         slot_prime<D, 2 * kHalfRounds>(ring, k, col, hh);
         for (int ct = ct_lo; ct < ct_lo + nct - 1; ++ct)
-          centroid_tile<D, true>(st, ring, ct, approximated(ring, ct), tk, qf, col, hh, scale_log2,
+          centroid_tile<D, true>(st, ring, ct, approximated(centroids, ct), tk, qf, col, hh, scale_log2,
                                  slot_step<D>(crefill(ct + 1, ring_lds), NoFrag{}, k));
         const int ct = ct_lo + nct - 1;
-        const uint64_t approx = approximated(ring, ct);
+        const uint64_t approx = approximated(centroids, ct);
         count = cursor.count();
         id = cursor();  // with no selected block, a valid one that nobody attends
         centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
@@ -1148,7 +1136,8 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
         // 3. Centroid pass.
         if (routed) load_masks();
         auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
-          const uint64_t approx = approximated(buf, ct);
+          const uint64_t approx =
+              approximated([&](auto&& fn) { return fn(lds_centroids<D>(buf, qh, lane)); }, ct);
           centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
         };
         tile_stream<D, NT, R>(ring, nct, RangeCursor{ct_lo}, crefill,
@@ -1506,7 +1495,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       // its V rows); its contributions run in the exact stream's prologue,
       // over the first exact tiles' DMA (group 0's first slot is slot 0).
       if (!routed && grp == 0) {
-        const uint32_t word = route_word<D>(p, ctile, s_qb, cut, qh, 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+        const uint32_t word = route_word<D>(p, lds_centroids<D>(ctile, qh, lane), s_qb, cut, 32 * qh, 0, nkb, b, qb,
+                                            lane, dbg_row);
         if (lane == 0) s_mask[qh] = word;
       }
       if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
@@ -1515,7 +1505,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
         if (!routed) {
           if (grp == 0) {
-            const uint32_t word = route_word<D>(p, buf, s_qb, cut, qh, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+            const uint32_t word = route_word<D>(p, lds_centroids<D>(buf, qh, lane), s_qb, cut, kBlock * ct + 32 * qh, 0, nkb,
+                                                b, qb, lane, dbg_row);
             if (lane == 0) s_mask[2 * ct + qh] = word;
           }
           lds_barrier();  // publishes the mask words

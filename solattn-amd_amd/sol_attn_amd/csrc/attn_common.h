@@ -69,7 +69,8 @@ __host__ __device__ inline unsigned balanced_grid(int F, int heads, int R) {
 // The other map (`flat`): XCD x takes one contiguous eighth of the list of
 // all heads' tiles, so its workgroups stay on one head (or few) from end to
 // end and that head's keys stay in its L2.
-__host__ __device__ inline int64_t flat_start(int64_t n, int x) { return n * x / kXcds; }
+// In 32 bits: a launch has fewer than 2^31 workgroups.
+__host__ __device__ inline int flat_start(int n, int x) { return n / kXcds * x + n % kXcds * x / kXcds; }
 
 // Workgroups of a flat launch of F front ids and `heads` x R regular tiles.
 __host__ __device__ inline unsigned flat_grid(int64_t F, int heads, int R) {
@@ -91,17 +92,18 @@ __device__ __forceinline__ TileTask sol_task(int i, int ntiles, int front, int s
   if (flat) {
     const int x = i % kXcds, k = i / kXcds;
     const int per = split_tiles * splits + (front - split_tiles);  // front ids per head
-    const int64_t F = int64_t(per) * heads, T = int64_t(ntiles - front) * heads;
-    const int nf = int(flat_start(F, x + 1) - flat_start(F, x));
+    const int rest = ntiles - front;
+    const int F = per * heads, T = rest * heads;
+    const int nf = F ? flat_start(F, x + 1) - flat_start(F, x) : 0;
     if (k < nf) {
-      const int64_t j = flat_start(F, x) + k;
-      const int h = int(j / per), e = int(j % per);
+      const uint32_t j = uint32_t(flat_start(F, x) + k);
+      const int h = int(j / uint32_t(per)), e = int(j % uint32_t(per));
       if (e < split_tiles * splits) return TileTask{h, e / splits, e % splits};
       return TileTask{h, split_tiles + e - split_tiles * splits};
     }
-    const int64_t j = flat_start(T, x) + (k - nf);
-    if (j >= flat_start(T, x + 1)) return TileTask{-1, 0};
-    return TileTask{int(j / (ntiles - front)), front + int(j % (ntiles - front))};
+    const uint32_t j = uint32_t(flat_start(T, x) + (k - nf));
+    if (int(j) >= flat_start(T, x + 1)) return TileTask{-1, 0};
+    return TileTask{int(j / uint32_t(rest)), front + int(j % uint32_t(rest))};
   }
   const int nsplit = split_tiles * heads * splits;
   if (i < nsplit) {
@@ -127,6 +129,7 @@ __host__ __device__ inline int sink_split_tiles(int splits, int q_sink_blocks, i
 
 // Key blocks [lo, hi) of part s of n of a key sequence of nkb blocks.
 __device__ __forceinline__ int2 split_range(int s, int n, int nkb) {
+  if (n == 1) return int2{0, nkb};
   return int2{int(int64_t(s) * nkb / n), int(int64_t(s + 1) * nkb / n)};
 }
 
@@ -445,6 +448,22 @@ __device__ __forceinline__ int tile_row(int t, int e, int hh) {
   return 32 * t + 8 * (e >> 2) + 4 * hh + (e & 3);
 }
 
+// Lane mask of a wave-uniform bit set over key rows: lanes 0 .. 31 take bit r,
+// lanes 32 .. 63 bit r + 4 (the rows that lane half 0 and 1 hold in the same
+// element; r and r + 4 are in one 32-bit half).
+__device__ __forceinline__ uint64_t row_mask(uint64_t bits, int r) {
+  const uint32_t w = uint32_t(bits >> (r & 32));
+  const int32_t lo = int32_t(w << (31 - (r & 31))) >> 31, hi = int32_t(w << (27 - (r & 31))) >> 31;
+  return uint64_t(uint32_t(lo)) | (uint64_t(uint32_t(hi)) << 32);
+}
+
+// `on` in the lanes of a wave-uniform mask, `off` in the others.
+__device__ __forceinline__ float mask_select(uint64_t mask, float off, float on) {
+  float x;
+  asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(off), "v"(on), "s"(mask));
+  return x;
+}
+
 // Materialises a value at this point of the instruction stream, so that the
 // work producing it stays ahead of a following branch (where the scheduler
 // can overlap it with matrix-core work) instead of being sunk past it.
@@ -523,7 +542,8 @@ struct HalfSoftmax {
   // After the last stage: acc follows the max if this half moved it.
   template <typename Raw>
   __device__ __forceinline__ void resolve(State<D>& st, float, Raw) {
-    if (rescale) rescale_acc<D>(st, alpha);
+    // alpha is 0 in every lane before any key: acc is 0 then.
+    if (rescale && __builtin_amdgcn_ballot_w64(alpha != 0.f)) rescale_acc<D>(st, alpha);
   }
   // Part k of n (n = 4 or 8) of the stages.
   template <int N>
