@@ -93,6 +93,20 @@ int sol_pool_kv(const void* k, const int64_t* k_strides,
                 float* chunk_sums, float* key_mean, float* key_var,
                 void* stream);
 
+/* sol_pool_kv for indexed windows (key_index, ctiles and tiles required),
+ * without the tile copies that sol_attention_windows does not need: block_rows
+ * (int32 [batch, ceil(key_tokens / 64)]) receives, per key block, its first
+ * row where the block is whole and its 64 keys are consecutive rows of K and
+ * V, else -1, and only the -1 blocks are written to tiles.  Frame or range
+ * windows are almost all consecutive blocks, read where they lie. */
+int sol_pool_windows(const void* k, const int64_t* k_strides,
+                     const void* v, const int64_t* v_strides,
+                     const int64_t* key_index, const int32_t* key_lengths,
+                     int64_t sequence_length, int64_t batch, int64_t key_tokens,
+                     int64_t heads, int64_t head_dim, void* ctiles, void* tiles,
+                     float* chunk_sums, float* key_mean, float* key_var,
+                     int32_t* block_rows, void* stream);
+
 /* Workspace bytes of sol_pair_strides (0: pairing does not apply, i.e. fewer
  * than 4 or more than 8192 query blocks, or an unsupported shape).
  * No counterpart in the reference (see sol_pair_strides). */
@@ -288,6 +302,26 @@ int sol_plan_protection(const int64_t* rows, const int64_t* keys, const int32_t*
                         int64_t windows, int64_t query_rows, int64_t key_count,
                         int64_t local_tokens, const int64_t* ranges, int64_t nranges,
                         uint8_t* protected_blocks, void* stream);
+
+/* sol_attention_fwd over indexed windows pooled by sol_pool_windows: block_rows
+ * and tiles as it wrote them, k and v its sources (16-byte aligned rows, token
+ * strides below 2^24 elements; batch strides ignored).  The other arguments
+ * and the results are sol_attention_fwd's with full tiles; every workgroup
+ * holds one query block (workgroup_form 2 is refused), the form
+ * sol_attention_fwd takes for windows of up to 16 MB of K and V per head. */
+int sol_attention_windows(const void* q, const int64_t* q_strides, const int64_t* query_index,
+                          int64_t sequence_length, int64_t batch, int64_t query_tokens, int64_t key_tokens,
+                          const int32_t* key_lengths, int64_t heads, int64_t head_dim,
+                          const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          const int32_t* block_rows, const void* tiles, const void* ctiles,
+                          const float* key_mean, const float* key_var, const float* key_cov,
+                          const uint8_t* protection, const int32_t* pair_strides, void* split_workspace,
+                          void* route_workspace, const float* query_means, double scale, double beta,
+                          int64_t local_blocks, int64_t kv_sink_tokens, int64_t query_sink_tokens,
+                          void* out, const int64_t* out_index, int32_t* counts,
+                          uint8_t* debug_selected, float* debug_proxy, float* debug_cutoff,
+                          const void* qk_int8_tiles, const float* qk_int8_scales,
+                          int workgroup_form, void* stream);
 
 /* Non-causal BF16 attention over all keys, FP32 softmax and accumulation.
  * Replaces `launch_dense` (kernels.py:193-200; kernel kernels.py:67-98).

@@ -45,6 +45,13 @@ _SIGNATURES = {
                            _p, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                            _dbl, _dbl, _i64, _i64, _i64,
                            _p, _p, _p, _p, _p, _p, _p, _p, _int, _p], ctypes.c_int),
+    "sol_pool_windows": ([_p, _i64p, _p, _i64p, _p, _p, _i64, _i64, _i64, _i64, _i64,
+                          _p, _p, _p, _p, _p, _p, _p], ctypes.c_int),
+    "sol_attention_windows": ([_p, _i64p, _p, _i64, _i64, _i64, _i64, _p, _i64, _i64,
+                               _p, _i64p, _p, _i64p,
+                               _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p,
+                               _dbl, _dbl, _i64, _i64, _i64,
+                               _p, _p, _p, _p, _p, _p, _p, _p, _int, _p], ctypes.c_int),
     "sol_dense_fwd": ([_p, _i64p, _p, _i64, _p, _i64p, _p, _i64p, _i64, _i64, _i64, _i64, _i64,
                        _dbl, _p, _p, _p, _p], ctypes.c_int),
     "sol_plan_protection": ([_p, _p, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _p], ctypes.c_int),
@@ -158,7 +165,8 @@ def _region(ws, offset, dtype, shape):
     return ws[offset:offset + n].view(dtype).view(shape)
 
 
-def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, views=True, qk_int8=False):
+def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, views=True, qk_int8=False,
+            windows=False):
     """Centroid tiles, attention tiles and key moments (one HBM pass over K and V).
 
     ``k``/``v``: ``[B, Tk, H, D]`` BF16 or, with ``key_index`` ``[B, Tk]``,
@@ -171,7 +179,10 @@ def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, v
     ``moments``); layouts per ``include/sol_attn_amd.h``.  The block tiles
     exist only when the keys do not qualify for rows mode (:func:`rows_mode`);
     otherwise the attention kernels read K and V themselves, which the dict
-    keeps (``k``, ``v``).  ``qk_int8`` also quantises K per block
+    keeps (``k``, ``v``).  ``windows`` (with ``key_index``): key blocks of
+    consecutive rows stay where they are (``sol_pool_windows``): the tiles
+    hold the other blocks only, and the dict keeps K, V and the blocks' first
+    rows (``block_rows_ptr``) for :func:`attend`.  ``qk_int8`` also quantises K per block
     (``sol_quantize_keys``) for the INT8-QK experiment.
     """
     lib = library()
@@ -193,18 +204,24 @@ def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, v
     sizes += [b * h * -(-nkb // 16) * 2 * d * 4, b * h * d * 4, b * h * d * 4] if moments else [0, 0, 0]
     if qk_int8:
         sizes += [b * h * nkb * BLOCK * d, b * h * nkb * 4]
+    windows = windows and indexed and max(k.stride(-3), v.stride(-3)) < (1 << 24)
+    if windows:
+        sizes.append(b * nkb * 4)
     offsets, total = _carve(tuple(sizes))
     ws = torch.empty(total, device=dev, dtype=torch.uint8)
     base = ws.data_ptr()
     ctiles, tiles = base + offsets[0], None if rows else base + offsets[1]
     sums, mean, var = (base + o for o in offsets[2:5]) if moments else (None, None, None)
-    _check(lib.sol_pool_kv(k.data_ptr(), _strides(k, indexed), v.data_ptr(), _strides(v, indexed),
-                           _ptr(key_index), _ptr(key_lengths), k.shape[0] if indexed else 0,
-                           b, tk, h, d, ctiles, tiles, sums, mean, var, stream))
+    block_rows = base + offsets[-1] if windows else None
+    args = (k.data_ptr(), _strides(k, indexed), v.data_ptr(), _strides(v, indexed),
+            _ptr(key_index), _ptr(key_lengths), k.shape[0] if indexed else 0,
+            b, tk, h, d, ctiles, tiles, sums, mean, var)
+    _check(lib.sol_pool_windows(*args, block_rows, stream) if windows else lib.sol_pool_kv(*args, stream))
     pooled = {"workspace": ws, "shape": (b, h, d), "ctiles_ptr": ctiles, "tiles_ptr": tiles,
               "mean_ptr": mean, "var_ptr": var, "cov_ptr": None, "key_tokens": tk,
               "key_blocks": nkb, "key_lengths": key_lengths, "k8_ptr": None, "k8_scale_ptr": None,
-              "k": k if rows else None, "v": v if rows else None}
+              "block_rows_ptr": block_rows,
+              "k": k if rows or windows else None, "v": v if rows or windows else None}
     if qk_int8:
         k8, k8s = base + offsets[5], base + offsets[6]
         _check(lib.sol_quantize_keys(k.data_ptr(), _strides(k, indexed), _ptr(key_index), _ptr(key_lengths),
@@ -256,13 +273,18 @@ PAIR_MIN_QUERY_BLOCKS = 8192
 ONE_BLOCK_KEY_BYTES = 16 << 20
 
 
+def _one_block_keys(nk, d):
+    """Key sequences whose launches hold one query block per workgroup."""
+    return -(-nk // BLOCK) * BLOCK * d * 4 <= ONE_BLOCK_KEY_BYTES
+
+
 def _pairs(b, nq, nk, h, d):
     """Whether a call's attention launch pairs query blocks (a forced
     WORKGROUP_FORM or ROUTE_PREPASS "always" leaves the size rule aside)."""
     if not PAIRING or b * h * -(-nq // BLOCK) < PAIR_MIN_QUERY_BLOCKS:
         return False
     return (WORKGROUP_FORM != 0 or ROUTE_PREPASS == "always"
-            or -(-nk // BLOCK) * BLOCK * d * 4 > ONE_BLOCK_KEY_BYTES)
+            or not _one_block_keys(nk, d))
 
 
 def _pair_buffers(q, rows, min_blocks):
@@ -445,10 +467,13 @@ def attend(q, pooled, scale, beta, local, kv_sink, q_sink, protection=None, rows
     else:
         query_means = None
     kr, vr = pooled["k"], pooled["v"]
-    _check(lib.sol_attention_fwd(
+    block_rows = pooled["block_rows_ptr"]
+    gathered = block_rows is not None
+    _check((lib.sol_attention_windows if gathered else lib.sol_attention_fwd)(
         q.data_ptr(), _strides(q, indexed), _ptr(rows), q.shape[0] if indexed else 0,
         b, nq, nk, _ptr(pooled["key_lengths"]), h, d,
-        _ptr(kr), None if kr is None else _strides(kr), _ptr(vr), None if vr is None else _strides(vr),
+        _ptr(kr), None if kr is None else _strides(kr, gathered), _ptr(vr),
+        None if vr is None else _strides(vr, gathered), *((block_rows,) if gathered else ()),
         pooled["tiles_ptr"], pooled["ctiles_ptr"], pooled["mean_ptr"], pooled["var_ptr"], pooled["cov_ptr"],
         _ptr(prot), _ptr(strides), _ptr(split), _ptr(route), _ptr(query_means), float(scale), float(beta),
         int(local), int(kv_sink), int(q_sink),
@@ -505,6 +530,7 @@ def _self_pooled(k, v):
     return {"workspace": None, "shape": (b, h, d), "ctiles_ptr": None, "tiles_ptr": None,
             "mean_ptr": None, "var_ptr": None, "cov_ptr": None, "key_tokens": nk,
             "key_blocks": -(-nk // BLOCK), "key_lengths": None, "k8_ptr": None, "k8_scale_ptr": None,
+            "block_rows_ptr": None,
             "k": k, "v": v}
 
 
@@ -572,7 +598,8 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
             strides, means = pairing[2], pairing[3]
     try:
         pooled = pool_kv(k, v, key_index=keys, moments=not math.isinf(beta), key_lengths=key_lengths,
-                         stream=stream, views=debug, qk_int8=qk_precision == "int8")
+                         stream=stream, views=debug, qk_int8=qk_precision == "int8",
+                         windows=WORKGROUP_FORM != 2 and _one_block_keys(nk, q.shape[-1]))
         if threshold_estimator == "full_covariance" and not math.isinf(beta):
             key_covariance(pooled, stream)
     finally:

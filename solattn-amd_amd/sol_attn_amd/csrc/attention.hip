@@ -95,20 +95,16 @@ struct NoFrag {
 // FragLane::k reads them from the LDS tile: k_fragments(...)(j)(t, ks).
 template <int D, bool KT>
 __device__ __forceinline__ auto k_fragments(const AttnParams& p, int b, int h, int col, int hh) {
-  const uint16_t* base = KT ? p.tiles + (int64_t(b) * p.H + h) * p.NKB * Shape<D>::TILE
-                            : p.k.base + int64_t(b) * p.k.sb + int64_t(h) * p.k.sh;
-  const int64_t st = p.k.st;
-  const int tk = p.Tk;
-  return [=](int j) {
-    return [=](int t, int ks) {
+  const uint16_t* tiles = KT ? p.tiles + (int64_t(b) * p.H + h) * p.NKB * Shape<D>::TILE : nullptr;
+  const uint16_t* base = p.k.base + int64_t(b) * p.k.sb + int64_t(h) * p.k.sh;
+  return [=, &p](int j) {
+    return [=, &p](int t, int ks) {
       const int c = fresh(col), x = fresh(hh);
-      if constexpr (KT) {
-        return load16(base + int64_t(j) * Shape<D>::TILE + (c + 32 * t) * D +
+      int row = KT ? block_row(p, b, j) : ((j + 1) * kBlock <= p.Tk ? j * kBlock : p.Tk - kBlock);
+      if (KT && row < 0)
+        return load16(tiles + int64_t(j) * Shape<D>::TILE + (c + 32 * t) * D +
                       (TileLayout<D>::k_lane_xor(c, x) ^ (16 * ks)));
-      } else {
-        const int row = ((j + 1) * kBlock <= tk ? j * kBlock : tk - kBlock) + 32 * t + c;
-        return load16(base + int64_t(row) * st + 16 * ks + 8 * x);
-      }
+      return load16(base + int64_t(row + 32 * t + c) * p.k.st + 16 * ks + 8 * x);
     };
   };
 }
@@ -481,13 +477,21 @@ __device__ __forceinline__ auto bf16_refills(Source source, int wave, int lane) 
 }
 
 // Refill factory of key block j's K + V tile pair for (entry b, head h):
-// from the pooled tile pairs (KT: indexed windows, or fewer than 64 keys) or
+// from the pooled tile pairs (KT: fewer than 64 keys, or indexed windows,
+// whose blocks of consecutive rows come from the K / V rows with WINDOWS) or
 // straight from the K / V rows.
-template <int D, int NT, bool KT>
+template <int D, int NT, bool KT, bool WINDOWS>
 __device__ __forceinline__ auto kv_refills(const AttnParams& p, int b, int h, int wave, int lane) {
   if constexpr (KT) {
     const uint16_t* tiles = p.tiles + (int64_t(b) * p.H + h) * p.NKB * Shape<D>::TILE;
-    return bf16_refills<D, NT>([=](int j) { return tiles + int64_t(j) * Shape<D>::TILE; }, wave, lane);
+    if constexpr (WINDOWS) {
+      const KvRows<D, NT> rows = kv_rows<D, NT>(p, b, h, wave * kWave + lane);
+      return [=, &p](int j, uint32_t lds) {
+        return WindowRefill<D, NT>(rows, tiles + int64_t(j) * Shape<D>::TILE, block_row(p, b, j), lds, wave, lane);
+      };
+    } else {
+      return bf16_refills<D, NT>([=](int j) { return tiles + int64_t(j) * Shape<D>::TILE; }, wave, lane);
+    }
   } else {
     const KvRows<D, NT> rows = kv_rows<D, NT>(p, b, h, wave * kWave + lane);
     return [=](int j, uint32_t lds) { return RowRefill<D, NT>(rows, j, lds, wave); };
@@ -1076,7 +1080,7 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
     // Only the last segment's last tile can be the partial tail block.  Tile
     // ids travel as tags 2 j + own-selection bit (UnionCursor).
     UnionCursor<G> cursor{&s_mask[0][0], s_mask[qg], kMaskWords, r0, r1, seg};
-    const auto kv = kv_refills<D, NT, KT>(p, b, h, wave, lane);
+    const auto kv = kv_refills<D, NT, KT, G == 1>(p, b, h, wave, lane);
     if constexpr (R == 1) {
       // One query block: every streamed tile is its own, and the centroid
       // tiles and the exact tiles are one stream (the last centroid tile's
@@ -1537,7 +1541,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
     UnionCursor<1> all{s_mask, s_mask, kMaskWords, 0, nkb, 0};
     const int steps = (all.count() + KS - 1) / KS;
     const int wg = wave & 1;  // the wave inside its group
-    const auto kv = kv_refills<D, 128, KT>(p, b, h, wg, lane);
+    const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
     auto selected = [](int tag) { return (tag & 1) != 0; };
     auto hit = [&](const uint16_t* buf, int, const auto& refill) {
       full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
@@ -1664,7 +1668,7 @@ __global__ __launch_bounds__(256, 2) void dense_attention_kernel(AttnParams p) {
     full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
   };
   tile_stream<D, NT, 2>(
-      ring, p.NKB, RangeCursor{0}, kv_refills<D, NT, KT>(p, b, h, wave, lane), tile_runs(always, hit, hit),
+      ring, p.NKB, RangeCursor{0}, kv_refills<D, NT, KT, false>(p, b, h, wave, lane), tile_runs(always, hit, hit),
       [&](const uint16_t* buf, int j, const auto& refill) {
         exact_tile<D, !KT>(st, buf, j, tk, qf, col, hh, scale_log2, ring_step(refill));
       },
@@ -1885,6 +1889,7 @@ hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
   // tiles, their order and its softmax state do not depend on its partner).
   int g = one_block_launch(int64_t(p.B) * p.H, p.NQB, p.NKB, D) ? 1 : 2;
   if (p.workgroup_form == 1 || p.workgroup_form == 2) g = p.workgroup_form;
+  if (p.block_rows) g = 1;  // read by the one-block form only
   AttnParams q = p;
   q.flat = head_key_bytes(p.NKB, D) <= kFlatKeyBytes ? 1 : 0;
   q.order = nullptr;

@@ -370,6 +370,62 @@ struct RowRefill {
   }
 };
 
+// DMA of key block j of an indexed window into the LDS slot at dst_lds: from
+// rows of K and V where the block's keys are consecutive (row >= 0, the first
+// one; RowRefill's addresses), else from its pooled tile pair (TileRefill's).
+template <int D, int NT>
+struct WindowRefill {
+  using Src = KvRows<D, NT>;
+  static constexpr int kHalf = Src::kHalfRounds;
+  static constexpr int kRounds = 2 * kHalf;
+  uint64_t ksrc, vsrc;
+  uint32_t kstep, vstep;
+  uint32_t klane, vlane, klane_odd;
+  uint32_t lds;
+
+  __device__ __forceinline__ WindowRefill(const Src& src, const uint16_t* tile, int row, uint32_t dst_lds, int wave,
+                                          int lane) {
+    const bool rows = row >= 0;
+    const uint64_t t = reinterpret_cast<uint64_t>(tile) + uint64_t(wave) * (kWave * 16);
+    ksrc = uniform64(rows ? src.k + uint64_t(uint32_t(row)) * src.stk : t);
+    vsrc = uniform64(rows ? src.v + uint64_t(uint32_t(row)) * src.stv : t + TileLayout<D>::kElems * 2);
+    kstep = rows ? Src::kRowsPerRound * src.stk : NT * 16;
+    vstep = rows ? Src::kRowsPerRound * src.stv : NT * 16;
+    const uint32_t linear = uint32_t(lane) * 16u;
+    klane = rows ? src.klane : linear;
+    vlane = rows ? src.vlane : linear;
+    klane_odd = rows ? src.klane_odd : linear;
+    lds = uint32_t(__builtin_amdgcn_readfirstlane(dst_lds + uint32_t(wave) * (kWave * 16)));
+  }
+  __device__ __forceinline__ void round(int r) const {
+    if (r < kHalf) {
+      const uint32_t lane = (Src::kOddK && (r & 1)) ? klane_odd : klane;
+      dma16(ksrc + uint64_t(uint32_t(r) * kstep), lane, lds + uint32_t(r * NT * 16));
+    } else {
+      const int rv = r - kHalf;
+      dma16(vsrc + uint64_t(uint32_t(rv) * vstep), vlane, lds + uint32_t(TileLayout<D>::kElems * 2 + rv * NT * 16));
+    }
+  }
+  __device__ __forceinline__ void all() const {
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) round(r);
+  }
+  template <int N>
+  __device__ __forceinline__ void after_step(int k) const {
+#pragma unroll
+    for (int r = k * kRounds / N; r < (k + 1) * kRounds / N; ++r) round(r);
+  }
+};
+
+// p.block_rows of key block j (wave-uniform) of entry b, or -1, through the
+// scalar cache: a vector load's wait would drain the DMAs in flight.
+__device__ __forceinline__ int block_row(const AttnParams& p, int b, int j) {
+  if (!p.block_rows) return -1;
+  typedef const int32_t __attribute__((address_space(4)))* scalar_ptr;
+  const scalar_ptr rows = (scalar_ptr)(uintptr_t)(p.block_rows + int64_t(b) * p.NKB);
+  return rows[__builtin_amdgcn_readfirstlane(j)];
+}
+
 // DMA for the quantised-QK experiment's exact tiles: the INT8 K tile of a
 // key block (64 rows x D bytes, contiguous in the INT8 tile array) at the
 // slot's start, then the block's V tile as the BF16 refill V moves it (Kv: a

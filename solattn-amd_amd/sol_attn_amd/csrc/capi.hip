@@ -221,7 +221,7 @@ int attention_fwd_impl(const void* q, const int64_t* q_strides, const int64_t* q
                       uint8_t* debug_selected, float* debug_proxy, float* debug_cutoff,
                       const void* qk_int8_tiles, const float* qk_int8_scales,
                       int workgroup_form, void* stream,
-                       const float* chunk_sums, bool tile_moments);
+                       const float* chunk_sums, bool tile_moments, const int32_t* block_rows = nullptr);
 
 }  // namespace
 
@@ -252,7 +252,7 @@ int pool_checked(const char* who, const void* k, const int64_t* k_strides, const
                  int64_t sequence_length, int64_t batch, int64_t key_tokens, int64_t heads,
                  int64_t head_dim, void* ctiles, void* tiles,
                  float* chunk_sums, float* key_mean, float* key_var, void* stream,
-                 bool fold_in_attention = false, bool blocks_only = false) {
+                 bool fold_in_attention = false, bool blocks_only = false, int32_t* block_rows = nullptr) {
   static thread_local std::string msg;
   auto err = [&](int code, const char* what) {
     msg = std::string(who) + ": " + what;
@@ -293,6 +293,9 @@ int pool_checked(const char* who, const void* k, const int64_t* k_strides, const
   if (blocks_only && (tiles || !ctiles || key_index || key_lengths || moments || nkb > sol::kPoolChunk))
     return err(SOL_ERR_INVALID, "centroid-only pooling needs plain rows, ctiles only and at most 16 key blocks");
   p.blocks_only = blocks_only ? 1 : 0;
+  if (block_rows && !(indexed && tiles && ctiles))
+    return err(SOL_ERR_INVALID, "block_rows need key_index, tiles and ctiles");
+  p.block_rows = block_rows;
   return hip_status(sol::launch_pool(p, int(head_dim), static_cast<hipStream_t>(stream)));
 }
 
@@ -305,6 +308,18 @@ int sol_pool_kv(const void* k, const int64_t* k_strides, const void* v, const in
   return pool_checked("sol_pool_kv", k, k_strides, v, v_strides, key_index, key_lengths,
                       sequence_length, batch, key_tokens, heads, head_dim, ctiles, tiles,
                       chunk_sums, key_mean, key_var, stream);
+}
+
+int sol_pool_windows(const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                     const int64_t* key_index, const int32_t* key_lengths, int64_t sequence_length,
+                     int64_t batch, int64_t key_tokens, int64_t heads, int64_t head_dim, void* ctiles,
+                     void* tiles, float* chunk_sums, float* key_mean, float* key_var, int32_t* block_rows,
+                     void* stream) {
+  if (!key_index || !tiles || !ctiles || !block_rows)
+    return fail(SOL_ERR_INVALID, "sol_pool_windows: key_index, ctiles, tiles and block_rows are required");
+  return pool_checked("sol_pool_windows", k, k_strides, v, v_strides, key_index, key_lengths,
+                      sequence_length, batch, key_tokens, heads, head_dim, ctiles, tiles,
+                      chunk_sums, key_mean, key_var, stream, false, false, block_rows);
 }
 
 int64_t sol_pair_workspace_size(int64_t batch, int64_t query_tokens, int64_t heads, int64_t head_dim) {
@@ -443,6 +458,33 @@ int sol_attention_fwd(const void* q, const int64_t* q_strides, const int64_t* qu
                             qk_int8_scales, workgroup_form, stream, nullptr, false);
 }
 
+int sol_attention_windows(const void* q, const int64_t* q_strides, const int64_t* query_index,
+                          int64_t sequence_length, int64_t batch, int64_t query_tokens, int64_t key_tokens,
+                          const int32_t* key_lengths, int64_t heads, int64_t head_dim,
+                          const void* k, const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          const int32_t* block_rows, const void* tiles, const void* ctiles, const float* key_mean,
+                          const float* key_var, const float* key_cov, const uint8_t* protection,
+                          const int32_t* pair_strides, void* split_workspace, void* route_workspace,
+                          const float* query_means, double scale, double beta,
+                          int64_t local_blocks, int64_t kv_sink_tokens, int64_t query_sink_tokens,
+                          void* out, const int64_t* out_index, int32_t* counts,
+                          uint8_t* debug_selected, float* debug_proxy, float* debug_cutoff,
+                          const void* qk_int8_tiles, const float* qk_int8_scales,
+                          int workgroup_form, void* stream) {
+  if (workgroup_form == 2)
+    return fail(SOL_ERR_INVALID, "sol_attention_windows: one query block per workgroup (workgroup_form 0 or 1)");
+  if (!block_rows || !tiles || !operand_ok(k, k_strides, true) || !operand_ok(v, v_strides, true) ||
+      k_strides[1] >= (int64_t(1) << 24) || v_strides[1] >= (int64_t(1) << 24))
+    return fail(SOL_ERR_INVALID, "sol_attention_windows: block_rows, tiles and 16-byte aligned K / V rows (token "
+                                 "stride < 2^24 elements) are required");
+  return attention_fwd_impl(q, q_strides, query_index, sequence_length, batch, query_tokens, key_tokens,
+                            key_lengths, heads, head_dim, k, k_strides, v, v_strides, tiles, ctiles, key_mean,
+                            key_var, key_cov, protection, pair_strides, split_workspace, route_workspace,
+                            query_means, scale, beta, local_blocks, kv_sink_tokens, query_sink_tokens, out,
+                            out_index, counts, debug_selected, debug_proxy, debug_cutoff, qk_int8_tiles,
+                            qk_int8_scales, workgroup_form, stream, nullptr, false, block_rows);
+}
+
 int sol_quantize_keys(const void* k, const int64_t* k_strides, const int64_t* key_index,
                       const int32_t* key_lengths, int64_t sequence_length, int64_t batch, int64_t key_tokens,
                       int64_t heads, int64_t head_dim, int rows_mode, void* k8_tiles, float* k8_scales,
@@ -543,7 +585,7 @@ int attention_fwd_impl(const void* q, const int64_t* q_strides, const int64_t* q
                       uint8_t* debug_selected, float* debug_proxy, float* debug_cutoff,
                       const void* qk_int8_tiles, const float* qk_int8_scales,
                       int workgroup_form, void* stream,
-                       const float* chunk_sums, bool tile_moments) {
+                       const float* chunk_sums, bool tile_moments, const int32_t* block_rows) {
   if (!shape_ok(batch, query_tokens, heads, head_dim) || key_tokens <= 0 ||
       key_tokens >= (int64_t(1) << 30))
     return fail(SOL_ERR_INVALID, "sol_attention_fwd: unsupported shape (head_dim must be 64 or 128)");
@@ -600,10 +642,12 @@ int attention_fwd_impl(const void* q, const int64_t* q_strides, const int64_t* q
   p.k8 = static_cast<const int8_t*>(qk_int8_tiles);
   p.k8_scale = qk_int8_scales;
   p.tiles = static_cast<const uint16_t*>(tiles);
-  if (!tiles) {
+  if (!tiles || block_rows) {
     p.k = rows_of(k, k_strides, nullptr, key_tokens);
     p.v = rows_of(v, v_strides, nullptr, key_tokens);
   }
+  if (block_rows) p.k.sb = p.v.sb = 0;  // rows of one [N, H, D] source for every entry
+  p.block_rows = block_rows;
   p.ctiles = static_cast<const uint16_t*>(ctiles);
   p.mean = chunk_sums || tile_moments ? nullptr : key_mean;
   p.var = chunk_sums || tile_moments ? nullptr : key_var;

@@ -24,6 +24,29 @@
 
 namespace sol {
 
+// First row of key block j (LANES adjacent lanes per block, this lane number
+// l) when its 64 keys are consecutive rows of an indexed source, else -1: the
+// attention kernels then read it from K and V themselves, and no tile copy is
+// made.  Index entries are checked one by one, so the rows read are the rows
+// the index names.
+template <int LANES>
+__device__ __forceinline__ int consecutive_row(const TokenRows& r, int b, int j, int tk, int lane) {
+  const int l = lane % LANES;
+  const bool whole = (j + 1) * kBlock <= tk;
+  const int64_t* idx = r.index + int64_t(b) * r.T + int64_t(j) * kBlock;
+  bool ok = whole;
+  int64_t first = 0;
+  if (whole) {
+    first = idx[0];
+#pragma unroll
+    for (int i = l; i < kBlock; i += LANES) ok = ok && idx[i] == first + i;
+    ok = ok && first >= 0 && first + kBlock <= r.N && first < (int64_t(1) << 30);
+  }
+  const uint64_t all = __builtin_amdgcn_ballot_w64(ok);
+  const uint64_t mine = LANES == 64 ? all : (all >> (lane - l)) & ((1ull << (LANES % 64)) - 1ull);
+  return mine == (LANES == 64 ? ~0ull : (1ull << (LANES % 64)) - 1ull) ? int(first) : -1;
+}
+
 // Two workgroup forms, both covering one 16-block chunk per workgroup:
 // - NW = 4 waves, each pooling 4 blocks in turn (large grids), each keeping
 //   16 rows x 16 bytes per lane in flight, with non-temporal loads (K and V
@@ -68,11 +91,15 @@ void pool_kv_kernel(PoolParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) s[e] = 0.f;
     int len = 0;
+    const int row = p.block_rows ? consecutive_row<LPB>(src, b, j, tk, lane) : -1;
+    if (p.block_rows && !is_v && h == 0 && j < p.NKB && lane % LPB == 0)
+      p.block_rows[int64_t(b) * p.NKB + j] = row;
     if (j < nkb) {
       len = min(kBlock, tk - kBlock * j);
       u32x4 x[16];
-      load_rows16<16, true>(src, b, kBlock * j + 16 * r4, kBlock * j + len - 1, h, 8 * dc, x);
-      if (p.tiles) {
+      load_rows16<16, true>(src, b, kBlock * j + 16 * r4, kBlock * j + len - 1, h, 8 * dc, x,
+                            row < 0 ? -1 : row + 16 * r4);
+      if (p.tiles && row < 0) {
         // Attention-ready tiles in the LDS image layout (zero past the end),
         // for keys the attention kernels cannot DMA row by row.
         uint16_t* tile = p.tiles + ((int64_t(b) * p.H + h) * p.NKB + j) * 2 * TL::kElems;
@@ -272,15 +299,18 @@ __global__ __launch_bounds__(1024) void pool_kv4_kernel(PoolParams p) {
   const int jb = wave;
   const int j = c * kPoolChunk + jb;
   const int len = j < nkb ? min(kBlock, tk - kBlock * j) : 0;
+  const int row = p.block_rows ? consecutive_row<kWave>(src, b, j, tk, lane) : -1;
+  if (p.block_rows && !is_v && h0 == 0 && j < p.NKB && lane == 0) p.block_rows[int64_t(b) * p.NKB + j] = row;
   float tot[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) tot[e] = 0.f;
   if (len > 0) {
-    uint16_t* tile = p.tiles ? p.tiles + ((int64_t(b) * p.H + h0 + hq) * p.NKB + j) * 2 * TL::kElems : nullptr;
+    uint16_t* tile = p.tiles && row < 0 ? p.tiles + ((int64_t(b) * p.H + h0 + hq) * p.NKB + j) * 2 * TL::kElems : nullptr;
 #pragma unroll 1
     for (int q = 0; q < 4; ++q) {
       u32x4 x[16];
-      load_rows16<16, true>(src, b, kBlock * j + 16 * q, kBlock * j + len - 1, h0 + hq, 8 * dc, x);
+      load_rows16<16, true>(src, b, kBlock * j + 16 * q, kBlock * j + len - 1, h0 + hq, 8 * dc, x,
+                            row < 0 ? -1 : row + 16 * q);
       if (tile) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {

@@ -115,11 +115,17 @@ __device__ __forceinline__ u32x4 load16(const uint16_t* p) {
 // every data load is then issued unconditionally -- rows past t_last re-read
 // row t_last -- so the N loads are in flight at once instead of each waiting
 // behind a branch.  STREAM marks the loads non-temporal (data read once).
+// first_row >= 0: t0's row when the entry's rows t0 .. t_last are consecutive
+// (indexed sources: no index entry is read).
 template <int N, bool STREAM = false>
 __device__ __forceinline__ void load_rows16(const TokenRows& r, int b, int t0, int t_last, int h, int col,
-                                            u32x4 (&x)[N]) {
+                                            u32x4 (&x)[N], int first_row = -1) {
   const uint16_t* p[N];
-  if (r.index) {
+  if (first_row >= 0) {
+    const uint16_t* base = r.base + int64_t(h) * r.sh + col;
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = base + int64_t(first_row + min(i, t_last - t0)) * r.st;
+  } else if (r.index) {
     const int64_t* idx = r.index + int64_t(b) * r.T;
     int64_t row[N];
 #pragma unroll

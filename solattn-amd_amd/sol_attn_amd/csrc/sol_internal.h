@@ -21,6 +21,8 @@ struct PoolParams {
   const int32_t* klen;  // [B] key tokens per batch entry (<= Tk), or null: all Tk
   uint16_t* ctiles;  // [B, H, NCT, 2, 64 * D] centroid tiles, or null
   uint16_t* tiles;   // [B, H, NKB, 2, 64 * D] K / V block tiles (TileLayout), or null
+  int32_t* block_rows;  // [B, NKB] or null (indexed keys only): the first row of each whole key block
+                        // whose 64 keys are consecutive rows, -1 for the others; only those go to tiles
   float* ksum;       // [B, H, NCH, 2, D] chunk sums, null -> no moments
   float* mean;       // [B, H, D]
   float* var;        // [B, H, D]
@@ -74,6 +76,8 @@ struct AttnParams {
   int64_t out_rows;            // N: rows of an out_index output (others are skipped)
   TokenRows k, v;              // key rows the kernels DMA straight into LDS (tiles null)
   const uint16_t* tiles;       // [B, H, NKB, 2, 64 * D] pooled block tiles, or null: rows of k / v
+  const int32_t* block_rows;   // [B, NKB] with tiles, or null: key blocks read from rows of k / v instead
+                               // (their first row; -1: from the tile)
   const uint16_t* ctiles;      // [B, H, NCT, 2, 64 * D] centroid tiles
   const float* mean;           // [B, H, D]
   const float* var;            // [B, H, D]
