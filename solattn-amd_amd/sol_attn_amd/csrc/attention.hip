@@ -67,6 +67,7 @@ struct SlotStep {
   const Refill& refill;  // the next tile's
   Frag frag;
   u32x4 (&k)[2][Shape<D>::KT];
+  const uint16_t* slot;  // where the next tile's K arrives
   // Part i of N of the K (V) rounds.
   template <int N>
   __device__ __forceinline__ void k_rounds(int i) const {
@@ -82,8 +83,9 @@ struct SlotStep {
 
 template <int D, typename Refill, typename Frag>
 __device__ __forceinline__ SlotStep<D, Refill, Frag> slot_step(const Refill& refill, Frag frag,
-                                                               u32x4 (&k)[2][Shape<D>::KT]) {
-  return {refill, frag, k};
+                                                               u32x4 (&k)[2][Shape<D>::KT],
+                                                               const uint16_t* slot) {
+  return {refill, frag, k, slot};
 }
 
 // For steps with the max-pass softmax, which never look again.
@@ -242,8 +244,8 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
     const int c4 = f / DT, dt = f % DT;
     st.acc[dt] = mfma32x32x16(as_bf16x8(vb[c4][dt]), h1.pb(c4), st.acc[dt]);
     if constexpr (ONE) {
-      step.k[0][f] = fl.k(buf, 0, f);  // KT = 2 DT fragments per half
-      step.k[1][f] = fl.k(buf, 1, f);
+      step.k[0][f] = fl.k(step.slot, 0, f);  // KT = 2 DT fragments per half
+      step.k[1][f] = fl.k(step.slot, 1, f);
       chunk_end();
     }
   }
@@ -264,21 +266,22 @@ __device__ __forceinline__ void full_tile(State<D>& st, const uint16_t* buf,
 // The rows of the sequence's partial last block j that hold its tk - 64 j
 // keys: [64 - len, 64) when the block was DMA'd from rows shifted back to the
 // sequence's last 64 rows (SHIFTED), else [0, len) (zero-padded tiles).
-// A whole block's are all 64.  Returned relative to this lane's rows, as the bounds a <= tile_row(t, e, 0)
+// A whole block's are all 64; none without `any`.  Returned relative to this lane's rows, as the bounds a <= tile_row(t, e, 0)
 // < z of the present keys.
 template <bool SHIFTED>
-__device__ __forceinline__ int2 tail_rows(int j, int tk, int hh) {
-  const int len = min(kBlock, tk - j * kBlock);
+__device__ __forceinline__ int2 tail_rows(int j, int tk, int hh, bool any = true) {
+  const int len = any ? min(kBlock, tk - j * kBlock) : 0;
   const int lo = SHIFTED ? kBlock - len : 0;
   return make_int2(fresh(lo - 4 * hh), fresh(lo + len - 4 * hh));
 }
 
-// The partial last block j, whose absent keys start at -inf.
+// The partial last block j, whose absent keys start at -inf (all of them
+// without `any`: a tile that adds nothing).
 template <int D, bool SHIFTED, bool FULL = false, typename Step>
-__device__ __forceinline__ void tail_tile(State<D>& st, const uint16_t* buf, int j, int tk,
+__device__ __forceinline__ void tail_tile(State<D>& st, const uint16_t* buf, int j, int tk, bool any,
                                           const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
                                           const Step& step) {
-  const int2 present = tail_rows<SHIFTED>(j, tk, hh);
+  const int2 present = tail_rows<SHIFTED>(j, tk, hh, any);
   const auto absent = [&](int t) {
     f32x16 bias;
 #pragma unroll
@@ -300,7 +303,7 @@ __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, in
   if ((j + 1) * kBlock <= tk) {
     full_tile<D, FULL>(st, buf, qf, col, hh, c, step);
   } else {
-    tail_tile<D, SHIFTED, FULL>(st, buf, j, tk, qf, col, hh, c, step);
+    tail_tile<D, SHIFTED, FULL>(st, buf, j, tk, true, qf, col, hh, c, step);
   }
 }
 
@@ -1111,26 +1114,26 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
         slot_prime<D, 2 * kHalfRounds>(ring, k, col, hh);
         for (int ct = ct_lo; ct < ct_lo + nct - 1; ++ct)
           centroid_tile<D, true>(st, ring, ct, approximated(centroids, ct), tk, qf, col, hh, scale_log2,
-                                 slot_step<D>(crefill(ct + 1, ring_lds), NoFrag{}, k));
+                                 slot_step<D>(crefill(ct + 1, ring_lds), NoFrag{}, k, ring));
         const int ct = ct_lo + nct - 1;
         const uint64_t approx = approximated(centroids, ct);
         count = cursor.count();
         id = cursor();  // with no selected block, a valid one that nobody attends
         centroid_tile<D, true>(st, ring, ct, approx, tk, qf, col, hh, scale_log2,
-                               slot_step<D>(make(id, ring_lds), NoFrag{}, k));
+                               slot_step<D>(make(id, ring_lds), NoFrag{}, k, ring));
       }
       count_selected();
       const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
       slot_stream(
           ring_lds, id, count, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
           [&](int, const auto& refill) {
-            full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
+            full_tile<D, true>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k, ring));
           },
           [&](int tag, const auto& refill) {
-            full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k));
+            full_tile<D>(st, ring, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k, ring));
           },
           [&](int tag, const auto& refill) {
-            tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k));
+            tail_tile<D, !KT, true>(st, ring, tag >> 1, tk, true, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k, ring));
           });
     } else {
       if (p.force == 1) {
@@ -1258,35 +1261,38 @@ struct SplitCursor {
 // chain (a query-sink block's chain is every key block).  Here KS groups of
 // two waves share a query block: wave (grp, qh) owns queries 32 qh .. +31 of
 // it, and group grp attends exact tiles grp, grp + KS, ... of its selected
-// blocks through a two-slot ring of its own, every group stepping in the
-// same workgroup barrier, so a chain of n tiles takes ceil(n / KS) steps.
-// Group 0 routes and adds the centroid contributions (skipped for a tile
-// with no approximated block); at the end every group publishes its
-// online-softmax state in LDS and merges and stores a share of the output
-// features (m = max m_g, acc and den weighted by 2^(m_g - m), groups in
-// order).  Decisions, counts and diagnostics are the
+// blocks through a K slot and a V slot of its own (SlotStep), every group
+// stepping in the same workgroup barriers, so a chain of n tiles takes ceil(n
+// / KS) steps.  Centroid tiles come first, group grp routing and attending
+// tiles grp, grp + KS, ...; the first of them travel while Q is staged and the
+// cutoff formed.  At the end every group publishes its online-softmax state
+// in LDS and merges and stores a share of the output features (m = max m_g,
+// acc and den weighted by 2^(m_g - m), groups in order).  Decisions, counts and diagnostics are the
 // one-block kernel's; the output agrees with it to rounding (other partial
 // sums).  POOL (plain K / V rows, at most one pooling chunk of key blocks,
 // no centroid tiles given): every workgroup forms its head's block centroids
 // and diagonal moments in LDS in the pooling kernel's order and arithmetic
 // (bit-identical values), so the whole call is this one launch.  Finite and
 // +inf beta only (beta = -inf launches take sol_attention_kernel).
-// The ring takes ~130 KB of LDS: one workgroup per CU, KS / 2 waves per SIMD.
+// The slots take 32 KB per group at head_dim 128 (16 at 64): four groups per
+// CU, two waves per SIMD, in 256 vector registers.  (Two-slot rings left room
+// for two groups at head_dim 128, one wave per SIMD, whose accumulators lay in
+// AGPRs and were copied to and fro: @@SMALL@@.)
 template <int D, int KS, bool KT, bool POOL>
-__global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams p) {
+__global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   using S = Shape<D>;
   using TL = TileLayout<D>;
   constexpr int NT = 128 * KS;
   constexpr int kMaskWords = kMaxKeyBlocks / 32;
   constexpr int NC = S::DT * 4;            // 4-feature output chunks per lane
-  constexpr int kStateFloats = 4 * NC + 2;  // per lane: acc, m, den
   constexpr int QPT = kBlock * S::DC / NT;  // Q staging chunks per thread
   static_assert(!POOL || !KT, "in-kernel pooling reads plain K / V rows");
   static_assert(QPT * NT == kBlock * S::DC, "Q rows split evenly over the workgroup");
-  static_assert(KS * 2 * kWave * kStateFloats * 4 <= 2 * KS * S::TILE * 2, "merge records fit the ring");
-  // Group g's ring slots at 2 g TILE (the centroid pass streams through the
-  // first two); Q staging and the pooled centroid tile alias them early on.
-  __shared__ __align__(256) uint16_t ring[2 * KS * S::TILE];
+  static_assert(KS * 2 * kWave * 4 * NC * 4 <= KS * S::TILE * 2, "the groups' accumulators fit the slots");
+  // Group g's slots at g TILE; the Q staging aliases the last group's, the
+  // pooled centroid tile is formed in the first one's.
+  __shared__ __align__(256) uint16_t ring[KS * S::TILE];
+  __shared__ float s_md[KS][2][2][kWave];  // the groups' m and den
   __shared__ float s_qm[D];
   __shared__ __align__(16) uint16_t s_qb[4 * kRouteRow<D>];  // its BF16 terms (route_word)
   __shared__ float s_red[4];
@@ -1307,10 +1313,23 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
   const int qlen = min(kBlock, p.Tq - qb * kBlock);
   const float scale_log2 = p.scale_log2;
   const bool routed = p.mask != nullptr;
-  uint16_t* const ctile = ring + S::TILE;  // the pooled centroid tile (slot 1)
+  uint16_t* const ctile = ring;  // POOL: the pooled centroid tile
+  uint16_t* const stage = ring + (KS - 1) * S::TILE;
+  uint16_t* const slot = ring + grp * S::TILE;
+  const uint32_t slot_lds = lds_address(slot);
+  const int wg = wave & 1;  // the wave inside its group
+  const int nct = POOL ? 1 : (nkb + kBlock - 1) / kBlock;
+  const uint16_t* ctiles = p.ctiles + head * p.NCT * S::TILE;
+  const auto crefill = bf16_refills<D, 128>([=](int ct) { return ctiles + int64_t(ct) * S::TILE; }, wg, lane);
+  constexpr int kHalfRounds = TileRefill<D, 128>::kRounds / 2;
+  if (!POOL && grp < KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
 
-  // 1. Q rows -> LDS (slot 0) -> fragments; with POOL, the head's centroids
-  // -> slot 1 in the tile layout (rows past the last block zero).  Every
+  // This thread's feature of the key moments: its loads travel with Q's.
+  KeyMoments<D> km;
+  if (!POOL && p.force == 0 && !routed && tid < D) km.load(p, head, tid);
+
+  // 1. Q rows -> LDS -> fragments; with POOL, the head's centroids -> group
+  // 0's slot in the tile layout (rows past the last block zero).  Every
   // global load is issued before the first LDS store that waits on one.
   u32x4 qx[QPT];
 #pragma unroll
@@ -1323,7 +1342,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
 #pragma unroll
     for (int i = 0; i < QPT; ++i) {
       const int idx = tid + i * NT, r = idx / S::DC, c = idx % S::DC;
-      *reinterpret_cast<u32x4*>(ring + r * S::KS + 8 * c) = qx[i];
+      *reinterpret_cast<u32x4*>(stage + r * S::KS + 8 * c) = qx[i];
     }
   };
   // Pooling units: block jb of K (u < 16) or of V (u - 16), 16 rows x 16
@@ -1416,7 +1435,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
   __syncthreads();
   bf16x8 qf[S::KT];
   {
-    const uint16_t* qrow = ring + myq * S::KS;
+    const uint16_t* qrow = stage + myq * S::KS;
 #pragma unroll
     for (int ks = 0; ks < S::KT; ++ks)
       qf[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(qrow + ks * 16 + 8 * hh));
@@ -1443,9 +1462,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
   // thread forms the cutoff from the published sums).
   float cut = 0.f;
   if (p.force == 0 && !routed) {
-    KeyMoments<D> km;  // this thread's feature of the key moments (pooled here: below)
-    if (!POOL && tid < D) km.load(p, head, tid);
-    if (tid < D) s_qm[tid] = query_mean<D>(ring, qlen, tid);
+    if (tid < D) s_qm[tid] = query_mean<D>(stage, qlen, tid);
     __syncthreads();  // also: every read of the Q staging rows is done
     float a = 0.f, g = 0.f;
     if (tid < D) {
@@ -1477,7 +1494,7 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
     __syncthreads();
     cut = cutoff_value(p, s_red[0], s_red[1], s_red[2], s_red[3]);
   } else {
-    __syncthreads();  // every wave's Q fragments are read: the ring is free
+    __syncthreads();  // every wave's Q fragments are read: the staging is dead
   }
   const int64_t dbg_row = ((int64_t(b) * p.NQB + qb) * p.H + h) * p.NKB;
   if (p.dbg_cutoff && tid == 0 && !routed)
@@ -1486,93 +1503,76 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
   State<D> st;
   state_init(st);
   const int nwords = (nkb + 31) / 32;
-  {
-    // 3. Centroid pass (group 0 attends; every wave takes part in the
-    // barriers and the ring's DMA).  Launches at beta = -inf take
-    // sol_attention_kernel.
-    if (routed) {
-      for (int w = tid; w < nwords; w += NT) s_mask[w] = p.mask[(head * p.NQB + qb) * p.NW + w];
-      __syncthreads();
-    }
-    if constexpr (POOL) {
-      // The one centroid tile sits in slot 1: route from it now (and finish
-      // its V rows); its contributions run in the exact stream's prologue,
-      // over the first exact tiles' DMA (group 0's first slot is slot 0).
-      if (!routed && grp == 0) {
-        const uint32_t word = route_word<D>(p, lds_centroids<D>(ctile, qh, lane), s_qb, cut, 32 * qh, 0, nkb, b, qb,
-                                            lane, dbg_row);
-        if (lane == 0) s_mask[qh] = word;
-      }
-      if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
-      lds_barrier();  // publishes the mask words and the V centroids
-    } else {
-      auto process = [&](const uint16_t* buf, int ct, const auto& refill) {
-        if (!routed) {
-          if (grp == 0) {
-            const uint32_t word = route_word<D>(p, lds_centroids<D>(buf, qh, lane), s_qb, cut, kBlock * ct + 32 * qh, 0, nkb,
-                                                b, qb, lane, dbg_row);
-            if (lane == 0) s_mask[2 * ct + qh] = word;
-          }
-          lds_barrier();  // publishes the mask words
-        }
-        // The workgroup's one query block decides for every wave: a tile
-        // without approximated blocks (a query-sink block's) is skipped.
-        const uint64_t approx = tile_approx(s_mask, ct, 0, nkb);
-        if (grp == 0 && approx != 0ull) {
-          centroid_tile<D>(st, buf, ct, approx, tk, qf, col, hh, scale_log2, ring_step(refill));
-        } else {
-          refill.all();
-        }
-      };
-      const uint16_t* ctiles = p.ctiles + head * p.NCT * S::TILE;
-      auto always = [](int) { return true; };
-      const auto crefill = bf16_refills<D, NT>([=](int ct) { return ctiles + int64_t(ct) * S::TILE; }, wave, lane);
-      tile_stream<D, NT, 2>(ring, (nkb + kBlock - 1) / kBlock, RangeCursor{0}, crefill,
-                            tile_runs(always, process, process), process, wave, lane);
-      lds_barrier();  // the ring's centroid tiles and the masks are settled
-    }
+  if (routed) {
+    for (int w = tid; w < nwords; w += NT) s_mask[w] = p.mask[(head * p.NQB + qb) * p.NW + w];
+    __syncthreads();
   }
+
+  // 3. Centroid tiles grp, grp + KS, ...: routed by their group, then attended
+  // while the group's next tile -- another centroid tile or, after the last
+  // round, its first exact tile -- travels.  A group past the last centroid
+  // tile goes through that one again with no block of it approximated (it
+  // adds nothing), so that all groups meet at the same barriers.  (Launches
+  // at beta = -inf take sol_attention_kernel.)
+  const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
+  const auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
+  u32x4 k[2][S::KT];
+  if (!POOL && grp == KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
+  if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
+  const uint16_t* const cslot = POOL ? ctile : slot;
+  slot_prime<D, 2 * kHalfRounds>(cslot, k, col, hh);
+  SplitCursor<KS> cursor{UnionCursor<1>{s_mask, s_mask, kMaskWords, 0, nkb, 0}, grp};
+  auto centroids = [&](auto&& fn) {
+    return qh ? fn([&](int ks) { return k[1][ks]; }) : fn([&](int ks) { return k[0][ks]; });
+  };
+  auto approximated = [&](int ct) {
+    if (!routed) {
+      if (ct < nct) {
+        const uint32_t word = centroids([&](const auto& kfrag) {
+          return route_word<D>(p, kfrag, s_qb, cut, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+        });
+        if (lane == 0) s_mask[2 * ct + qh] = word;
+      }
+      lds_barrier();  // publishes the mask words
+    }
+    return ct < nct ? tile_approx(s_mask, ct, 0, nkb) : 0ull;
+  };
+  int ct = grp;
+  if (!POOL)
+    for (; ct - grp + KS < nct; ct += KS)
+      centroid_tile<D, true>(st, slot, ct, approximated(ct), tk, qf, col, hh, scale_log2,
+                             slot_step<D>(crefill(min(ct + KS, nct - 1), slot_lds), NoFrag{}, k, slot));
+  const uint64_t approx = approximated(ct);
+  const int steps = (cursor.all.count() + KS - 1) / KS;
+  const int id = cursor();
+  centroid_tile<D, true>(st, cslot, min(ct, nct - 1), approx, tk, qf, col, hh, scale_log2,
+                         slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot));
   int nsel = 0;
   if (p.counts && tid == 0)
     for (int w = 0; w < nwords; ++w) nsel += __builtin_popcount(s_mask[w] & uint32_t(bit_range64(0, nkb - 32 * w)));
 
   // 4. Exact pass: group grp's share of the selected blocks, ascending.
-  {
-    UnionCursor<1> all{s_mask, s_mask, kMaskWords, 0, nkb, 0};
-    const int steps = (all.count() + KS - 1) / KS;
-    const int wg = wave & 1;  // the wave inside its group
-    const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
-    auto selected = [](int tag) { return (tag & 1) != 0; };
-    auto hit = [&](const uint16_t* buf, int, const auto& refill) {
-      full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
-    };
-    auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
-    tile_stream<D, 128, 2>(
-        ring + grp * 2 * S::TILE, steps, SplitCursor<KS>{all, grp},
-        [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); }, tile_runs(selected, hit, miss),
-        [&](const uint16_t* buf, int tag, const auto& refill) {
-          if (tag & 1) {
-            exact_tile<D, !KT>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
-          } else {
-            refill.all();
-          }
-        },
-        wg, lane, [&] {
-          if constexpr (POOL) {
-            const uint64_t approx = tile_approx(s_mask, 0, 0, nkb);
-            if (grp == 0 && approx != 0ull)
-              centroid_tile<D>(st, ctile, 0, approx, tk, qf, col, hh, scale_log2, ring_step(NoRefill{}));
-          }
-        });
-  }
+  const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
+  slot_stream(
+      slot_lds, id, steps, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
+      [&](int, const auto& refill) {
+        full_tile<D, true>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k, slot));
+      },
+      [&](int tag, const auto& refill) {
+        full_tile<D>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k, slot));
+      },
+      [&](int tag, const auto& refill) {
+        tail_tile<D, !KT, true>(st, slot, tag >> 1, tk, (tag & 1) != 0, qf, col, hh, scale_log2,
+                                slot_step<D>(refill, NoFrag{}, k, slot));
+      });
 
   // 5. Merge and store, spread over the groups: every group publishes its
   // state; group g then combines output chunks c = g, g + KS, ... of every
   // state -- O = sum_s 2^(m_s - m) acc_s / sum_s 2^(m_s - m) den_s, m =
   // max_s m_s, states in order -- and stores them (store_output's rows).
-  __syncthreads();  // every group's stream is done with the ring
+  __syncthreads();  // every group's stream is done with the slots
   float* rec = reinterpret_cast<float*>(ring);
-  auto state = [&](int g) { return rec + (g * 2 + qh) * (kWave * kStateFloats); };
+  auto state = [&](int g) { return rec + (g * 2 + qh) * (kWave * 4 * NC); };
   {
     float* mine = state(grp);
 #pragma unroll
@@ -1582,23 +1582,24 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       for (int i = 0; i < 4; ++i) x[i] = st.acc[c / 4][4 * (c % 4) + i];
       *reinterpret_cast<f32x4*>(mine + (c * kWave + lane) * 4) = x;
     }
-    mine[4 * NC * kWave + lane] = st.m;
-    mine[4 * NC * kWave + kWave + lane] = st.den;
+    s_md[grp][qh][0][lane] = st.m;
+    s_md[grp][qh][1][lane] = st.den;
   }
   __syncthreads();
   float ms[KS], m = kNegInf;
 #pragma unroll
   for (int g = 0; g < KS; ++g) {
-    ms[g] = state(g)[4 * NC * kWave + lane];
+    ms[g] = s_md[g][qh][0][lane];
     m = fmaxf(m, ms[g]);
   }
   float w[KS], den = 0.f;
 #pragma unroll
   for (int g = 0; g < KS; ++g) {
     w[g] = ms[g] == kNegInf ? 0.f : fast_exp2(ms[g] - m);
-    den = den + w[g] * state(g)[4 * NC * kWave + kWave + lane];
+    den = den + w[g] * s_md[g][qh][1][lane];
   }
   den = pair_sum(den);
+  const float inv = __fdiv_rn(1.f, den);  // one division per row, as store_output
   if (p.counts && tid == 0) p.counts[(int64_t(b) * p.NQB + qb) * p.H + h] = nsel;
   const int t = qb * kBlock + myq;
   if (t >= p.Tq) return;
@@ -1618,8 +1619,8 @@ __global__ __launch_bounds__(128 * KS, KS / 2) void sol_small_kernel(AttnParams 
       for (int i = 0; i < 4; ++i) o[i] = o[i] + w[g] * x[i];
     }
     u32x2 v;
-    v[0] = pack_bf16x2(__fdiv_rn(o[0], den), __fdiv_rn(o[1], den));
-    v[1] = pack_bf16x2(__fdiv_rn(o[2], den), __fdiv_rn(o[3], den));
+    v[0] = pack_bf16x2(o[0] * inv, o[1] * inv);
+    v[1] = pack_bf16x2(o[2] * inv, o[3] * inv);
     *reinterpret_cast<u32x2*>(orow + (c / 4) * 32 + 8 * (c % 4) + 4 * hh) = v;
   }
 }
@@ -1858,10 +1859,10 @@ void launch_small(const AttnParams& p, hipStream_t stream) {
   const dim3 grid(unsigned(p.B * p.H * p.NQB)), block(128 * KS);
   if (p.tiles)
     hipLaunchKernelGGL((sol_small_kernel<D, KS, true, false>), grid, block, 0, stream, p);
-  else if (!p.ctiles)
-    hipLaunchKernelGGL((sol_small_kernel<D, KS, false, true>), grid, block, 0, stream, p);
-  else
+  else if (p.ctiles)
     hipLaunchKernelGGL((sol_small_kernel<D, KS, false, false>), grid, block, 0, stream, p);
+  else if constexpr (D == 64 && KS == 4)  // sol_attention_pools_keys
+    hipLaunchKernelGGL((sol_small_kernel<D, KS, false, true>), grid, block, 0, stream, p);
 }
 
 hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
@@ -1877,12 +1878,13 @@ hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
   // beta = -inf keep sol_attention_kernel, whose every-block-exact path
   // equals the dense kernel bit for bit.
   const int ks = p.workgroup_form == 0 && !p.k8 && p.splits == 1 && p.force != 1
-                     ? small_key_split(int64_t(p.B) * p.H * p.NQB, p.NKB, D) : 0;
+                     ? small_key_split(int64_t(p.B) * p.H * p.NQB, p.NKB, p.q_sink_blocks, D) : 0;
   if (ks) {
-    if (D == 128)
-      launch_small<128, 2>(p, stream);
-    else
-      launch_small<64, 4>(p, stream);
+    if (D == 128) {
+      if (ks == 4) launch_small<128, 4>(p, stream); else launch_small<128, 2>(p, stream);
+    } else {
+      if (ks == 4) launch_small<64, 4>(p, stream); else launch_small<64, 2>(p, stream);
+    }
     return hipGetLastError();
   }
   // AttnParams::workgroup_form 1 or 2 forces one form (tests run both: results are bit-identical -- a wave's

@@ -124,7 +124,7 @@ int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int
                           (bh * nqb <= 2048 && nkb >= 128 && sol::one_block_launch(bh, nqb, nkb, head_dim));
   // Launches of the small kernel split every query block's chain inside its
   // workgroup instead.
-  if (sol::small_key_split(bh * nqb, nkb, head_dim)) return 1;
+  if (sol::small_key_split(bh * nqb, nkb, q_sink_blocks, head_dim)) return 1;
   if (force == 1 || q_sink_blocks < 2 || 4 * q_sink_blocks > nqb || nkb > sol::kMaxKeyBlocks ||
       !(few_groups || (force == 2 && bh * nqb <= 8192)))
     return 1;
@@ -143,7 +143,7 @@ int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int
 bool pools_keys(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads, int64_t head_dim) {
   const int64_t nkb = cdiv(key_tokens, SOL_BLOCK);
   return head_dim == 64 && key_tokens >= SOL_BLOCK && nkb <= sol::kPoolChunk &&
-         sol::small_key_split(batch * heads * cdiv(query_tokens, SOL_BLOCK), nkb, head_dim) > 0;
+         batch * heads * cdiv(query_tokens, SOL_BLOCK) <= sol::kSmallBlocks;
 }
 
 int64_t sink_blocks(int64_t query_sink_tokens) {

@@ -135,17 +135,19 @@ struct QuantParams {
 
 // Key-split groups of sol_small_kernel for a launch of `blocks` query blocks
 // (over all entries and heads) against nkb key blocks, or 0 when the launch
-// takes sol_attention_kernel.  Small launches (at most kSmallBlocks query
-// blocks, a workgroup each) leave most SIMDs idle, so their time is one
-// workgroup's tile chain: KS groups of two waves split it KS ways, within the
-// LDS of two ring slots per group (4 groups at D = 64, 2 at D = 128), while
-// the chain stays at most kSmallChain steps.  Longer key sequences go to the
-// one-block kernel, whose query-sink tiles split over workgroups instead.
+// takes sol_attention_kernel.  Small launches leave most SIMDs idle, so their
+// time is one workgroup's tile chain: KS groups of two waves split it KS ways,
+// four while a CU holds one workgroup (at most kSmallBlocks query blocks), two
+// while it holds two.  A query-sink block's chain is every key block: with two
+// or more of them, over keys of more than kSmallChain steps, the launch goes
+// to the one-block kernel, whose sink tiles split over workgroups instead (a
+// single sink block is not split there).  @@RULE@@
 constexpr int64_t kSmallBlocks = 256;
-constexpr int64_t kSmallChain = 16;
-inline int small_key_split(int64_t blocks, int64_t nkb, int64_t head_dim) {
-  const int ks = head_dim == 64 ? 4 : 2;
-  return blocks <= kSmallBlocks && nkb <= kSmallChain * ks ? ks : 0;
+constexpr int64_t kSmallChain = 8;  // at head_dim 128; twice that at 64
+inline int small_key_split(int64_t blocks, int64_t nkb, int64_t q_sink_blocks, int64_t head_dim) {
+  const int ks = blocks <= kSmallBlocks ? 4 : 2;
+  if (blocks > 2 * kSmallBlocks || nkb > kMaxKeyBlocks) return 0;
+  return q_sink_blocks < 2 || nkb <= kSmallChain * ks * (128 / head_dim) ? ks : 0;
 }
 
 // K and V bytes of one head's key blocks.
