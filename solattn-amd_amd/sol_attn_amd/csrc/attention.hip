@@ -1277,7 +1277,13 @@ struct SplitCursor {
 // The slots take 32 KB per group at head_dim 128 (16 at 64): four groups per
 // CU, two waves per SIMD, in 256 vector registers.  (Two-slot rings left room
 // for two groups at head_dim 128, one wave per SIMD, whose accumulators lay in
-// AGPRs and were copied to and fro: @@SMALL@@.)
+// AGPRs and were copied to and fro: 1,024 x 4 heads 17.4 us against 15.5,
+// 4,096 x 4 27.4 against 23.0.)
+// POOL launches (head_dim 64, at most four tiles per group) keep rings of two
+// slots, 128 KB: with chains this short the four workgroup barriers of a
+// one-slot tile cost more than its fragments' early reads save, and every
+// group would go through the centroid tile that here is group 0's alone
+// (1,024 x 8 heads 17.6 us per call against 20.2).
 template <int D, int KS, bool KT, bool POOL>
 __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   using S = Shape<D>;
@@ -1289,9 +1295,10 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   static_assert(!POOL || !KT, "in-kernel pooling reads plain K / V rows");
   static_assert(QPT * NT == kBlock * S::DC, "Q rows split evenly over the workgroup");
   static_assert(KS * 2 * kWave * 4 * NC * 4 <= KS * S::TILE * 2, "the groups' accumulators fit the slots");
-  // Group g's slots at g TILE; the Q staging aliases the last group's, the
-  // pooled centroid tile is formed in the first one's.
-  __shared__ __align__(256) uint16_t ring[KS * S::TILE];
+  // Group g's slots at g SLOTS TILE; the Q staging aliases the last group's.
+  // POOL: the centroid tile is formed in group 0's second slot.
+  constexpr int SLOTS = POOL ? 2 : 1;
+  __shared__ __align__(256) uint16_t ring[SLOTS * KS * S::TILE];
   __shared__ float s_md[KS][2][2][kWave];  // the groups' m and den
   __shared__ float s_qm[D];
   __shared__ __align__(16) uint16_t s_qb[4 * kRouteRow<D>];  // its BF16 terms (route_word)
@@ -1313,9 +1320,9 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   const int qlen = min(kBlock, p.Tq - qb * kBlock);
   const float scale_log2 = p.scale_log2;
   const bool routed = p.mask != nullptr;
-  uint16_t* const ctile = ring;  // POOL: the pooled centroid tile
-  uint16_t* const stage = ring + (KS - 1) * S::TILE;
-  uint16_t* const slot = ring + grp * S::TILE;
+  uint16_t* const ctile = ring + S::TILE;  // POOL: the pooled centroid tile
+  uint16_t* const stage = ring + SLOTS * (KS - 1) * S::TILE;
+  uint16_t* const slot = ring + grp * SLOTS * S::TILE;
   const uint32_t slot_lds = lds_address(slot);
   const int wg = wave & 1;  // the wave inside its group
   const int nct = POOL ? 1 : (nkb + kBlock - 1) / kBlock;
@@ -1329,7 +1336,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   if (!POOL && p.force == 0 && !routed && tid < D) km.load(p, head, tid);
 
   // 1. Q rows -> LDS -> fragments; with POOL, the head's centroids -> group
-  // 0's slot in the tile layout (rows past the last block zero).  Every
+  // 0's second slot in the tile layout (rows past the last block zero).  Every
   // global load is issued before the first LDS store that waits on one.
   u32x4 qx[QPT];
 #pragma unroll
@@ -1508,63 +1515,92 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
     __syncthreads();
   }
 
-  // 3. Centroid tiles grp, grp + KS, ...: routed by their group, then attended
-  // while the group's next tile -- another centroid tile or, after the last
-  // round, its first exact tile -- travels.  A group past the last centroid
-  // tile goes through that one again with no block of it approximated (it
-  // adds nothing), so that all groups meet at the same barriers.  (Launches
-  // at beta = -inf take sol_attention_kernel.)
   const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
   const auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
-  u32x4 k[2][S::KT];
-  if (!POOL && grp == KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
-  if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
-  const uint16_t* const cslot = POOL ? ctile : slot;
-  slot_prime<D, 2 * kHalfRounds>(cslot, k, col, hh);
   SplitCursor<KS> cursor{UnionCursor<1>{s_mask, s_mask, kMaskWords, 0, nkb, 0}, grp};
-  auto centroids = [&](auto&& fn) {
-    return qh ? fn([&](int ks) { return k[1][ks]; }) : fn([&](int ks) { return k[0][ks]; });
-  };
-  auto approximated = [&](int ct) {
-    if (!routed) {
-      if (ct < nct) {
-        const uint32_t word = centroids([&](const auto& kfrag) {
-          return route_word<D>(p, kfrag, s_qb, cut, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
-        });
-        if (lane == 0) s_mask[2 * ct + qh] = word;
-      }
-      lds_barrier();  // publishes the mask words
+  if constexpr (POOL) {
+    // 3. Group 0 routes from the centroid tile (and the V centroids are
+    // finished); its contributions run in the exact stream's prologue, over
+    // the first exact tiles' DMA.
+    if (!routed && grp == 0) {
+      const uint32_t word = route_word<D>(p, lds_centroids<D>(ctile, qh, lane), s_qb, cut, 32 * qh, 0, nkb, b, qb,
+                                          lane, dbg_row);
+      if (lane == 0) s_mask[qh] = word;
     }
-    return ct < nct ? tile_approx(s_mask, ct, 0, nkb) : 0ull;
-  };
-  int ct = grp;
-  if (!POOL)
+    if constexpr (kLateV) finish_unit(u_first + PER_PASS, xv, len_v);
+    lds_barrier();  // publishes the mask words and the V centroids
+    // 4. Exact pass: group grp's share of the selected blocks, ascending.
+    const int steps = (cursor.all.count() + KS - 1) / KS;
+    auto hit = [&](const uint16_t* buf, int, const auto& refill) {
+      full_tile<D>(st, buf, qf, col, hh, scale_log2, ring_step(refill));
+    };
+    auto miss = [&](const uint16_t*, int, const auto& refill) { refill.all(); };
+    tile_stream<D, 128, SLOTS>(
+        slot, steps, cursor, make, tile_runs([](int tag) { return (tag & 1) != 0; }, hit, miss),
+        [&](const uint16_t* buf, int tag, const auto& refill) {
+          if (tag & 1) {
+            exact_tile<D, true>(st, buf, tag >> 1, tk, qf, col, hh, scale_log2, ring_step(refill));
+          } else {
+            refill.all();
+          }
+        },
+        wg, lane, [&] {
+          const uint64_t approx = tile_approx(s_mask, 0, 0, nkb);
+          if (grp == 0 && approx != 0ull)
+            centroid_tile<D>(st, ctile, 0, approx, tk, qf, col, hh, scale_log2, ring_step(NoRefill{}));
+        });
+  } else {
+    // 3. Centroid tiles grp, grp + KS, ...: routed by their group, then attended
+    // while the group's next tile -- another centroid tile or, after the last
+    // round, its first exact tile -- travels.  A group past the last centroid
+    // tile goes through that one again with no block of it approximated (it
+    // adds nothing), so that all groups meet at the same barriers.  (Launches
+    // at beta = -inf take sol_attention_kernel.)
+    u32x4 k[2][S::KT];
+    if (grp == KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
+    slot_prime<D, 2 * kHalfRounds>(slot, k, col, hh);
+    auto centroids = [&](auto&& fn) {
+      return qh ? fn([&](int ks) { return k[1][ks]; }) : fn([&](int ks) { return k[0][ks]; });
+    };
+    auto approximated = [&](int ct) {
+      if (!routed) {
+        if (ct < nct) {
+          const uint32_t word = centroids([&](const auto& kfrag) {
+            return route_word<D>(p, kfrag, s_qb, cut, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
+          });
+          if (lane == 0) s_mask[2 * ct + qh] = word;
+        }
+        lds_barrier();  // publishes the mask words
+      }
+      return ct < nct ? tile_approx(s_mask, ct, 0, nkb) : 0ull;
+    };
+    int ct = grp;
     for (; ct - grp + KS < nct; ct += KS)
       centroid_tile<D, true>(st, slot, ct, approximated(ct), tk, qf, col, hh, scale_log2,
                              slot_step<D>(crefill(min(ct + KS, nct - 1), slot_lds), NoFrag{}, k, slot));
-  const uint64_t approx = approximated(ct);
-  const int steps = (cursor.all.count() + KS - 1) / KS;
-  const int id = cursor();
-  centroid_tile<D, true>(st, cslot, min(ct, nct - 1), approx, tk, qf, col, hh, scale_log2,
-                         slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot));
+    const uint64_t approx = approximated(ct);
+    const int steps = (cursor.all.count() + KS - 1) / KS;
+    const int id = cursor();
+    centroid_tile<D, true>(st, slot, min(ct, nct - 1), approx, tk, qf, col, hh, scale_log2,
+                           slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot));
+    // 4. Exact pass: group grp's share of the selected blocks, ascending.
+    const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
+    slot_stream(
+        slot_lds, id, steps, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
+        [&](int, const auto& refill) {
+          full_tile<D, true>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k, slot));
+        },
+        [&](int tag, const auto& refill) {
+          full_tile<D>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k, slot));
+        },
+        [&](int tag, const auto& refill) {
+          tail_tile<D, !KT, true>(st, slot, tag >> 1, tk, (tag & 1) != 0, qf, col, hh, scale_log2,
+                                  slot_step<D>(refill, NoFrag{}, k, slot));
+        });
+  }
   int nsel = 0;
   if (p.counts && tid == 0)
     for (int w = 0; w < nwords; ++w) nsel += __builtin_popcount(s_mask[w] & uint32_t(bit_range64(0, nkb - 32 * w)));
-
-  // 4. Exact pass: group grp's share of the selected blocks, ascending.
-  const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
-  slot_stream(
-      slot_lds, id, steps, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },
-      [&](int, const auto& refill) {
-        full_tile<D, true>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, NoFrag{}, k, slot));
-      },
-      [&](int tag, const auto& refill) {
-        full_tile<D>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k, slot));
-      },
-      [&](int tag, const auto& refill) {
-        tail_tile<D, !KT, true>(st, slot, tag >> 1, tk, (tag & 1) != 0, qf, col, hh, scale_log2,
-                                slot_step<D>(refill, NoFrag{}, k, slot));
-      });
 
   // 5. Merge and store, spread over the groups: every group publishes its
   // state; group g then combines output chunks c = g, g + KS, ... of every

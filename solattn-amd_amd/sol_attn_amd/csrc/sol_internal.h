@@ -141,7 +141,7 @@ struct QuantParams {
 // while it holds two.  A query-sink block's chain is every key block: with two
 // or more of them, over keys of more than kSmallChain steps, the launch goes
 // to the one-block kernel, whose sink tiles split over workgroups instead (a
-// single sink block is not split there).  @@RULE@@
+// single sink block is not split there).
 constexpr int64_t kSmallBlocks = 256;
 constexpr int64_t kSmallChain = 8;  // at head_dim 128; twice that at 64
 inline int small_key_split(int64_t blocks, int64_t nkb, int64_t q_sink_blocks, int64_t head_dim) {
