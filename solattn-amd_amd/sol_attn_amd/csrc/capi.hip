@@ -101,17 +101,16 @@ int64_t route_mask_bytes(int64_t batch, int64_t query_tokens, int64_t key_tokens
 // query-sink block selects every key block, so its workgroup streams all of
 // them and, in a launch of few workgroups, ends long after the rest.  Split:
 // launches of fewer than 512 query-block pairs over all (entry, head) pairs,
-// and one-block launches of at most 2,048 query blocks over at least 128 key
-// blocks (8,192 tokens x 16 heads 210 -> 188), at finite beta, and at beta = +inf (every other workgroup streams its protected blocks only)
-// launches of up to 8,192 query blocks (8 rounds of 512 two-block
-// workgroups).  Parts hold at least 16 key blocks, at most 8 parts, while
-// their partial states fit kSplitBytesMax.  Measured (us per call, 4 heads,
-// beta 1): 4,096 tokens 97 -> 60, 8,192 tokens 172 -> 108; at 2 x 4,096 x 16
-// heads beta +inf 109 -> 91, while beta 0 or 1 there (128 -> 137) and more
-// rounds of workgroups (8,192 x 24 heads 257 -> 270) lose: the other
-// workgroups fill the time, and the merge comes on top.  beta = -inf (every block exact),
-// fewer than two sink blocks and sinks over a quarter of the query blocks
-// are not split.
+// one-block launches at finite beta of at most 2,048 query blocks over at least
+// 128 key blocks (8,192 tokens x 16 heads beta 1 210 -> 188, beta 0 343 ->
+// 335), or whose sink chain is at least twice the steps a workgroup slot has
+// on average (sink_chain_ratio), and at beta = +inf (every other workgroup
+// streams its protected blocks only) launches of up to 8,192 query blocks (8
+// rounds of 512 two-block workgroups).  Parts hold at least 16 key blocks, at
+// most 8 parts, while their partial states fit kSplitBytesMax.  Otherwise the
+// other workgroups fill the time, and the merge comes on top (2 x 4,096 x 16
+// heads beta 1 116 -> 123).  beta = -inf (every block exact), fewer than two
+// sink blocks and sinks over a quarter of the query blocks are not split.
 constexpr int64_t kSplitBytesMax = int64_t(64) << 20;
 
 int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t head_dim) {
@@ -119,9 +118,30 @@ int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t h
   return splits > 1 ? bh * (q_sink_blocks / 2 * 2) * SOL_BLOCK * splits * (head_dim + 4) * 4 : 0;
 }
 
-int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, int64_t head_dim) {
+// Steps of a query-sink block's chain (every key block) over the steps each
+// of a one-block launch's workgroup slots (256 CUs x 4 at head_dim 128, x 6 at
+// 64) has on average.  A regular block takes the share of a normal above beta
+// (what the threshold aims at), its centroid tiles, and about 8 steps' time
+// for its local blocks, staging and cutoff.  us per call, 128-token sinks, not
+// split -> split, with the ratio: 4,096 x 16 heads x D128 beta 1 (3.3) 92 ->
+// 80, beta 0 (1.6) 108 -> 119; 2 x 4,096 x 16 beta 1 (1.6) 116 -> 123; 4,096 x
+// 24 (2.2) 101 -> 99; 6,000 x 16 (2.6) 126 -> 117; D64: 6,000 x 20 (3.1) 102
+// -> 91, 4,096 x 32 (2.4) 78 -> 77.
+double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, double beta, int64_t head_dim) {
+  const double slots = head_dim == 64 ? 1536 : 1024;
+  const double share = 0.5 * std::erfc(beta / std::sqrt(2.0));
+  const double regular = share * double(nkb) + double(nkb) / SOL_BLOCK + 8;
+  const double sinks = double(std::min(q_sink_blocks, nqb));
+  const double steps = double(bh) * (sinks * double(nkb) + (double(nqb) - sinks) * regular);
+  return double(nkb) * slots / steps;
+}
+
+int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, double beta,
+                int64_t head_dim) {
   const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
-                          (bh * nqb <= 2048 && nkb >= 128 && sol::one_block_launch(bh, nqb, nkb, head_dim));
+                          (force == 0 && sol::one_block_launch(bh, nqb, nkb, head_dim) &&
+                           ((bh * nqb <= 2048 && nkb >= 128) ||
+                            sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2));
   // Launches of the small kernel split every query block's chain inside its
   // workgroup instead.
   if (sol::small_key_split(bh * nqb, nkb, q_sink_blocks, head_dim)) return 1;
@@ -416,7 +436,7 @@ int64_t sol_split_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
     return 0;
   const int64_t bh = batch * heads, nqb = cdiv(query_tokens, SOL_BLOCK), qsb = sink_blocks(query_sink_tokens);
   const int force = std::isinf(beta) ? (beta < 0 ? 1 : 2) : 0;
-  const int s = sink_splits(bh, nqb, cdiv(key_tokens, SOL_BLOCK), qsb, force, head_dim);
+  const int s = sink_splits(bh, nqb, cdiv(key_tokens, SOL_BLOCK), qsb, force, beta, head_dim);
   return split_bytes(bh, qsb, s, head_dim);
 }
 
@@ -675,7 +695,7 @@ int attention_fwd_impl(const void* q, const int64_t* q_strides, const int64_t* q
   p.local_blocks = int(local_blocks < 0 ? -1 : (local_blocks > big ? big : local_blocks));
   p.kv_sink_blocks = int(cdiv(kv_sink_tokens > big ? big : kv_sink_tokens, SOL_BLOCK));
   p.q_sink_blocks = int(sink_blocks(query_sink_tokens));
-  p.splits = split_workspace ? sink_splits(batch * heads, nqb, nkb, p.q_sink_blocks, force, head_dim) : 1;
+  p.splits = split_workspace ? sink_splits(batch * heads, nqb, nkb, p.q_sink_blocks, force, beta, head_dim) : 1;
   p.partial = p.splits > 1 ? static_cast<float*>(split_workspace) : nullptr;
   p.mask = force != 1 ? static_cast<uint32_t*>(route_workspace) : nullptr;
   p.order = p.mask ? reinterpret_cast<int32_t*>(static_cast<uint8_t*>(route_workspace) +

@@ -253,6 +253,20 @@ def test_split_workspace_only_where_sinks_set_the_launch_end():
     assert size(1, 4096, 600000, 1, 128, 1.0, 128) == 0       # more than one routing segment
 
 
+@pytest.mark.parametrize("shape,split", [
+    ((1, 4096, 4096, 16, 128, 1.0, 128), True),    # the sink chain is 3.3 times a slot's average steps
+    ((1, 4096, 4096, 16, 128, 0.0, 128), False),   # 1.6 times
+    ((2, 4096, 4096, 16, 64, 1.0, 128), True),     # six workgroups per CU at head_dim 64: 2.4
+    ((1, 8192, 8192, 16, 128, 0.0, 128), True),    # at most 2,048 query blocks over at least 128 key blocks
+    ((1, 8192, 8192, 24, 128, 1.0, 128), False),   # 1.4 times
+    ((1, 4096, 1984, 16, 128, 1.0, 128), False),   # 31 key blocks: one part
+])
+def test_split_workspace_follows_the_sink_chain(shape, split):
+    if not os.path.exists(_native.LIB_PATH):
+        pytest.skip("libsol_attn_amd.so not built")
+    assert (_native.library().sol_split_workspace_size(*shape) > 0) == split
+
+
 def test_self_pooling_sizes_and_null_centroid_tiles():
     if not os.path.exists(_native.LIB_PATH):
         pytest.skip("libsol_attn_amd.so not built")

@@ -18,7 +18,7 @@ import math
 import pytest
 import torch
 
-from sol_attn_amd import _native, sol_attention
+from sol_attn_amd import _native, dense_attention, sol_attention
 from sol_testlib import HAS_GPU, assert_close, block_smooth, tensors
 from test_kernels import check_routing
 
@@ -76,3 +76,21 @@ def test_split_agrees_with_unsplit_and_forms_are_identical(case, monkeypatch):
     assert torch.equal(forms[1][1].exact_blocks, forms[2][1].exact_blocks)
     assert torch.equal(forms[1][1].exact_blocks, split_stats.exact_blocks)
 
+
+# More than 512 query-block pairs, but a sink chain of at least twice the steps a workgroup slot has on average
+# (sink_chain_ratio in csrc/capi.hip): two parts of 17 and 16 key blocks, odd lengths.
+@pytest.mark.parametrize("d,heads", [(64, 64), (128, 64)])
+def test_long_sink_chains_of_larger_launches_are_split(d, heads, monkeypatch):
+    tq, tk = 1000, 2100
+    assert _native.library().sol_split_workspace_size(1, tq, tk, heads, d, 1.0, 128) > 0
+    q, k, v = tensors(nq=tq, nk=tk, d=d, b=1, h=heads, device="cuda", seed=65)
+    print(f"long sink chains d {d}", flush=True)
+    kw = dict(beta=1.0, kv_sink_tokens=64, query_sink_tokens=128, return_stats=True)
+    split, split_stats = sol_attention(q, k, v, **kw)
+    monkeypatch.setattr(_native, "SPLIT_SINKS", False)
+    whole, whole_stats = sol_attention(q, k, v, **kw)
+    assert torch.equal(split_stats.exact_blocks, whole_stats.exact_blocks)
+    assert_close(split.cpu(), whole.cpu())
+    # Sink rows attend every key exactly; the others are not split.
+    assert_close(split[:, :128].cpu(), dense_attention(q, k, v)[:, :128].cpu())
+    assert torch.equal(split[:, 128:], whole[:, 128:])
