@@ -654,25 +654,27 @@ struct RangeCursor {
   __device__ __forceinline__ int operator()() { return j++; }
 };
 
-// FP32 mean of a query block's qlen staged rows (LDS, row stride KS) at
-// feature f, in torch's cascade order: four sequential 16-row sums folded in
-// order (kernels.py:56).
+// FP32 mean of a query block's qlen staged rows (LDS, row stride KS, zero past
+// them) at feature f, in torch's cascade order: four sequential 16-row sums
+// (query_chunk) folded in order (kernels.py:56).  The zero rows leave a sum
+// from +0 as it is.
+template <int D>
+__device__ __forceinline__ float query_chunk(const uint16_t* rows, int c, int f) {
+  // The chunk's 16 values are read first, so the reads overlap.
+  float x[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] = bf16_bits_to_f32(rows[(16 * c + i) * Shape<D>::KS + f]);
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sum = __fadd_rn(sum, x[i]);
+  return sum;
+}
+
 template <int D>
 __device__ __forceinline__ float query_mean(const uint16_t* rows, int qlen, int f) {
   float tot = 0.f;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    // The chunk's 16 values are read first (every staged row exists), so the
-    // reads overlap; the sum then takes the block's rows in order.
-    float x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = bf16_bits_to_f32(rows[(16 * c + i) * Shape<D>::KS + f]);
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (16 * c + i < qlen) sum = __fadd_rn(sum, x[i]);
-    tot = __fadd_rn(tot, sum);
-  }
+  for (int c = 0; c < 4; ++c) tot = __fadd_rn(tot, query_chunk<D>(rows, c, f));
   return __fdiv_rn(tot, float(qlen));
 }
 
@@ -1300,7 +1302,8 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   constexpr int SLOTS = POOL ? 2 : 1;
   __shared__ __align__(256) uint16_t ring[SLOTS * KS * S::TILE];
   __shared__ float s_md[KS][2][2][kWave];  // the groups' m and den
-  __shared__ float s_qm[D];
+  __shared__ float s_qm[D];        // query mean (full covariance)
+  __shared__ float s_chunk[4][D];  // its 16-row sums
   __shared__ __align__(16) uint16_t s_qb[4 * kRouteRow<D>];  // its BF16 terms (route_word)
   __shared__ float s_red[4];
   __shared__ float s_mom[2][POOL ? D : 1];  // pooled key mean, variance
@@ -1376,13 +1379,11 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) sm[e] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if (16 * r4 + i < len) {
+    for (int i = 0; i < 16; ++i) {  // rows past len were loaded as zero
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t w = x[i][e >> 1];
-          sm[e] = __fadd_rn(sm[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
-        }
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t w = x[i][e >> 1];
+        sm[e] = __fadd_rn(sm[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
       }
     }
     float t1[8], t2[8], t3[8];
@@ -1393,16 +1394,18 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
       t3[e] = __shfl(sm[e], lane + 3 * DC);
     }
     if (r4 == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sm[e] = __fadd_rn(__fadd_rn(__fadd_rn(sm[e], t1[e]), t2[e]), t3[e]);
+      if (__builtin_amdgcn_ballot_w64(len != kBlock) == 0) {  // the same: a power of two
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sm[e] = __fmul_rn(sm[e], 1.f / kBlock);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sm[e] = len > 0 ? __fdiv_rn(sm[e], float(len)) : 0.f;
+      }
       u32x4 o;
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        float m0 = 0.f, m1 = 0.f;
-        if (len > 0) {
-          m0 = __fdiv_rn(__fadd_rn(__fadd_rn(__fadd_rn(sm[e], t1[e]), t2[e]), t3[e]), float(len));
-          m1 = __fdiv_rn(__fadd_rn(__fadd_rn(__fadd_rn(sm[e + 1], t1[e + 1]), t2[e + 1]), t3[e + 1]), float(len));
-        }
-        o[e >> 1] = pack_bf16x2(m0, m1);
-      }
+      for (int e = 0; e < 8; e += 2) o[e >> 1] = pack_bf16x2(sm[e], sm[e + 1]);
       const int jb = u % kPoolChunk;
       *reinterpret_cast<u32x4*>(ctile + (u >= kPoolChunk ? TL::kElems + TL::v_offset(jb, dc) : TL::k_offset(jb, dc))) = o;
     }
@@ -1447,33 +1450,50 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
     for (int ks = 0; ks < S::KT; ++ks)
       qf[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(qrow + ks * 16 + 8 * hh));
   }
-  if constexpr (POOL) {
-    // Diagonal moments of the BF16 centroids: sequential sums over the
-    // blocks, E[x^2] - mu^2 clamped at 0, each step rounded on its own.
-    if (tid < D) {
-      float s1 = 0.f, s2 = 0.f;
-      for (int jb = 0; jb < nkb; ++jb) {
-        const float x = bf16_bits_to_f32(ctile[TL::k_offset(jb, tid / 8) + tid % 8]);
-        s1 = __fadd_rn(s1, x);
-        s2 = __fadd_rn(s2, __fmul_rn(x, x));
-      }
-      const float n = float(nkb);
-      const float m = __fdiv_rn(s1, n);
-      const float v = __fsub_rn(__fdiv_rn(s2, n), __fmul_rn(m, m));
-      s_mom[0][tid] = m;
-      s_mom[1][tid] = v > 0.f ? v : 0.f;
-    }
-  }
 
   // 2. In-kernel routing: query mean and cutoff (group 0's threads sum; every
-  // thread forms the cutoff from the published sums).
+  // thread forms the cutoff from the published sums).  The mean's four chunk
+  // sums per feature are spread over the workgroup, query_mean's fold follows
+  // the barrier: as one thread's chain they were 2,500 of a workgroup's 33,000
+  // cycles (1,024 tokens).
   float cut = 0.f;
   if (p.force == 0 && !routed) {
-    if (tid < D) s_qm[tid] = query_mean<D>(stage, qlen, tid);
+#pragma unroll
+    for (int x = tid; x < 4 * D; x += NT) s_chunk[x / D][x % D] = query_chunk<D>(stage, x / D, x % D);
+    if constexpr (POOL) {
+      // Diagonal moments of the BF16 centroids: sequential sums over the
+      // blocks, E[x^2] - mu^2 clamped at 0, each step rounded on its own (the
+      // rows past the last block are zero and leave both sums as they are).
+      // By the last waves, which hold no chunk sums.
+      if (tid >= NT - D) {
+        const int f = tid - (NT - D);
+        float x[kPoolChunk], s1 = 0.f, s2 = 0.f;
+#pragma unroll
+        for (int jb = 0; jb < kPoolChunk; ++jb) x[jb] = bf16_bits_to_f32(ctile[TL::k_offset(jb, f / 8) + f % 8]);
+#pragma unroll
+        for (int jb = 0; jb < kPoolChunk; ++jb) {
+          s1 = __fadd_rn(s1, x[jb]);
+          s2 = __fadd_rn(s2, __fmul_rn(x[jb], x[jb]));
+        }
+        const float n = float(nkb);
+        const float m = __fdiv_rn(s1, n);
+        const float v = __fsub_rn(__fdiv_rn(s2, n), __fmul_rn(m, m));
+        s_mom[0][f] = m;
+        s_mom[1][f] = v > 0.f ? v : 0.f;
+      }
+    }
     __syncthreads();  // also: every read of the Q staging rows is done
-    float a = 0.f, g = 0.f;
+    float a = 0.f, g = 0.f, qm = 0.f;
     if (tid < D) {
-      const float qm = s_qm[tid];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) qm = __fadd_rn(qm, s_chunk[c][tid]);
+      qm = __fdiv_rn(qm, float(qlen));
+    }
+    if (p.cov) {  // every feature's mean
+      if (tid < D) s_qm[tid] = qm;
+      __syncthreads();
+    }
+    if (tid < D) {
       split_query_mean<D>(s_qb, tid, qm);
       float mu;
       if (POOL) {

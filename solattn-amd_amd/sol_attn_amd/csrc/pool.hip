@@ -14,7 +14,9 @@
 // Both are streamed into LDS by the attention kernels with DMA.
 // Sums follow torch's CPU outer-reduction order (16-row sequential chunks,
 // folded in order), so the FP32 means and the BF16-rounded centroids equal the
-// reference oracle's `x[:, i:i+64].float().mean(1)` bit for bit.
+// reference oracle's `x[:, i:i+64].float().mean(1)` bit for bit.  Rows past a
+// partial block's end are loaded as zero (load_rows16), which leaves a sum
+// from +0 as it is.
 #include "sol_device.h"
 #include "sol_internal.h"
 
@@ -112,12 +114,10 @@ void pool_kv_kernel(PoolParams p) {
       // Sequential accumulation inside the 16-row chunk (torch order).
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        if (16 * r4 + i < len) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t w = x[i][e >> 1];
-            s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
-          }
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t w = x[i][e >> 1];
+          s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
         }
       }
     }
@@ -234,12 +234,10 @@ __global__ __launch_bounds__(256) void pool_blocks_kernel(PoolParams p) {
     load_rows16<16, true>(src, b, kBlock * j + 16 * r4, kBlock * j + len - 1, h, 8 * dc, x);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      if (16 * r4 + i < len) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t w = x[i][e >> 1];
-          s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
-        }
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t w = x[i][e >> 1];
+        s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
       }
     }
   }
@@ -323,12 +321,10 @@ __global__ __launch_bounds__(1024) void pool_kv4_kernel(PoolParams p) {
       for (int e = 0; e < 8; ++e) s[e] = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        if (16 * q + i < len) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t w = x[i][e >> 1];
-            s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
-          }
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t w = x[i][e >> 1];
+          s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
         }
       }
 #pragma unroll
