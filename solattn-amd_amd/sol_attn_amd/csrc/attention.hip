@@ -309,19 +309,21 @@ __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, in
 
 // Centroid tile ct: the block centroids 64 ct + r whose bit r is set in
 // `approx` contribute logit q . Kc_j + ln(len_j) and value Vc_j: their scores
-// start at log2(len_j) / c (c = scale * log2(e)), the others at -inf.
+// start at log2(len_j) / c (c = scale * log2(e)), the others at -inf.  With
+// `exact` the tile is a full exact block instead, every score from 0: waves
+// that attend one in the same step as others their centroid tile.
 template <int D, bool FULL = false, typename Step>
 __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf, int ct, uint64_t approx,
                                               int tk, const bf16x8 (&qf)[Shape<D>::KT], int col, int hh,
-                                              float c, const Step& step) {
+                                              float c, const Step& step, bool exact = false) {
   const float inv_c = 1.f / c;
   // Every block is whole but the sequence's last one: whole blocks share one
   // offset, log2(64) / c.  The approximated blocks are wave-uniform, so each
   // element's choice is a lane mask formed on the scalar unit: rows r (lanes
   // 0 .. 31) and r + 4 (lanes 32 .. 63).
-  const uint64_t bits = uniform64(approx);
-  const float whole = __builtin_amdgcn_logf(float(kBlock)) * inv_c;
-  const int last = (tk - 1) / kBlock - kBlock * ct;           // the last block's row, if in this tile
+  const uint64_t bits = uniform64(exact ? ~0ull : approx);
+  const float whole = exact ? 0.f : __builtin_amdgcn_logf(float(kBlock)) * inv_c;
+  const int last = exact ? kBlock : (tk - 1) / kBlock - kBlock * ct;  // the last block's row, if in this tile
   const int len = tk - kBlock * (kBlock * ct + last);         // and its keys
   const auto lengths = [&](int t) {
     f32x16 bias;
@@ -1267,7 +1269,9 @@ struct SplitCursor {
 // stepping in the same workgroup barriers, so a chain of n tiles takes ceil(n
 // / KS) steps.  Centroid tiles come first, group grp routing and attending
 // tiles grp, grp + KS, ...; the first of them travel while Q is staged and the
-// cutoff formed.  At the end every group publishes its online-softmax state
+// cutoff formed.  With fewer than KS centroid tiles, the groups without one
+// take whole blocks of the local band, which are exact whatever the routing
+// says, in that step (with them idle 4,096 x 4 heads took 30.8 us per call, now 28.8).  At the end every group publishes its online-softmax state
 // in LDS and merges and stores a share of the output features (m = max m_g,
 // acc and den weighted by 2^(m_g - m), groups in order).  Decisions, counts and diagnostics are the
 // one-block kernel's; the output agrees with it to rounding (other partial
@@ -1300,7 +1304,10 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   // Group g's slots at g SLOTS TILE; the Q staging aliases the last group's.
   // POOL: the centroid tile is formed in group 0's second slot.
   constexpr int SLOTS = POOL ? 2 : 1;
-  __shared__ __align__(256) uint16_t ring[SLOTS * KS * S::TILE];
+  // Four one-slot groups leave room for the Q staging beside their slots (one
+  // workgroup per CU), so that every group's first tile travels meanwhile.
+  constexpr bool kApart = !POOL && KS == 4;
+  __shared__ __align__(256) uint16_t ring[SLOTS * KS * S::TILE + (kApart ? kBlock * S::KS : 0)];
   __shared__ float s_md[KS][2][2][kWave];  // the groups' m and den
   __shared__ float s_qm[D];        // query mean (full covariance)
   __shared__ float s_chunk[4][D];  // its 16-row sums
@@ -1308,6 +1315,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   __shared__ float s_red[4];
   __shared__ float s_mom[2][POOL ? D : 1];  // pooled key mean, variance
   __shared__ uint32_t s_mask[kMaskWords];
+  __shared__ uint32_t s_exact[POOL ? 1 : kMaskWords];  // less the blocks attended beside the centroid tiles
 
   const int nbh = p.B * p.H;
   const int bh = blockIdx.x % nbh, qb = blockIdx.x / nbh;  // every head's first blocks dispatch first
@@ -1324,7 +1332,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   const float scale_log2 = p.scale_log2;
   const bool routed = p.mask != nullptr;
   uint16_t* const ctile = ring + S::TILE;  // POOL: the pooled centroid tile
-  uint16_t* const stage = ring + SLOTS * (KS - 1) * S::TILE;
+  uint16_t* const stage = ring + (kApart ? KS * S::TILE : SLOTS * (KS - 1) * S::TILE);
   uint16_t* const slot = ring + grp * SLOTS * S::TILE;
   const uint32_t slot_lds = lds_address(slot);
   const int wg = wave & 1;  // the wave inside its group
@@ -1332,7 +1340,24 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   const uint16_t* ctiles = p.ctiles + head * p.NCT * S::TILE;
   const auto crefill = bf16_refills<D, 128>([=](int ct) { return ctiles + int64_t(ct) * S::TILE; }, wg, lane);
   constexpr int kHalfRounds = TileRefill<D, 128>::kRounds / 2;
-  if (!POOL && grp < KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
+  const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
+  const auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
+  // Blocks [early0, early1): the first whole blocks of the local band, one for
+  // each group without a centroid tile.  Launches whose keys could be pooled
+  // here as well deal their blocks as the POOL form does (the same bits).
+  const bool poolable = D == 64 && KS == 4 && p.NKB <= kPoolChunk;
+  const int early0 = max(qb - max(p.local_blocks, 0), 0);
+  const int early1 = poolable || p.local_blocks < 0
+                         ? early0
+                         : max(early0, min(min(qb + p.local_blocks + 1, tk / kBlock), early0 + max(KS - nct, 0)));
+  const bool early = grp >= nct && early0 + grp - nct < early1;
+  auto first_tile = [&] {
+    if (early)
+      make(2 * (early0 + grp - nct), slot_lds).all();
+    else
+      crefill(min(grp, nct - 1), slot_lds).all();
+  };
+  if (!POOL && (kApart || grp < KS - 1)) first_tile();
 
   // This thread's feature of the key moments: its loads travel with Q's.
   KeyMoments<D> km;
@@ -1531,13 +1556,16 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
   state_init(st);
   const int nwords = (nkb + 31) / 32;
   if (routed) {
-    for (int w = tid; w < nwords; w += NT) s_mask[w] = p.mask[(head * p.NQB + qb) * p.NW + w];
+    for (int w = tid; w < nwords; w += NT) {
+      const uint32_t word = p.mask[(head * p.NQB + qb) * p.NW + w];
+      s_mask[w] = word;
+      if (!POOL) s_exact[w] = word & ~uint32_t(bit_range64(early0 - 32 * w, early1 - 32 * w));
+    }
     __syncthreads();
   }
 
-  const auto kv = kv_refills<D, 128, KT, true>(p, b, h, wg, lane);
-  const auto make = [=](int tag, uint32_t lds) { return kv(tag >> 1, lds); };
-  SplitCursor<KS> cursor{UnionCursor<1>{s_mask, s_mask, kMaskWords, 0, nkb, 0}, grp};
+  const uint32_t* const exact = POOL ? s_mask : s_exact;
+  SplitCursor<KS> cursor{UnionCursor<1>{exact, exact, kMaskWords, 0, nkb, 0}, grp};
   if constexpr (POOL) {
     // 3. Group 0 routes from the centroid tile (and the V centroids are
     // finished); its contributions run in the exact stream's prologue, over
@@ -1573,11 +1601,11 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
     // 3. Centroid tiles grp, grp + KS, ...: routed by their group, then attended
     // while the group's next tile -- another centroid tile or, after the last
     // round, its first exact tile -- travels.  A group past the last centroid
-    // tile goes through that one again with no block of it approximated (it
-    // adds nothing), so that all groups meet at the same barriers.  (Launches
-    // at beta = -inf take sol_attention_kernel.)
+    // tile attends its early block or goes through that tile again with no
+    // block of it approximated (it adds nothing), so that all groups meet at
+    // the same barriers.  (Launches at beta = -inf take sol_attention_kernel.)
     u32x4 k[2][S::KT];
-    if (grp == KS - 1) crefill(min(grp, nct - 1), slot_lds).all();
+    if (!kApart && grp == KS - 1) first_tile();
     slot_prime<D, 2 * kHalfRounds>(slot, k, col, hh);
     auto centroids = [&](auto&& fn) {
       return qh ? fn([&](int ks) { return k[1][ks]; }) : fn([&](int ks) { return k[0][ks]; });
@@ -1588,7 +1616,11 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
           const uint32_t word = centroids([&](const auto& kfrag) {
             return route_word<D>(p, kfrag, s_qb, cut, kBlock * ct + 32 * qh, 0, nkb, b, qb, lane, dbg_row);
           });
-          if (lane == 0) s_mask[2 * ct + qh] = word;
+          if (lane == 0) {
+            const int w = 2 * ct + qh;
+            s_mask[w] = word;
+            s_exact[w] = word & ~uint32_t(bit_range64(early0 - 32 * w, early1 - 32 * w));
+          }
         }
         lds_barrier();  // publishes the mask words
       }
@@ -1602,8 +1634,8 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
     const int steps = (cursor.all.count() + KS - 1) / KS;
     const int id = cursor();
     centroid_tile<D, true>(st, slot, min(ct, nct - 1), approx, tk, qf, col, hh, scale_log2,
-                           slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot));
-    // 4. Exact pass: group grp's share of the selected blocks, ascending.
+                           slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot), early);
+    // 4. Exact pass: group grp's share of the other selected blocks, ascending.
     const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
     slot_stream(
         slot_lds, id, steps, cursor, make, [&] { return __builtin_amdgcn_ballot_w64(st.m == kNegInf) != 0; },

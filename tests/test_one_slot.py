@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from sol_attn_amd import IndexedPlan, _native, dense_attention, sol_attention_indexed
-from sol_testlib import HAS_GPU, block_smooth, tensors
+from sol_testlib import HAS_GPU, assert_close, block_smooth, tensors
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not HAS_GPU, reason="AMD ROCm GPU required")]
 
@@ -54,6 +54,25 @@ def test_forms_agree(d, tq, tk, beta, monkeypatch):
         two, c2 = _launch(q, k, v, 2, monkeypatch, beta, **kw)
         assert torch.equal(c1, c2)
         assert torch.equal(one, two)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("tq,tk,heads", [
+    (130, 130, 2), (1100, 1090, 3), (700, 2304, 1),  # one centroid tile: three early blocks, partial last blocks
+    (64, 4097, 2), (400, 8192, 3), (300, 8200, 1),   # two and three
+    (200, 12288, 2), (200, 12289, 2),                # three and four (none early)
+    (4160, 1100, 6),                                 # two groups
+])
+def test_early_local_blocks_of_small_launches(d, tq, tk, heads, monkeypatch):
+    # Local blocks attended beside the centroid tiles: the same blocks, so equal counts, and outputs that differ
+    # from the one-block kernel's in the order of the sums only.
+    print(f"early blocks: D{d} Tq{tq} Tk{tk} H{heads}", flush=True)
+    q, k, v = (block_smooth(1, t, heads, d, seed=s, device="cuda") for t, s in ((tq, 1), (tk, 2), (tk, 3)))
+    for local, beta in ((0, 1.0), (1, 1.0), (2, math.inf), (7, 0.0), (1 << 30, 1.0)):
+        small, c0 = _launch(q, k, v, 0, monkeypatch, beta, local=local)
+        one, c1 = _launch(q, k, v, 1, monkeypatch, beta, local=local)
+        assert torch.equal(c0, c1)
+        assert_close(small.cpu(), one.cpu())
 
 
 def _windows(kind, n):
