@@ -133,6 +133,16 @@ def _rows(x):
     return x if _aligned(x) else x.clone(memory_format=torch.contiguous_format)
 
 
+def _bthd_rows(x):
+    """``(x, data pointer, stride array)`` of a BTHD operand, copied once when
+    misaligned (:func:`_rows` and :func:`_strides` in one look)."""
+    ptr, s = x.data_ptr(), x.stride()
+    if (ptr & 15) or (s[0] | s[1] | s[2]) & 7:
+        x = x.clone(memory_format=torch.contiguous_format)
+        ptr, s = x.data_ptr(), x.stride()
+    return x, ptr, _stride_array(s[0], s[1], s[2])
+
+
 def _tiles(b, h, nkb, d, device):
     return torch.empty((b, h, nkb, 2, BLOCK * d), device=device, dtype=torch.bfloat16)
 
@@ -506,18 +516,20 @@ def _all_in_size(b, nq, nk, h, d, beta, q_sink, k_stride, v_stride):
 
 def _all_in(q, k, v, scale, beta, local, kv_sink, q_sink, stats):
     """``(out, counts)`` of one sol_attention_all_in call (BTHD, the caller's stream)."""
-    q, k, v = _rows(q), _rows(k), _rows(v)
+    q, q_ptr, q_strides = _bthd_rows(q)
+    k, k_ptr, k_strides = _bthd_rows(k)
+    v, v_ptr, v_strides = _bthd_rows(v)
     b, nq, h, d = q.shape
     nk = k.shape[1]
     dev = q.device
-    size = _all_in_size(b, nq, nk, h, d, beta, q_sink, k.stride(1), v.stride(1))
+    size = _all_in_size(b, nq, nk, h, d, beta, q_sink, k_strides[1], v_strides[1])
     if size < 0:
         raise RuntimeError("sol_attention_workspace_size rejected the sizes")
     ws = torch.empty(size, device=dev, dtype=torch.uint8) if size else None
     out = torch.empty((b, nq, h, d), device=dev, dtype=torch.bfloat16)
     counts = torch.empty((b, -(-nq // BLOCK), h), device=dev, dtype=torch.int32) if stats else None
     _check(library().sol_attention_all_in(
-        q.data_ptr(), _strides(q), k.data_ptr(), _strides(k), v.data_ptr(), _strides(v), b, nq, nk, h, d,
+        q_ptr, q_strides, k_ptr, k_strides, v_ptr, v_strides, b, nq, nk, h, d,
         scale, beta, local, kv_sink, q_sink, _ptr(ws), size, out.data_ptr(), _ptr(counts), _stream(dev)))
     return out, counts
 

@@ -5,10 +5,13 @@ the reference; the device work goes through the HIP C-ABI library
 (``_native``).  There is no fallback: inputs off an AMD ROCm GPU are rejected.
 """
 
+import contextlib
 from dataclasses import dataclass
 import math
 
 import torch
+
+from . import _native
 
 
 @dataclass(frozen=True)
@@ -33,14 +36,14 @@ class SolStats:
 
 def _validate(q, k, v, scale):
     """Input contract of ``attention.py:19-39``; returns the effective scale."""
-    if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
+    qs, ks, device = q.shape, k.shape, q.device
+    if len(qs) != 4 or len(ks) != 4 or v.ndim != 4:
         raise ValueError("Q/K/V must have BTHD rank-4 layout")
-    if (k.shape != v.shape or q.shape[0] != k.shape[0]
-            or q.shape[2:] != k.shape[2:] or min(q.shape + k.shape) <= 0):
+    if ks != v.shape or qs[0] != ks[0] or qs[2:] != ks[2:] or min(qs + ks) <= 0:
         raise ValueError("Q/K/V batch, head and dimension shapes must agree and be nonempty")
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
         raise ValueError("Only BF16 Q/K/V are implemented")
-    if q.shape[-1] not in (64, 128):
+    if qs[3] not in (64, 128):
         raise ValueError("Only head dimensions 64 and 128 are implemented")
     if q.requires_grad or k.requires_grad or v.requires_grad:
         raise ValueError("Inference only: Q/K/V must not require gradients")
@@ -48,13 +51,23 @@ def _validate(q, k, v, scale):
         strides = t.stride()
         if strides[-1] != 1 or min(strides) <= 0:
             raise ValueError("Q/K/V need positive strides and contiguous head dimension")
-    scale = q.shape[-1] ** -0.5 if scale is None else float(scale)
+    scale = qs[3] ** -0.5 if scale is None else float(scale)
     if not math.isfinite(scale) or scale <= 0:
         raise ValueError("scale must be finite and positive")
-    if (torch.version.hip is None or q.device.type != "cuda"
-            or k.device != q.device or v.device != q.device):
+    if torch.version.hip is None or device.type != "cuda" or k.device != device or v.device != device:
         raise ValueError("The HIP backend requires Q/K/V on the same AMD ROCm GPU")
     return scale
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(device):
+    """The context a launch on ``device`` runs in: nothing to switch when it is
+    the current device (inputs never require gradients, so there is no graph to
+    keep them out of either; the two context managers were 2 of the 15 us that
+    a short call spends on the host)."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 # Key tokens one pooling call takes (SOL_MAX_KEY_TOKENS in
@@ -81,9 +94,8 @@ def dense_attention(q, k, v, *, scale=None):
     HIP kernel.
     """
     scale = _validate(q, k, v, scale)
-    from ._native import launch_dense
-    with torch.no_grad(), torch.cuda.device(q.device):
-        return launch_dense(q, k, v, scale)
+    with _on(q.device):
+        return _native.launch_dense(q, k, v, scale)
 
 
 THRESHOLD_ESTIMATORS = ("diagonal_covariance", "full_covariance")
@@ -141,11 +153,10 @@ def sol_attention(q, k, v, *, beta=1.0, scale=None, local_blocks=1,
     if kv_sink_tokens > k.shape[1] or query_sink_tokens > q.shape[1]:
         raise ValueError("Sink token counts must not exceed their sequence lengths")
     _key_length(k.shape[1])
-    from ._native import launch_sol
-    with torch.no_grad(), torch.cuda.device(q.device):
-        out, counts = launch_sol(q, k, v, scale, beta, local_blocks,
-                                 kv_sink_tokens, query_sink_tokens, return_stats,
-                                 threshold_estimator=threshold_estimator, qk_precision=qk_precision)
+    with _on(q.device):
+        out, counts = _native.launch_sol(q, k, v, scale, beta, local_blocks,
+                                         kv_sink_tokens, query_sink_tokens, return_stats,
+                                         threshold_estimator=threshold_estimator, qk_precision=qk_precision)
     if return_stats:
         return out, SolStats(counts, (k.shape[1] + 63) // 64)
     return out
