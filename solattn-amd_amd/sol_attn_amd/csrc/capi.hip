@@ -755,8 +755,14 @@ int all_in(const char* who, const void* q, const int64_t* q_strides, const void*
                                     kv_sink_tokens, query_sink_tokens, out);
   if (arc != SOL_OK) return arc;
   const bool rows = rows_mode_possible(nullptr, nullptr, key_tokens, k_strides, v_strides);
-  const AllInLayout l = all_in_layout(batch, query_tokens, key_tokens, heads, head_dim, beta, query_sink_tokens,
-                                      rows);
+  AllInLayout l = all_in_layout(batch, query_tokens, key_tokens, heads, head_dim, beta, query_sink_tokens, rows);
+  // Larger launches split their sink tiles for speed only: unsplit where the
+  // library's array has no room for the partial states.
+  if (scratch && l.total > ws_bytes && l.split_bytes && std::isfinite(beta) &&
+      batch * heads * ((cdiv(query_tokens, SOL_BLOCK) + 1) / 2) >= sol::kSmallLaunchGroups) {
+    l.split_bytes = 0;
+    l.total = l.split;
+  }
   // One attention launch that pools the keys itself: no workspace at all.
   if (l.self_pooled)
     return sol_attention_fwd(q, q_strides, nullptr, 0, batch, query_tokens, key_tokens, nullptr, heads, head_dim,

@@ -13,8 +13,8 @@ import sys
 import pytest
 import torch
 
-from sol_attn_amd import _native
-from sol_testlib import HAS_GPU, block_smooth
+from sol_attn_amd import _native, sol_attention
+from sol_testlib import HAS_GPU, assert_close, block_smooth
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not HAS_GPU, reason="AMD ROCm GPU required")]
 
@@ -66,10 +66,28 @@ def test_noalloc_matches_the_allocating_path_on_consecutive_calls(monkeypatch):
         assert torch.equal(counts, ref_counts), f"case {i}"
 
 
+def test_noalloc_leaves_sink_tiles_whole_where_their_split_does_not_fit():
+    # Pooled keys of 72 MiB and partial states of 60 MiB: together more than the 128 MiB array, so the split that
+    # the caller's workspace would hold is left out; equal decisions, outputs that differ in the order of the sums.
+    tq, tk, heads, d, beta = 512, 65536, 256, 64, 2.0
+    size = _native.library().sol_attention_workspace_size(1, tq, tk, heads, d, beta, 128, heads * d, heads * d)
+    assert size > 128 << 20 > size - _native.library().sol_split_workspace_size(1, tq, tk, heads, d, beta, 128)
+    print("noalloc without room for the split", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(71)
+    q, k, v = (torch.randn((1, t, heads, d), generator=gen, device="cuda", dtype=torch.bfloat16) for t in (tq, tk, tk))
+    ref, stats = sol_attention(q, k, v, beta=beta, kv_sink_tokens=64, query_sink_tokens=128, return_stats=True)
+    out = torch.full_like(q, 7.0)
+    counts = torch.full_like(stats.exact_blocks, -5)
+    _noalloc(q, k, v, beta, 1, 64, 128, out, counts)
+    torch.cuda.synchronize()
+    assert torch.equal(counts, stats.exact_blocks)
+    assert_close(out.cpu(), ref.cpu())
+
+
 _FIRST_CALL = r"""
 import ctypes
 import torch
-from sol_attn_amd import _native
+from sol_attn_amd import _native, sol_attention
 from sol_testlib import block_smooth
 b, tq, tk, h, d = 1, 4096, 4096, 4, 128
 q = block_smooth(b, tq, h, d, seed=41, device="cuda")
