@@ -151,9 +151,12 @@ int sol_key_covariance(const void* ctiles, const float* key_mean, const int32_t*
 /* Bytes of the split_workspace sol_attention_fwd takes for a problem (0:
  * the problem is not split, pass NULL).  Launches with at least two
  * query-sink blocks and at most a quarter of the query blocks, at most
- * 524,288 keys, and either fewer than 512 query-block pairs over all (entry,
- * head) pairs (finite beta) or beta = +INFINITY and at most 8,192 query
- * blocks, split the key blocks of sink blocks [0, 2 floor(sink blocks / 2))
+ * 524,288 keys split where the sink blocks' chains would set the launch's
+ * end: at fewer than 512 query-block pairs over all (entry, head) pairs; at
+ * beta = +INFINITY up to 8,192 query blocks; at finite beta and one query
+ * block per workgroup up to 2,048 query blocks over at least 128 key blocks,
+ * or when the chain is at least twice the steps a workgroup slot has on
+ * average.  They split the key blocks of sink blocks [0, 2 floor(sink blocks / 2))
  * over up to 8 workgroups each (parts of at least 16 blocks); a merge kernel
  * combines their partial softmax states.  Split launches pair adjacent query
  * blocks (pair_strides is ignored).
@@ -225,13 +228,14 @@ int64_t sol_route_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
  * centroid terms and P V stay BF16; sol_quantize_keys's rows_mode must be
  * nonzero exactly when tiles is NULL here.
  * workgroup_form: 0 picks the schedule by launch size: launches at finite
- * or +INFINITY beta of at most 256 query blocks (over all entries and
- * heads) whose keys span at most
- * 64 (head_dim 64) or 32 (head_dim 128) blocks run one query block per
- * workgroup with its key tiles split over 4 (2) groups of two waves, merged
- * in LDS (outputs agree with the other forms to rounding; decisions and
- * counts are the same); otherwise one query block per workgroup below 512
- * query-block pairs, else 2.  1 or 2 force one or two query blocks per
+ * or +INFINITY beta of at most 512 query blocks (over all entries and
+ * heads) run one query block per workgroup with its key tiles split over 4
+ * (at most 256 query blocks) or 2 groups of two waves, merged in LDS (outputs
+ * agree with the other forms to rounding; decisions and counts are the
+ * same), unless two or more query-sink blocks meet long keys
+ * (small_key_split in csrc/sol_internal.h); otherwise one query block per
+ * workgroup while a head's K and V are at most 16 MB or the launch has fewer
+ * than 512 query-block pairs, else 2.  1 or 2 force one or two query blocks per
  * workgroup without the key split (bit-identical results).  No counterpart
  * in the reference (one Triton program per query block).
  * ctiles / key_mean / key_var: NULL at beta = -INFINITY (unused), or where
