@@ -276,6 +276,9 @@ __global__ __launch_bounds__(256) void pool_blocks_kernel(PoolParams p) {
 // 84,672-token K 5.5% faster.  The lane sums its block's 64 rows in torch's
 // order itself -- four sequential 16-row sums folded in order -- so the
 // centroids, chunk sums and moments are the one-head kernel's bit for bit.
+// The row test changes no sum but keeps each row's additions behind its own
+// scalar branch, in the order its loads arrive: without it 84,672 tokens x 24
+// heads take 200 us instead of 181.
 template <int D>
 __global__ __launch_bounds__(1024) void pool_kv4_kernel(PoolParams p) {
   constexpr int DC = D / 8;
@@ -321,10 +324,12 @@ __global__ __launch_bounds__(1024) void pool_kv4_kernel(PoolParams p) {
       for (int e = 0; e < 8; ++e) s[e] = 0.f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
+        if (16 * q + i < len) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t w = x[i][e >> 1];
-          s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t w = x[i][e >> 1];
+            s[e] = __fadd_rn(s[e], bf16_bits_to_f32((e & 1) ? (w >> 16) : (w & 0xFFFFu)));
+          }
         }
       }
 #pragma unroll
