@@ -131,10 +131,10 @@ __device__ __forceinline__ void landed_barrier() {
 //   [every wave holds its K fragments]  half 0's scores; the next K's DMA
 //   [V has landed]                      half 1's scores; V^T reads
 //   [every wave holds its V fragments]  half 0's P V; the next V's DMA
-//   [the next K has landed]             half 1's P V; its K reads  FULL: the max-pass softmax from the start (HalfSoftmax, the
-// same results), for a SlotStep that may have to look at the raw scores again:
-// a state without any key yet.  Scores
-// start from bias(t) when BIASED (-inf drops a key, log2(len) / c adds a
+//   [the next K has landed]             half 1's P V; its K reads
+// FULL: the max-pass softmax from the start (HalfSoftmax, the same results),
+// for a SlotStep that may have to look at the raw scores again: a state
+// without any key yet.  Scores start from bias(t) when BIASED (-inf drops a key, log2(len) / c adds a
 // centroid's ln(len) logit term), else from 0.  LATE: the bias (0 or -inf
 // only) is added once a half's products are done instead, which keeps it out
 // of the registers live across the score chain; the same values (x + 0 is x
@@ -832,8 +832,6 @@ __device__ __forceinline__ auto lds_centroids(const uint16_t* buf, int t, int la
 
 }  // namespace
 
-
-
 // __launch_bounds__ second argument: minimum waves per SIMD.  Two waves per
 // SIMD leave each wave 256 VGPRs: the exact path keeps the 64-register
 // accumulator, 32 registers of Q fragments and 64 of K or V fragments live.
@@ -1271,15 +1269,17 @@ struct SplitCursor {
 // tiles grp, grp + KS, ...; the first of them travel while Q is staged and the
 // cutoff formed.  With fewer than KS centroid tiles, the groups without one
 // take whole blocks of the local band, which are exact whatever the routing
-// says, in that step (with them idle 4,096 x 4 heads took 30.8 us per call, now 28.8).  At the end every group publishes its online-softmax state
-// in LDS and merges and stores a share of the output features (m = max m_g,
-// acc and den weighted by 2^(m_g - m), groups in order).  Decisions, counts and diagnostics are the
-// one-block kernel's; the output agrees with it to rounding (other partial
-// sums).  POOL (plain K / V rows, at most one pooling chunk of key blocks,
-// no centroid tiles given): every workgroup forms its head's block centroids
-// and diagonal moments in LDS in the pooling kernel's order and arithmetic
-// (bit-identical values), so the whole call is this one launch.  Finite and
-// +inf beta only (beta = -inf launches take sol_attention_kernel).
+// says, in that step (with them idle 4,096 x 4 heads took 30.8 us per call,
+// now 28.8).  At the end every group publishes its online-softmax state in LDS
+// and merges and stores a share of the output features (m = max m_g, acc and
+// den weighted by 2^(m_g - m), groups in order).  Decisions, counts and
+// diagnostics are the one-block kernel's; the output agrees with it to
+// rounding (other partial sums).  POOL (plain K / V rows, at most one pooling
+// chunk of key blocks, no centroid tiles given): every workgroup forms its
+// head's block centroids and diagonal moments in LDS in the pooling kernel's
+// order and arithmetic (bit-identical values), so the whole call is this one
+// launch.  Finite and +inf beta only (beta = -inf launches take
+// sol_attention_kernel).
 // The slots take 32 KB per group at head_dim 128 (16 at 64): four groups per
 // CU, two waves per SIMD, in 256 vector registers.  (Two-slot rings left room
 // for two groups at head_dim 128, one wave per SIMD, whose accumulators lay in
