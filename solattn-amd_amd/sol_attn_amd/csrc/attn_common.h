@@ -232,6 +232,19 @@ __device__ __forceinline__ void dma16(uint64_t sbase, uint32_t lane_bytes, uint3
       : "memory", "m0");
 }
 
+// The byte offset of a DMA round, through an empty asm: the address is formed
+// right before the DMA by a scalar add, from an immediate or a scalar product,
+// and not kept live in registers of its own across the whole stream.  The add
+// is also what makes the address safe to use: the base comes from
+// v_readfirstlane, and a vector memory instruction may read an SGPR that a
+// vector instruction wrote only five wait states later, which the compiler
+// does not see to around inline assembly (tests/test_device_code.py checks the
+// distances).  So every round goes through it, offset 0 as well.
+__device__ __forceinline__ uint32_t round_offset(uint32_t off) {
+  asm volatile("" : "+s"(off));
+  return off;
+}
+
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return uint32_t(reinterpret_cast<uintptr_t>((SOL_LDS const void*)p));
 }
@@ -260,11 +273,7 @@ struct TileRefill {
         lane_bytes(uint32_t(lane) * 16u) {}
 
   __device__ __forceinline__ void round(int r) const {
-    // The round's offset passes through an empty asm so that it is formed
-    // here from an immediate, not kept live in registers of its own across
-    // the whole stream.
-    uint32_t off = uint32_t(r) * (NT * 16);
-    asm volatile("" : "+s"(off));
+    const uint32_t off = round_offset(uint32_t(r) * (NT * 16));
     dma16(src + off, lane_bytes, lds + off);
   }
   __device__ __forceinline__ void all() const {
@@ -353,10 +362,10 @@ struct RowRefill {
   __device__ __forceinline__ void round(int r) const {
     if (r < kHalf) {
       const uint32_t lane = (Src::kOddK && (r & 1)) ? klane_odd : klane;
-      dma16(ksrc + uint64_t(uint32_t(r) * kstep), lane, lds + uint32_t(r * NT * 16));
+      dma16(ksrc + round_offset(uint32_t(r) * kstep), lane, lds + uint32_t(r * NT * 16));
     } else {
       const int rv = r - kHalf;
-      dma16(vsrc + uint64_t(uint32_t(rv) * vstep), vlane, lds + uint32_t(TileLayout<D>::kElems * 2 + rv * NT * 16));
+      dma16(vsrc + round_offset(uint32_t(rv) * vstep), vlane, lds + uint32_t(TileLayout<D>::kElems * 2 + rv * NT * 16));
     }
   }
   __device__ __forceinline__ void all() const {
@@ -400,10 +409,10 @@ struct WindowRefill {
   __device__ __forceinline__ void round(int r) const {
     if (r < kHalf) {
       const uint32_t lane = (Src::kOddK && (r & 1)) ? klane_odd : klane;
-      dma16(ksrc + uint64_t(uint32_t(r) * kstep), lane, lds + uint32_t(r * NT * 16));
+      dma16(ksrc + round_offset(uint32_t(r) * kstep), lane, lds + uint32_t(r * NT * 16));
     } else {
       const int rv = r - kHalf;
-      dma16(vsrc + uint64_t(uint32_t(rv) * vstep), vlane, lds + uint32_t(TileLayout<D>::kElems * 2 + rv * NT * 16));
+      dma16(vsrc + round_offset(uint32_t(rv) * vstep), vlane, lds + uint32_t(TileLayout<D>::kElems * 2 + rv * NT * 16));
     }
   }
   __device__ __forceinline__ void all() const {
@@ -448,8 +457,7 @@ struct Q8Refill {
 
   __device__ __forceinline__ void round(int r) const {
     if (r < kK8Rounds) {
-      uint32_t off = uint32_t(r) * (NT * 16);
-      asm volatile("" : "+s"(off));
+      const uint32_t off = round_offset(uint32_t(r) * (NT * 16));
       dma16(k8src + off, lane_bytes, k8lds + off);
     } else {
       kv.round(r - kK8Rounds + kVRounds);
