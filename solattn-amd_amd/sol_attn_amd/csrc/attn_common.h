@@ -521,11 +521,13 @@ __device__ __forceinline__ uint64_t row_mask(uint64_t bits, int r) {
   return uint64_t(uint32_t(lo)) | (uint64_t(uint32_t(hi)) << 32);
 }
 
-// `on` in the lanes of a wave-uniform mask, `off` in the others.
+// `on` in the lanes of a wave-uniform mask, `off` in the others: one v_cndmask
+// on the mask's SGPRs.  (A builtin and not inline assembly: a vector
+// instruction may read an SGPR that another one wrote -- a mask spilled to a
+// vector register's lanes and read back -- only two wait states later, and the
+// compiler keeps that distance for its own instructions alone.)
 __device__ __forceinline__ float mask_select(uint64_t mask, float off, float on) {
-  float x;
-  asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(x) : "v"(off), "v"(on), "s"(mask));
-  return x;
+  return __builtin_amdgcn_inverse_ballot_w64(mask) ? on : off;
 }
 
 // Materialises a value at this point of the instruction stream, so that the

@@ -11,7 +11,8 @@ Wait states.  The compiler keeps the distances that the hardware does not check
 itself between instructions of its own, but does not look into inline assembly.
 An SGPR that a vector instruction wrote (v_readfirstlane, v_readlane, a compare)
 may be read by a vector memory instruction five wait states later, so the DMA's
-address must not come from one directly.
+address must not come from one directly, and by another vector instruction two
+wait states later.
 """
 
 import os
@@ -97,3 +98,9 @@ def test_dma_addresses_keep_their_distance_from_vector_writes(attention_asm):
     close = [(text, age) for text, inline, age in _sgpr_distances(attention_asm)
              if inline and text.startswith("global_load_lds") and age < 5]
     assert not close, f"{len(close)} DMAs read an SGPR a vector instruction has just written: {close[:4]!r}"
+
+
+def test_inline_vector_instructions_keep_their_distance_from_vector_writes(attention_asm):
+    close = [(text, age) for text, inline, age in _sgpr_distances(attention_asm)
+             if inline and text.startswith("v_") and age < 2]
+    assert not close, f"{len(close)} vector instructions read an SGPR another has just written: {close[:4]!r}"
