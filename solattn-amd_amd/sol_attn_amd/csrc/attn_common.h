@@ -622,12 +622,14 @@ struct HalfSoftmax {
 // Common case of HalfSoftmax without its max pass: the probabilities
 // p = exp2(s c - m) are formed against the running max m as it stands, and
 // the row sum tells whether that was what HalfSoftmax would have done.  If
-// no lane's sum exceeds 65,535 (or, before any key, 0), every p is below
+// every lane has a max and no lane's sum exceeds 65,535, every p is below
 // 2^16, i.e. every s c - m < log2(65,535) < kRescaleSlack, so HalfSoftmax would not
 // have moved m and would have formed these same p, den += lsum, with acc
 // untouched: the results are bit-identical.  Otherwise `redo` is set (a
 // wave-uniform ballot) and the caller re-forms the half's raw scores and
-// runs HalfSoftmax on them (resolve).  The stages are:
+// runs HalfSoftmax on them (resolve).  A lane without any key yet always asks
+// for that: the sum tells nothing there, as scores below -150 give p = 0 while
+// any key at all moves m.  The stages are:
 // 4 x 4 probabilities and the row sum; the redo ballot; BF16 packing; den.
 constexpr float kFastSumMax = 65535.f;
 
@@ -641,9 +643,9 @@ struct FastHalf {
   __device__ __forceinline__ void stage(int k, State<D>& st, float c) {
     if (k < 4) {
       if (k == 0) {
-        const bool none = st.m == kNegInf;  // nothing yet: p = exp2(s c), and any key moves m
+        const bool none = st.m == kNegInf;  // nothing yet: any sum exceeds -1
         neg_m = none ? 0.f : -st.m;
-        thr = none ? 0.f : kFastSumMax;
+        thr = none ? -1.f : kFastSumMax;
         lsum = 0.f;
       }
 #pragma unroll
