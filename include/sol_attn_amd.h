@@ -234,8 +234,7 @@ int64_t sol_route_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
  * agree with the other forms to rounding; decisions and counts are the
  * same), unless two or more query-sink blocks meet long keys
  * (small_key_split in csrc/sol_internal.h); otherwise one query block per
- * workgroup while a head's K and V are at most 16 MB or the launch has fewer
- * than 512 query-block pairs, else 2.  1 or 2 force one or two query blocks per
+ * workgroup where sol_attention_one_block says so, else 2.  1 or 2 force one or two query blocks per
  * workgroup without the key split (bit-identical results).  No counterpart
  * in the reference (one Triton program per query block).
  * ctiles / key_mean / key_var: NULL at beta = -INFINITY (unused), or where
@@ -257,6 +256,13 @@ int64_t sol_route_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
  * `_moments`, `_threshold` and `_sol` separately (kernels.py:203-225). */
 int sol_attention_pools_keys(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads,
                              int64_t head_dim);
+
+/* 1 when workgroup_form 0 holds one query block per workgroup for a problem
+ * (qk_int8: with INT8 key tiles), else 0.  Such launches make no use of
+ * pair_strides, and indexed windows pooled by sol_pool_windows are meant for
+ * them.  No counterpart in the reference. */
+int sol_attention_one_block(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads,
+                            int64_t head_dim, int qk_int8);
 
 int sol_attention_fwd(const void* q, const int64_t* q_strides, const int64_t* query_index,
                       int64_t sequence_length, int64_t batch, int64_t query_tokens, int64_t key_tokens,

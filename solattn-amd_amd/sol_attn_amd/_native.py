@@ -59,6 +59,7 @@ _SIGNATURES = {
     "sol_key_covariance": ([_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p], ctypes.c_int),
     "sol_quantize_keys": ([_p, _i64p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p, _p, _p], ctypes.c_int),
     "sol_attention_pools_keys": ([_i64, _i64, _i64, _i64, _i64], ctypes.c_int),
+    "sol_attention_one_block": ([_i64, _i64, _i64, _i64, _i64, _int], ctypes.c_int),
     "sol_attention_noalloc": ([_p, _i64p, _p, _i64p, _p, _i64p, _i64, _i64, _i64, _i64, _i64,
                                _dbl, _dbl, _i64, _i64, _i64, _p, _p, _p], ctypes.c_int),
     "sol_attention_workspace_size": ([_i64, _i64, _i64, _i64, _i64, _dbl, _i64, _i64, _i64], ctypes.c_int64),
@@ -278,23 +279,34 @@ PAIRING = True
 # paired: the three pairing kernels cost ~27 us, more than the union they
 # save on a short attention launch.
 PAIR_MIN_QUERY_BLOCKS = 8192
-# Nor are launches whose keys keep one query block per workgroup
-# (one_block_launch in csrc/sol_internal.h): K and V bytes per head up to this.
-ONE_BLOCK_KEY_BYTES = 16 << 20
+# Nor are launches that hold one query block per workgroup (_one_block).
+
+
+@functools.lru_cache(maxsize=256)
+def _one_block(b, nq, nk, h, d, int8):
+    return bool(library().sol_attention_one_block(b, nq, nk, h, d, int8))
 
 
 def _one_block_keys(nk, d):
-    """Key sequences whose launches hold one query block per workgroup."""
-    return -(-nk // BLOCK) * BLOCK * d * 4 <= ONE_BLOCK_KEY_BYTES
+    """Key sequences whose launches hold one query block per workgroup
+    however many query blocks there are."""
+    return _one_block(1, 1 << 20, nk, 64, d, False)
 
 
-def _pairs(b, nq, nk, h, d):
+def _pairs(b, nq, nk, h, d, int8):
     """Whether a call's attention launch pairs query blocks (a forced
     WORKGROUP_FORM or ROUTE_PREPASS "always" leaves the size rule aside)."""
     if not PAIRING or b * h * -(-nq // BLOCK) < PAIR_MIN_QUERY_BLOCKS:
         return False
     return (WORKGROUP_FORM != 0 or ROUTE_PREPASS == "always"
-            or not _one_block_keys(nk, d))
+            or not _one_block(b, nq, nk, h, d, int8))
+
+
+def _windows(b, nq, nk, h, d, int8):
+    """Whether an indexed launch reads key blocks of consecutive rows from K
+    and V (sol_pool_windows), which the one-block form does."""
+    return _one_block_keys(nk, d) and (WORKGROUP_FORM == 1 or (
+        WORKGROUP_FORM == 0 and _one_block(b, nq, nk, h, d, int8)))
 
 
 def _pair_buffers(q, rows, min_blocks):
@@ -580,7 +592,8 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
              and ROUTE_PREPASS != "always")
     b, nq = rows.shape if rows is not None else q.shape[:2]
     nk = keys.shape[1] if keys is not None else k.shape[1]
-    pairs = _pairs(b, nq, nk, *q.shape[-2:])
+    int8 = qk_precision == "int8"
+    pairs = _pairs(b, nq, nk, *q.shape[-2:], int8)
     if ALL_IN and plain and protection is None and out is None and SELF_POOLING and SPLIT_SINKS and not pairs:
         # No pairing pass: pooling and attention in one C-ABI call.
         return _all_in(q, k, v, float(scale), float(beta), int(local), int(kv_sink), int(q_sink), stats)
@@ -610,8 +623,8 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
             strides, means = pairing[2], pairing[3]
     try:
         pooled = pool_kv(k, v, key_index=keys, moments=not math.isinf(beta), key_lengths=key_lengths,
-                         stream=stream, views=debug, qk_int8=qk_precision == "int8",
-                         windows=WORKGROUP_FORM != 2 and _one_block_keys(nk, q.shape[-1]))
+                         stream=stream, views=debug, qk_int8=int8,
+                         windows=keys is not None and _windows(b, nq, nk, *q.shape[-2:], int8))
         if threshold_estimator == "full_covariance" and not math.isinf(beta):
             key_covariance(pooled, stream)
     finally:

@@ -137,9 +137,9 @@ double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blo
 }
 
 int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, double beta,
-                int64_t head_dim) {
+                int64_t head_dim, bool int8) {
   const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
-                          (force == 0 && sol::one_block_launch(bh, nqb, nkb, head_dim) &&
+                          (force == 0 && sol::one_block_launch(bh, nqb, nkb, head_dim, int8) &&
                            ((bh * nqb <= 2048 && nkb >= 128) ||
                             sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2));
   // Launches of the small kernel split every query block's chain inside its
@@ -436,7 +436,7 @@ int64_t sol_split_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
     return 0;
   const int64_t bh = batch * heads, nqb = cdiv(query_tokens, SOL_BLOCK), qsb = sink_blocks(query_sink_tokens);
   const int force = std::isinf(beta) ? (beta < 0 ? 1 : 2) : 0;
-  const int s = sink_splits(bh, nqb, cdiv(key_tokens, SOL_BLOCK), qsb, force, beta, head_dim);
+  const int s = sink_splits(bh, nqb, cdiv(key_tokens, SOL_BLOCK), qsb, force, beta, head_dim, false);
   return split_bytes(bh, qsb, s, head_dim);
 }
 
@@ -453,6 +453,14 @@ int sol_attention_pools_keys(int64_t batch, int64_t query_tokens, int64_t key_to
                              int64_t head_dim) {
   return shape_ok(batch, query_tokens, heads, head_dim) && key_tokens > 0 && key_tokens < (int64_t(1) << 30) &&
                  pools_keys(batch, query_tokens, key_tokens, heads, head_dim)
+             ? 1 : 0;
+}
+
+int sol_attention_one_block(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads,
+                            int64_t head_dim, int qk_int8) {
+  return shape_ok(batch, query_tokens, heads, head_dim) && key_tokens > 0 && key_tokens < (int64_t(1) << 30) &&
+                 sol::one_block_launch(batch * heads, cdiv(query_tokens, SOL_BLOCK), cdiv(key_tokens, SOL_BLOCK),
+                                       head_dim, qk_int8 != 0)
              ? 1 : 0;
 }
 
@@ -695,7 +703,9 @@ int attention_fwd_impl(const void* q, const int64_t* q_strides, const int64_t* q
   p.local_blocks = int(local_blocks < 0 ? -1 : (local_blocks > big ? big : local_blocks));
   p.kv_sink_blocks = int(cdiv(kv_sink_tokens > big ? big : kv_sink_tokens, SOL_BLOCK));
   p.q_sink_blocks = int(sink_blocks(query_sink_tokens));
-  p.splits = split_workspace ? sink_splits(batch * heads, nqb, nkb, p.q_sink_blocks, force, beta, head_dim) : 1;
+  // INT8 launches split no more than others of the same sizes: the workspace holds either.
+  p.splits = split_workspace ? sink_splits(batch * heads, nqb, nkb, p.q_sink_blocks, force, beta, head_dim,
+                                           qk_int8_tiles != nullptr) : 1;
   p.partial = p.splits > 1 ? static_cast<float*>(split_workspace) : nullptr;
   p.mask = force != 1 ? static_cast<uint32_t*>(route_workspace) : nullptr;
   p.order = p.mask ? reinterpret_cast<int32_t*>(static_cast<uint8_t*>(route_workspace) +

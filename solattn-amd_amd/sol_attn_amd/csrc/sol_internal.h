@@ -166,10 +166,17 @@ inline int64_t head_key_bytes(int64_t nkb, int64_t head_dim) { return nkb * kBlo
 // 2896 -> 2902; 40,960 x 8 1505 -> 1573, 1713 -> 1648; 65,536 x 8 3705 ->
 // 4585, at D64 (16 MB) 2077 -> 1995.  Launches of fewer than 512 pairs (256
 // CUs x 2 workgroups) would leave CUs idle with two.
+// INT8 scores (the experiment) have no one-slot form: at head_dim 128 a
+// one-block workgroup holds a 64 KB ring too, so a CU has half the waves of the
+// two-block form.  us per call, one block -> two: 2 x 4,096 x 16 heads beta 1
+// 155 -> 130, beta 0 269 -> 207; 16,384 x 8 367 -> 307; 32,768 x 16 2417 ->
+// 2052; 21 x 4,032 windows x 24 10258 -> 8587.  (At 64 the ring is 32 KB: 2 x
+// 4,096 x 16 93 -> 83 the other way round.)
 constexpr int64_t kOneBlockKeyBytes = int64_t(16) << 20;
 constexpr int64_t kSmallLaunchGroups = 512;
-inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_dim) {
-  return head_key_bytes(nkb, head_dim) <= kOneBlockKeyBytes || bh * ((nqb + 1) / 2) < kSmallLaunchGroups;
+inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_dim, bool int8) {
+  if (bh * ((nqb + 1) / 2) < kSmallLaunchGroups) return true;
+  return head_key_bytes(nkb, head_dim) <= kOneBlockKeyBytes && !(int8 && head_dim == 128);
 }
 
 // The flat workgroup map (sol_task) keeps an XCD on its own heads, so a head's
