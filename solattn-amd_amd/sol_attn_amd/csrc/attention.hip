@@ -861,7 +861,7 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
   const int ntiles = (p.NQB + G - 1) / G;
   const int front = min(p.q_sink_blocks, ntiles);
   const int split_tiles = sink_split_tiles(p.splits, p.q_sink_blocks, G, front);
-  TileTask task = sol_task(blockIdx.x, ntiles, front, split_tiles, p.B * p.H, p.splits, p.flat);
+  TileTask task = sol_task(blockIdx.x, ntiles, front, split_tiles, p.B * p.H, p.splits, p.head_xcds);
   if (task.bh < 0) return;
   if (G == 2 && p.order && task.tile >= front)  // the order_kernel's deal of the regular tiles
     task.tile = front + p.order[int64_t(task.bh) * p.NQB + task.tile - front];
@@ -1902,11 +1902,12 @@ constexpr int kSlots1 = 1;
 template <int D, int G, bool SEG>
 void launch_sol_variant(const AttnParams& p, hipStream_t stream) {
   // Grid of sol_task: the sink-holding tiles of every head (p.splits
-  // workgroups each), then balanced_task's.
+  // workgroups each), then balanced_task's or HeadMap's.
   const int ntiles = (p.NQB + G - 1) / G, front = std::min(p.q_sink_blocks, ntiles);
   const int split_tiles = sink_split_tiles(p.splits, p.q_sink_blocks, G, front);
   const int F = (split_tiles * (p.splits - 1) + front) * (p.B * p.H);
-  const unsigned grid = p.flat ? flat_grid(F, p.B * p.H, ntiles - front) : balanced_grid(F, p.B * p.H, ntiles - front);
+  const unsigned grid = p.head_xcds ? head_grid(F, p.B * p.H, ntiles - front, p.head_xcds)
+                                    : balanced_grid(F, p.B * p.H, ntiles - front);
   // Key blocks from pooled tile pairs (p.tiles) or straight from K / V rows.
   if (p.tiles) {
     if (p.k8)
@@ -1981,7 +1982,8 @@ hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
   if (p.workgroup_form == 1 || p.workgroup_form == 2) g = p.workgroup_form;
   if (p.block_rows) g = 1;  // read by the one-block form only
   AttnParams q = p;
-  q.flat = head_key_bytes(p.NKB, D) <= kFlatKeyBytes ? 1 : 0;
+  q.head_xcds = g == 1 && head_key_bytes(p.NKB, D) <= kHeadMapKeyBytes
+                    ? xcds_per_head(int64_t(p.B) * p.H, p.NKB) : 0;
   q.order = nullptr;
   if (g == 2 && p.order && p.mask && p.force != 1 && p.splits == 1) {
     const int ntiles = (p.NQB + 1) / 2, front = std::min(p.q_sink_blocks, ntiles);

@@ -107,7 +107,7 @@ struct AttnParams {
                        // null: the attention kernel routes tile by tile
   int NW;              // ceil(NKB / 32)
   const float* qc;     // [B, H, NQB, D] FP32 query-block means for route_kernel, or null (formed from Q)
-  int flat;            // workgroup map: 1 = one eighth of all heads' tiles per XCD (sol_task)
+  int head_xcds;       // workgroup map: XCDs a head's tiles are kept on (HeadMap), or 0: all (balanced_task)
   int32_t* order;      // [B H, NQB] with mask: the regular query tiles of a two-block launch in
                        // the order order_kernel deals them to the XCDs, or null: tile order
 };
@@ -179,14 +179,33 @@ inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_
   return head_key_bytes(nkb, head_dim) <= kOneBlockKeyBytes && !(int8 && head_dim == 128);
 }
 
-// The flat workgroup map (sol_task) keeps an XCD on its own heads, so a head's
-// keys are read into one or two L2s instead of eight: 4,096 x 10,000 keys x 24
-// heads 185 -> 138 us, 19,003 x 16 708 -> 632 (one block per workgroup).  With
-// K and V per head far beyond the L2 it gains nothing, and eight heads at a
-// time no longer fit the 256 MB memory-side cache: 40,960 x 8 heads (20 MB)
-// 1544 -> 1505, 49,152 (24 MB) 2264 -> 2258, 65,536 (32 MB) 3662 -> 3705,
-// 84,672 x 24 (43 MB) 17056 -> 18243 (two blocks).
-constexpr int64_t kFlatKeyBytes = int64_t(24) << 20;
+// XCDs per head of a one-block launch (HeadMap; 0: balanced_task, every head
+// on all eight).  On fewer, more of an XCD's workgroups stream the same keys
+// through its L2 -- heads alike, 1, 2, 4 XCDs and all: 19,003 tokens x 16 heads
+// 654, 657, 686, 777 us a call, 8,192 x 24 212, 213, 227, 264, 2 x 4,096 x 16
+// 100, 101, 108, 121 -- but an XCD's work is what its heads select, and heads
+// do differ: with one of 16 heads at half the blocks and the others at 2% (19,003,
+// beta 2) 640, 501, 379, 334 us, where two-block workgroups on the
+// balanced map took 388.  So the fewest XCDs at which the most that one head can
+// hold up its group is kUnevenMax times the average.  A head costs at least 8
+// steps' time and its centroid tiles per query block, at most half the key
+// blocks more (the threshold is at least the mean); one such head among a
+// group's P and the launch's `heads`.  Over 150 inputs -- one dense head, a
+// quarter, every fourth, random densities; 4,096 to 24,576 tokens, 8 to 32 heads
+// -- the launches took 0.69 to 1.04 of the two-block form's time there.
+constexpr double kUnevenMax = 1.7;
+inline int xcds_per_head(int64_t heads, int64_t nkb) {
+  const double base = 8.0 + double(nkb) / kBlock, more = 0.5 * double(nkb) / base;
+  for (int xcds = 1; xcds <= 4; xcds *= 2) {
+    const double group = double(heads) * xcds / 8.0;
+    if ((more / group + 1.0) <= kUnevenMax * (more / double(heads) + 1.0)) return xcds;
+  }
+  return 0;
+}
+
+// With K and V per head far beyond the L2 a head's own XCDs gain nothing, and
+// eight heads at a time no longer fit the 256 MB memory-side cache.
+constexpr int64_t kHeadMapKeyBytes = int64_t(24) << 20;
 
 hipError_t launch_pool(const PoolParams& p, int D, hipStream_t stream);
 hipError_t launch_quantize_keys(const QuantParams& p, int D, hipStream_t stream);
