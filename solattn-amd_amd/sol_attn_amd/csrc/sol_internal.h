@@ -182,17 +182,17 @@ inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_
 // XCDs per head of a one-block launch (HeadMap; 0: balanced_task, every head
 // on all eight).  On fewer, more of an XCD's workgroups stream the same keys
 // through its L2 -- heads alike, 1, 2, 4 XCDs and all: 19,003 tokens x 16 heads
-// 654, 657, 686, 777 us a call, 8,192 x 24 212, 213, 227, 264, 2 x 4,096 x 16
-// 100, 101, 108, 121 -- but an XCD's work is what its heads select, and heads
+// 654, 657, 692, 777 us a call, 8,192 x 24 212, 212, 227, 264, 2 x 4,096 x 16
+// 100, 100, 108, 121 -- but an XCD's work is what its heads select, and heads
 // do differ: with one of 16 heads at half the blocks and the others at 2% (19,003,
 // beta 2) 640, 501, 379, 334 us, where two-block workgroups on the
 // balanced map took 388.  So the fewest XCDs at which the most that one head can
 // hold up its group is kUnevenMax times the average.  A head costs at least 8
 // steps' time and its centroid tiles per query block, at most half the key
 // blocks more (the threshold is at least the mean); one such head among a
-// group's P and the launch's `heads`.  Over 150 inputs -- one dense head, a
+// group's P and the launch's `heads`.  Over 72 inputs -- one dense head, a
 // quarter, every fourth, random densities; 4,096 to 24,576 tokens, 8 to 32 heads
-// -- the launches took 0.69 to 1.04 of the two-block form's time there.
+// -- the launches took 0.61 to 0.99 of the two-block form's time there.
 constexpr double kUnevenMax = 1.7;
 inline int xcds_per_head(int64_t heads, int64_t nkb) {
   const double base = 8.0 + double(nkb) / kBlock, more = 0.5 * double(nkb) / base;

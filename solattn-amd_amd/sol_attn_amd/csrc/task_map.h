@@ -58,39 +58,53 @@ __host__ __device__ inline unsigned balanced_grid(int F, int heads, int R) {
   return unsigned(kXcds * ((total + kXcds - 1) / kXcds));
 }
 
+// Start of XCD x's even share of n tasks in a row.
+__host__ __device__ inline int xcd_start(int n, int x) { return n / kXcds * x + n % kXcds * x / kXcds; }
+
 // The other map (`head_xcds` = 1, 2 or 4): every head -- (entry, head) pair --
 // belongs to a group of that many XCDs, so that its keys are read into those
 // L2s alone instead of all eight.  Whole rounds of heads are dealt to the 8 /
 // head_xcds groups in turn, each round starting three groups further on (heads
 // that cost alike at a regular distance, as those of a batch's entries, meet
 // different groups); the tiles of the last, partial round are one list that is
-// cut evenly over the groups.  A group's XCDs take its list's tiles in turn.
+// cut evenly over the XCDs.  A group's XCDs take a slice of a head's tiles each
+// -- neighbouring tiles select much the same keys: dealt out one by one a video
+// field of 19,003 tokens x 16 heads took 719 us a call, in slices 659 -- and the
+// slices are passed round from head to head, as R need not divide evenly.
 struct HeadMap {
   int xcds, groups;     // XCDs per group; groups
   int rounds, rest, R;  // whole rounds of heads, heads of the partial one, tiles per head
   __host__ __device__ HeadMap(int heads, int R, int xcds)
       : xcds(xcds), groups(kXcds / xcds), rounds(heads / groups), rest(heads % groups), R(R) {}
-  // Start of group g's part of the partial round's list.
-  __host__ __device__ int cut(int g) const { return rest * R / groups * g + rest * R % groups * g / groups; }
-  // Tiles of XCD x.
-  __host__ __device__ int count(int x) const {
-    const int g = x / xcds, m = x % xcds, n = rounds * R + cut(g + 1) - cut(g);
-    return n > m ? (n - m - 1) / xcds + 1 : 0;
+  // Start of slice s of a head's tiles, and the slice the m-th XCD takes in round r.
+  __host__ __device__ int slice(int s) const { return R / xcds * s + R % xcds * s / xcds; }
+  __host__ __device__ int turn(int m, int r) const { return (m + r) % xcds; }
+  // Tiles of XCD x in the whole rounds (R in every `xcds` of them), and in all.
+  __host__ __device__ int whole(int x) const {
+    int n = rounds / xcds * R;
+    for (int r = 0; r < rounds % xcds; ++r) n += slice(turn(x % xcds, r) + 1) - slice(turn(x % xcds, r));
+    return n;
   }
+  __host__ __device__ int count(int x) const { return whole(x) + xcd_start(rest * R, x + 1) - xcd_start(rest * R, x); }
   // The k-th tile of XCD x (-1: past its last one).
   __host__ __device__ TileTask task(int x, int k) const {
     if (k >= count(x)) return TileTask{-1, 0};
-    const int g = x / xcds;
-    const uint32_t j = uint32_t(k * xcds + x % xcds);
-    const int r = int(j / uint32_t(R)), t = int(j % uint32_t(R));
-    if (r < rounds) return TileTask{r * groups + (g + 3 * r) % groups, t};
-    const uint32_t e = uint32_t(cut(g)) + (j - uint32_t(rounds * R));
-    return TileTask{rounds * groups + int(e / uint32_t(R)), int(e % uint32_t(R))};
+    const int w = whole(x);
+    if (k >= w) {
+      const uint32_t j = uint32_t(xcd_start(rest * R, x) + (k - w));
+      return TileTask{rounds * groups + int(j / uint32_t(R)), int(j % uint32_t(R))};
+    }
+    const int m = x % xcds;
+    int r = int(uint32_t(k) / uint32_t(R)) * xcds, t = int(uint32_t(k) % uint32_t(R));
+    int s = m, n = slice(s + 1) - slice(s);  // round r is a whole cycle's first: turn(m, r) = m
+    while (t >= n) {
+      t -= n;
+      s = turn(m, ++r);
+      n = slice(s + 1) - slice(s);
+    }
+    return TileTask{r * groups + (x / xcds + 3 * r) % groups, slice(s) + t};
   }
 };
-
-// Start of XCD x's even share of n front ids.
-__host__ __device__ inline int front_start(int n, int x) { return n / kXcds * x + n % kXcds * x / kXcds; }
 
 // Workgroups of a HeadMap launch of F front ids and `heads` x R regular tiles:
 // the fullest XCD's, eight times.
@@ -98,7 +112,7 @@ inline unsigned head_grid(int F, int heads, int R, int xcds) {
   const HeadMap map(heads, R, xcds);
   int most = 0;
   for (int x = 0; x < kXcds; ++x) {
-    const int n = front_start(F, x + 1) - front_start(F, x) + map.count(x);
+    const int n = xcd_start(F, x + 1) - xcd_start(F, x) + map.count(x);
     most = n > most ? n : most;
   }
   return unsigned(kXcds) * unsigned(most);
@@ -120,9 +134,9 @@ __host__ __device__ inline TileTask sol_task(int i, int ntiles, int front, int s
     const int x = i % kXcds, k = i / kXcds;
     const int per = split_tiles * splits + (front - split_tiles);  // front ids per head
     const int F = per * heads;
-    const int nf = front_start(F, x + 1) - front_start(F, x);
+    const int nf = xcd_start(F, x + 1) - xcd_start(F, x);
     if (k < nf) {
-      const uint32_t j = uint32_t(front_start(F, x) + k);
+      const uint32_t j = uint32_t(xcd_start(F, x) + k);
       const int h = int(j / uint32_t(per)), e = int(j % uint32_t(per));
       if (e < split_tiles * splits) return TileTask{h, e / splits, e % splits};
       return TileTask{h, split_tiles + e - split_tiles * splits};
