@@ -259,10 +259,10 @@ int sol_attention_pools_keys(int64_t batch, int64_t query_tokens, int64_t key_to
 
 /* 1 when workgroup_form 0 holds one query block per workgroup for a problem
  * (qk_int8: with INT8 key tiles), else 0.  Such launches make no use of
- * pair_strides, and indexed windows pooled by sol_pool_windows are meant for
- * them.  No counterpart in the reference. */
+ * pair_strides.  windows: 1 when indexed windows are worth pooling by
+ * sol_pool_windows (sol_attention_windows always holds one query block).  No counterpart in the reference. */
 int sol_attention_one_block(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads,
-                            int64_t head_dim, int qk_int8);
+                            int64_t head_dim, double beta, int qk_int8, int windows);
 
 int sol_attention_fwd(const void* q, const int64_t* q_strides, const int64_t* query_index,
                       int64_t sequence_length, int64_t batch, int64_t query_tokens, int64_t key_tokens,

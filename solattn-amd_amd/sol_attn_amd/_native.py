@@ -59,7 +59,7 @@ _SIGNATURES = {
     "sol_key_covariance": ([_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p, _p], ctypes.c_int),
     "sol_quantize_keys": ([_p, _i64p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _p, _p, _p], ctypes.c_int),
     "sol_attention_pools_keys": ([_i64, _i64, _i64, _i64, _i64], ctypes.c_int),
-    "sol_attention_one_block": ([_i64, _i64, _i64, _i64, _i64, _int], ctypes.c_int),
+    "sol_attention_one_block": ([_i64, _i64, _i64, _i64, _i64, _dbl, _int, _int], ctypes.c_int),
     "sol_attention_noalloc": ([_p, _i64p, _p, _i64p, _p, _i64p, _i64, _i64, _i64, _i64, _i64,
                                _dbl, _dbl, _i64, _i64, _i64, _p, _p, _p], ctypes.c_int),
     "sol_attention_workspace_size": ([_i64, _i64, _i64, _i64, _i64, _dbl, _i64, _i64, _i64], ctypes.c_int64),
@@ -283,30 +283,30 @@ PAIR_MIN_QUERY_BLOCKS = 8192
 
 
 @functools.lru_cache(maxsize=256)
-def _one_block(b, nq, nk, h, d, int8):
-    return bool(library().sol_attention_one_block(b, nq, nk, h, d, int8))
+def _one_block(b, nq, nk, h, d, beta, int8, windows):
+    return bool(library().sol_attention_one_block(b, nq, nk, h, d, beta, int8, windows))
 
 
 def _one_block_keys(nk, d):
-    """Key sequences whose launches hold one query block per workgroup
+    """Key sequences whose launches may hold one query block per workgroup
     however many query blocks there are."""
-    return _one_block(1, 1 << 20, nk, 64, d, False)
+    return _one_block(1, 1 << 20, nk, 64, d, math.inf, False, False)
 
 
-def _pairs(b, nq, nk, h, d, int8):
+def _pairs(b, nq, nk, h, d, beta, int8, windows):
     """Whether a call's attention launch pairs query blocks (a forced
     WORKGROUP_FORM or ROUTE_PREPASS "always" leaves the size rule aside)."""
     if not PAIRING or b * h * -(-nq // BLOCK) < PAIR_MIN_QUERY_BLOCKS:
         return False
     return (WORKGROUP_FORM != 0 or ROUTE_PREPASS == "always"
-            or not _one_block(b, nq, nk, h, d, int8))
+            or not _one_block(b, nq, nk, h, d, beta, int8, windows))
 
 
-def _windows(b, nq, nk, h, d, int8):
+def _windows(b, nq, nk, h, d, beta, int8):
     """Whether an indexed launch reads key blocks of consecutive rows from K
     and V (sol_pool_windows), which the one-block form does."""
     return _one_block_keys(nk, d) and (WORKGROUP_FORM == 1 or (
-        WORKGROUP_FORM == 0 and _one_block(b, nq, nk, h, d, int8)))
+        WORKGROUP_FORM == 0 and _one_block(b, nq, nk, h, d, beta, int8, True)))
 
 
 def _pair_buffers(q, rows, min_blocks):
@@ -593,7 +593,8 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
     b, nq = rows.shape if rows is not None else q.shape[:2]
     nk = keys.shape[1] if keys is not None else k.shape[1]
     int8 = qk_precision == "int8"
-    pairs = _pairs(b, nq, nk, *q.shape[-2:], int8)
+    beta = float(beta)
+    pairs = _pairs(b, nq, nk, *q.shape[-2:], beta, int8, keys is not None)
     if ALL_IN and plain and protection is None and out is None and SELF_POOLING and SPLIT_SINKS and not pairs:
         # No pairing pass: pooling and attention in one C-ABI call.
         return _all_in(q, k, v, float(scale), float(beta), int(local), int(kv_sink), int(q_sink), stats)
@@ -624,7 +625,7 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
     try:
         pooled = pool_kv(k, v, key_index=keys, moments=not math.isinf(beta), key_lengths=key_lengths,
                          stream=stream, views=debug, qk_int8=int8,
-                         windows=keys is not None and _windows(b, nq, nk, *q.shape[-2:], int8))
+                         windows=keys is not None and _windows(b, nq, nk, *q.shape[-2:], beta, int8))
         if threshold_estimator == "full_covariance" and not math.isinf(beta):
             key_covariance(pooled, stream)
     finally:

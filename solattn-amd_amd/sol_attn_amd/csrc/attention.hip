@@ -1978,7 +1978,8 @@ hipError_t launch_sol(const AttnParams& p, int D, hipStream_t stream) {
   }
   // AttnParams::workgroup_form 1 or 2 forces one form (tests run both: results are bit-identical -- a wave's
   // tiles, their order and its softmax state do not depend on its partner).
-  int g = one_block_launch(int64_t(p.B) * p.H, p.NQB, p.NKB, D, p.k8 != nullptr) ? 1 : 2;
+  int g = one_block_launch(int64_t(p.B) * p.H, p.NQB, p.NKB, D, selected_share(p.force, p.beta), p.k8 != nullptr,
+                           false) ? 1 : 2;
   if (p.workgroup_form == 1 || p.workgroup_form == 2) g = p.workgroup_form;
   if (p.block_rows) g = 1;  // read by the one-block form only
   AttnParams q = p;

@@ -101,7 +101,7 @@ int64_t route_mask_bytes(int64_t batch, int64_t query_tokens, int64_t key_tokens
 // query-sink block selects every key block, so its workgroup streams all of
 // them and, in a launch of few workgroups, ends long after the rest.  Split:
 // launches of fewer than 512 query-block pairs over all (entry, head) pairs,
-// one-block launches at finite beta of at most 2,048 query blocks over at least
+// launches at finite beta with K and V of at most 16 MB per head, of at most 2,048 query blocks over at least
 // 128 key blocks (8,192 tokens x 16 heads beta 1 210 -> 188, beta 0 343 ->
 // 335), or whose sink chain is at least twice the steps a workgroup slot has
 // on average (sink_chain_ratio), and at beta = +inf (every other workgroup
@@ -112,6 +112,7 @@ int64_t route_mask_bytes(int64_t batch, int64_t query_tokens, int64_t key_tokens
 // heads beta 1 116 -> 123).  beta = -inf (every block exact), fewer than two
 // sink blocks and sinks over a quarter of the query blocks are not split.
 constexpr int64_t kSplitBytesMax = int64_t(64) << 20;
+constexpr int64_t kSplitKeyBytes = int64_t(16) << 20;  // K and V per head of larger launches
 
 int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t head_dim) {
   // Split tiles hold sink blocks [0, 2 floor(q_sink_blocks / 2)) (sink_split_tiles).
@@ -129,7 +130,7 @@ int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t h
 // -> 91, 4,096 x 32 (2.4) 78 -> 77.
 double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, double beta, int64_t head_dim) {
   const double slots = head_dim == 64 ? 1536 : 1024;
-  const double share = 0.5 * std::erfc(beta / std::sqrt(2.0));
+  const double share = sol::selected_share(0, beta);
   const double regular = share * double(nkb) + double(nkb) / SOL_BLOCK + 8;
   const double sinks = double(std::min(q_sink_blocks, nqb));
   const double steps = double(bh) * (sinks * double(nkb) + (double(nqb) - sinks) * regular);
@@ -139,7 +140,7 @@ double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blo
 int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, double beta,
                 int64_t head_dim, bool int8) {
   const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
-                          (force == 0 && sol::one_block_launch(bh, nqb, nkb, head_dim, int8) &&
+                          (force == 0 && sol::head_key_bytes(nkb, head_dim) <= kSplitKeyBytes && !(int8 && head_dim == 128) &&
                            ((bh * nqb <= 2048 && nkb >= 128) ||
                             sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2));
   // Launches of the small kernel split every query block's chain inside its
@@ -457,10 +458,11 @@ int sol_attention_pools_keys(int64_t batch, int64_t query_tokens, int64_t key_to
 }
 
 int sol_attention_one_block(int64_t batch, int64_t query_tokens, int64_t key_tokens, int64_t heads,
-                            int64_t head_dim, int qk_int8) {
+                            int64_t head_dim, double beta, int qk_int8, int windows) {
+  const int force = std::isinf(beta) ? (beta < 0 ? 1 : 2) : 0;
   return shape_ok(batch, query_tokens, heads, head_dim) && key_tokens > 0 && key_tokens < (int64_t(1) << 30) &&
                  sol::one_block_launch(batch * heads, cdiv(query_tokens, SOL_BLOCK), cdiv(key_tokens, SOL_BLOCK),
-                                       head_dim, qk_int8 != 0)
+                                       head_dim, sol::selected_share(force, beta), qk_int8 != 0, windows != 0)
              ? 1 : 0;
 }
 

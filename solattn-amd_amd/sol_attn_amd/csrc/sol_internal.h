@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "sol_device.h"
 
 namespace sol {
@@ -153,30 +155,46 @@ inline int small_key_split(int64_t blocks, int64_t nkb, int64_t q_sink_blocks, i
 // K and V bytes of one head's key blocks.
 inline int64_t head_key_bytes(int64_t nkb, int64_t head_dim) { return nkb * kBlock * head_dim * 4; }
 
+// Share of the key blocks that a query block selects, as the threshold aims at
+// it: that of a normal above beta (force 1: beta = -inf, 2: +inf).
+inline double selected_share(int force, double beta) {
+  return force == 1 ? 1.0 : force == 2 ? 0.0 : 0.5 * std::erfc(beta / std::sqrt(2.0));
+}
+
 // One query block per workgroup (a K and a V slot each, four workgroups per
 // CU at head_dim 128) or two (a ring of two slots, the union of the pair's
 // blocks, two workgroups per CU); AttnParams::workgroup_form 0.  Two blocks
 // stream fewer bytes, but a wave idles on the tiles only its partner selected.
-// While the keys come from the L2s the idle waves cost more; past about 16 MB
-// of K and V per head the bytes do (more than the 4 MB L2s hold, at about 7
-// TB/s from beyond them).  Attention launches, one box, us, two blocks -> one,
-// flat map: 4,096 x 10,000 keys x 24 heads x D128 170 -> 138; 2 x 4,096 x 16
-// 103 -> 94; 16,384 x 8 x D64 200 -> 160; 24,576 x 8 x D128 565 -> 531 (video
-// field), 618 -> 541 (random); 32,768 x 8 945 -> 927, 1075 -> 982, x 24 heads
-// 2896 -> 2902; 40,960 x 8 1505 -> 1573, 1713 -> 1648; 65,536 x 8 3705 ->
-// 4585, at D64 (16 MB) 2077 -> 1995.  Launches of fewer than 512 pairs (256
-// CUs x 2 workgroups) would leave CUs idle with two.
+// One block while at most half the key blocks are selected, these are no more
+// than half the head's query blocks (the workgroups that share a key tile's
+// read from the L2), and K and V are at most 12 MB per head, 5 MB of them
+// selected.  us a call, two blocks -> one, video field and random: 2 x 4,096 x
+// 16 heads x D128 beta 1 119 -> 102, 125 -> 100, beta 0 205 -> 192, 217 -> 194,
+// beta -1 9% and 5% slower; 4,096 x 10,000 keys x 24 beta 1 193 -> 179, 219 ->
+// 185, beta 0 3% slower in the field; 2,048 x 8,192 x 32 beta 1 8% slower in the
+// field; 24,576 x 24 beta 1 1860 -> 1719, 1971 -> 1932, beta 0 7% and 1% slower.
+// Indexed windows need no copies of their keys in the one-block form: while 70%
+// are selected, or with at most 192 key blocks (two -> one: 21 x 4,032 x 24
+// beta 0 13753 -> 11878, beta -1 1% slower, at D64 beta -inf 9480 -> 9793; 21 x
+// 2,000 x 24 beta -inf 4815 -> 4372).
+// Launches of fewer than 512 pairs (256 CUs x 2 workgroups) would leave CUs
+// idle with two.
 // INT8 scores (the experiment) have no one-slot form: at head_dim 128 a
 // one-block workgroup holds a 64 KB ring too, so a CU has half the waves of the
 // two-block form.  us per call, one block -> two: 2 x 4,096 x 16 heads beta 1
 // 155 -> 130, beta 0 269 -> 207; 16,384 x 8 367 -> 307; 32,768 x 16 2417 ->
 // 2052; 21 x 4,032 windows x 24 10258 -> 8587.  (At 64 the ring is 32 KB: 2 x
 // 4,096 x 16 93 -> 83 the other way round.)
-constexpr int64_t kOneBlockKeyBytes = int64_t(16) << 20;
+constexpr int64_t kOneBlockKeyBytes = int64_t(12) << 20;
+constexpr double kOneBlockSelectedBytes = 5 << 20;
 constexpr int64_t kSmallLaunchGroups = 512;
-inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_dim, bool int8) {
+inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_dim, double share, bool int8,
+                             bool windows) {
   if (bh * ((nqb + 1) / 2) < kSmallLaunchGroups) return true;
-  return head_key_bytes(nkb, head_dim) <= kOneBlockKeyBytes && !(int8 && head_dim == 128);
+  const int64_t bytes = head_key_bytes(nkb, head_dim);
+  if (bytes > kOneBlockKeyBytes || (int8 && head_dim == 128)) return false;
+  if (windows) return share <= 0.7 || nkb <= 192;
+  return share <= 0.5 && 2 * share * double(nkb) <= double(nqb) && share * double(bytes) <= kOneBlockSelectedBytes;
 }
 
 // XCDs per head of a one-block launch (HeadMap; 0: balanced_task, every head
