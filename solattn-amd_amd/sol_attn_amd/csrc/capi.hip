@@ -101,12 +101,11 @@ int64_t route_mask_bytes(int64_t batch, int64_t query_tokens, int64_t key_tokens
 // query-sink block selects every key block, so its workgroup streams all of
 // them and, in a launch of few workgroups, ends long after the rest.  Split:
 // launches of fewer than 512 query-block pairs over all (entry, head) pairs,
-// launches at finite beta with K and V of at most 16 MB per head, of at most 2,048 query blocks over at least
-// 128 key blocks (8,192 tokens x 16 heads beta 1 210 -> 188, beta 0 343 ->
-// 335), or whose sink chain is at least twice the steps a workgroup slot has
-// on average (sink_chain_ratio), and at beta = +inf (every other workgroup
-// streams its protected blocks only) launches of up to 8,192 query blocks (8
-// rounds of 512 two-block workgroups).  Parts hold at least 16 key blocks, at
+// launches at finite beta with K and V of at most 16 MB per head whose sink
+// chain is at least twice the steps a workgroup slot has on average
+// (sink_chain_ratio), and at beta = +inf (every other workgroup streams its
+// protected blocks only) launches of up to 8,192 query blocks (8 rounds of 512
+// two-block workgroups).  Parts hold at least 16 key blocks, at
 // most 8 parts, while their partial states fit kSplitBytesMax.  Otherwise the
 // other workgroups fill the time, and the merge comes on top (2 x 4,096 x 16
 // heads beta 1 116 -> 123).  beta = -inf (every block exact), fewer than two
@@ -126,8 +125,11 @@ int64_t split_bytes(int64_t bh, int64_t q_sink_blocks, int64_t splits, int64_t h
 // for its local blocks, staging and cutoff.  us per call, 128-token sinks, not
 // split -> split, with the ratio: 4,096 x 16 heads x D128 beta 1 (3.3) 92 ->
 // 80, beta 0 (1.6) 108 -> 119; 2 x 4,096 x 16 beta 1 (1.6) 116 -> 123; 4,096 x
-// 24 (2.2) 101 -> 99; 6,000 x 16 (2.6) 126 -> 117; D64: 6,000 x 20 (3.1) 102
-// -> 91, 4,096 x 32 (2.4) 78 -> 77.
+// 24 (2.2) 101 -> 99; 6,000 x 16 (2.6) 126 -> 117; 20,000 x 4 beta 0.5 (2.3)
+// 401 -> 362; 8,192 x 16 beta 1 (2.0) 188 -> 170, beta 0.5 (1.3) 246 -> 239,
+// beta 0 (0.9) 348 -> 332, but x 14, 12, 9 beta 0 (1.0, 1.1, 1.5) 292 -> 298, 269 ->
+// 276, 219 -> 231 and 12,288 x 10 beta 0.5 (1.4) 304 -> 317; D64: 6,000 x 20
+// (3.1) 102 -> 91, 4,096 x 32 (2.4) 78 -> 77, 12,288 x 10 beta 0.5 (2.2) 204 -> 211.
 double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, double beta, int64_t head_dim) {
   const double slots = head_dim == 64 ? 1536 : 1024;
   const double share = sol::selected_share(0, beta);
@@ -140,9 +142,9 @@ double sink_chain_ratio(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blo
 int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int force, double beta,
                 int64_t head_dim, bool int8) {
   const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
-                          (force == 0 && sol::head_key_bytes(nkb, head_dim) <= kSplitKeyBytes && !(int8 && head_dim == 128) &&
-                           ((bh * nqb <= 2048 && nkb >= 128) ||
-                            sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2));
+                          (force == 0 && sol::head_key_bytes(nkb, head_dim) <= kSplitKeyBytes &&
+                           !(int8 && head_dim == 128) &&
+                           sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2);
   // Launches of the small kernel split every query block's chain inside its
   // workgroup instead.
   if (sol::small_key_split(bh * nqb, nkb, q_sink_blocks, head_dim)) return 1;

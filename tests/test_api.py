@@ -257,7 +257,9 @@ def test_split_workspace_only_where_sinks_set_the_launch_end():
     ((1, 4096, 4096, 16, 128, 1.0, 128), True),    # the sink chain is 3.3 times a slot's average steps
     ((1, 4096, 4096, 16, 128, 0.0, 128), False),   # 1.6 times
     ((2, 4096, 4096, 16, 64, 1.0, 128), True),     # six workgroups per CU at head_dim 64: 2.4
-    ((1, 8192, 8192, 16, 128, 0.0, 128), True),    # at most 2,048 query blocks over at least 128 key blocks
+    ((1, 8192, 8192, 16, 128, 1.0, 128), True),    # 2.01 times
+    ((1, 8192, 8192, 16, 128, 0.0, 128), False),   # 0.86 times: no size is split for itself
+    ((1, 8192, 8192, 12, 128, 0.0, 128), False), ((1, 12288, 12288, 10, 128, 0.0, 128), False),
     ((1, 8192, 8192, 24, 128, 1.0, 128), False),   # 1.4 times
     ((1, 4096, 1984, 16, 128, 1.0, 128), False),   # 31 key blocks: one part
 ])
