@@ -304,7 +304,8 @@ def _pairs(b, nq, nk, h, d, beta, int8, windows):
 
 def _windows(b, nq, nk, h, d, beta, int8):
     """Whether an indexed launch reads key blocks of consecutive rows from K
-    and V (sol_pool_windows), which the one-block form does."""
+    and V (sol_pool_windows), which the one-block form does.  (A debug launch
+    hands out every block's tiles instead.)"""
     return _one_block_keys(nk, d) and (WORKGROUP_FORM == 1 or (
         WORKGROUP_FORM == 0 and _one_block(b, nq, nk, h, d, beta, int8, True)))
 
@@ -625,7 +626,7 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
     try:
         pooled = pool_kv(k, v, key_index=keys, moments=not math.isinf(beta), key_lengths=key_lengths,
                          stream=stream, views=debug, qk_int8=int8,
-                         windows=keys is not None and _windows(b, nq, nk, *q.shape[-2:], beta, int8))
+                         windows=keys is not None and not debug and _windows(b, nq, nk, *q.shape[-2:], beta, int8))
         if threshold_estimator == "full_covariance" and not math.isinf(beta):
             key_covariance(pooled, stream)
     finally:

@@ -136,3 +136,15 @@ def test_block_rows(d, h, copies):
     copied = torch.from_numpy(want < 0).cuda()
     for b in range(w):
         assert torch.equal(out["tiles"][b, :, copied[b]], full["tiles"][b, :, copied[b]])
+
+
+@pytest.mark.parametrize("kind", ["runs", "joined"])
+def test_debug_launches_of_windows_hand_out_every_tile(kind):
+    n, h, d = 1600, 2, 64
+    gen = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn((n, h, d), generator=gen).to(torch.bfloat16).cuda() for _ in range(3))
+    rows, keys = (x.cuda() for x in _windows(kind, n))
+    out, _, dbg = _native.launch_sol(q, k, v, d ** -0.5, 1.0, -1, 0, 0, False, rows=rows, keys=keys, debug=True)
+    assert torch.equal(dbg["tiles"], _native.pool_kv(k, v, key_index=keys)["tiles"])
+    plain, _ = _native.launch_sol(q, k, v, d ** -0.5, 1.0, -1, 0, 0, False, rows=rows, keys=keys)
+    assert torch.equal(out, plain)
