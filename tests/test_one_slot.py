@@ -108,6 +108,81 @@ def test_windows_from_rows_equal_windows_from_tiles(d, h, kind, small, monkeypat
             assert torch.equal(got, sol_attention_indexed(q, k, v, plan, beta=beta))
 
 
+CLASSES = 20
+
+
+def _peaked(t, h, d, seed):
+    """Q, K, V [t, h, d]: query i scores about 40 log2 units more against the
+    keys of every 20th run of 32 than against the others.  So the max of some
+    query of every wave jumps in nearly every half tile, and that half's scores are
+    what its output is made of."""
+    gen = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn((t, h, d), generator=gen) for _ in range(3))
+    peak = (40 * d ** 0.5 / math.log2(math.e)) ** 0.5
+    i = torch.arange(t)
+    q[i, :, i % CLASSES] += peak
+    k[i, :, i // 32 % CLASSES] += peak
+    return tuple(x.to(torch.bfloat16).cuda() for x in (q, k, v))
+
+
+def _check_dense64(got, q, k, v, groups):
+    """got [nq, h, d] against dense attention in 64 bits.  P and the output are
+    rounded to BF16 (8 significant bits: by at most 2^-8 each, of at most sum
+    p |v|), exponents and sums to FP32 (2^-11 together, generously).  Also that
+    every key-split group meets half tiles whose row sum exceeds the lazy
+    softmax's bound after the group's first tile."""
+    d = q.shape[-1]
+    for h in range(q.shape[1]):
+        s = q[:, h].double() @ k[:, h].double().t().contiguous() * d ** -0.5
+        p = torch.softmax(s, 1)
+        vh = v[:, h].double()
+        bound = (2 ** -7 + 2 ** -11) * (p @ vh.abs())
+        err = (got[:, h].double() - p @ vh).abs()
+        assert bool((err <= bound).all()), f"head {h}: {float((err / bound).max()):.2f} times the bound"
+        if h == 0:
+            s = s[:32] * math.log2(math.e)   # one wave's queries
+            for g in range(groups):
+                own = [t for j in range(g, -(-s.shape[1] // 64), groups) for t in (s[:, 64 * j:64 * j + 32],
+                                                                                  s[:, 64 * j + 32:64 * j + 64])]
+                m, jumps = torch.cat(own[:2], 1).amax(1), 0
+                for half in own[2:]:
+                    if half.shape[1] == 0:
+                        continue
+                    jumps += bool((torch.exp2(half - m[:, None]).sum(1) > 65535).any())
+                    m = torch.maximum(m, half.amax(1))
+                assert jumps >= 2 or len(own) < 8, f"group {g}: {jumps} jumps"
+
+
+@pytest.mark.parametrize("d,h", [(64, 3), (128, 2), (64, 33), (128, 33)])   # four groups; two
+@pytest.mark.parametrize("kind", ["runs", "joined", "sparse", "ragged"])
+@pytest.mark.parametrize("form", [0, 1])
+def test_jumping_scores_of_windows_equal_dense(d, h, kind, form, monkeypatch):
+    print(f"jumping scores: D{d} H{h} {kind} form {form}", flush=True)
+    n = 1600
+    q, k, v = _peaked(n, h, d, seed=8)
+    rows, keys = _windows(kind, n)
+    plan = IndexedPlan.create(rows, keys, n, protected_ranges=((0, n),), local_tokens=0).to("cuda")
+    monkeypatch.setattr(_native, "WORKGROUP_FORM", form)
+    groups = 1 if form else (4 if 2 * 4 * h <= 256 else 2)
+    for beta in (1.0, math.inf) if form == 0 else (1.0, -math.inf):
+        got = sol_attention_indexed(q, k, v, plan, beta=beta)
+        for w in range(2):
+            kw = keys[w].cuda()
+            _check_dense64(got[w], q[rows[w].cuda()], k[kw], v[kw], groups)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("tk", [700, 2304, 4133])
+@pytest.mark.parametrize("h", [2, 90])   # four groups; two
+def test_jumping_scores_of_plain_keys_equal_dense(d, tk, h, monkeypatch):
+    print(f"jumping scores: D{d} Tk{tk} H{h}", flush=True)
+    q, k, v = _peaked(tk, h, d, seed=9)
+    q = q[:150].contiguous()
+    for form in (0, 1):
+        got, _ = _launch(q[None], k[None], v[None], form, monkeypatch, 1.0, local=1 << 30)
+        _check_dense64(got[0], q, k, v, 1 if form else (4 if 3 * h <= 256 else 2))
+
+
 @pytest.mark.parametrize("d,h,copies", [(64, 2, 1), (128, 4, 1), (128, 4, 160)])
 def test_block_rows(d, h, copies):
     # copies: enough windows for the four-head pooling kernel.

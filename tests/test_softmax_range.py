@@ -1,6 +1,6 @@
 """Softmax states at the ends of their range: every form of the attention
-kernels on scores far below 0, on a running max that jumps by more than FP32's
-exponents, and on values whose sums come near the FP32 range.
+kernels on scores far below 0 and on a first half whose 2^score is 0 in FP32
+while the second's is not.
 
 Queries are one constant and every key block one score level, so that a block
 equals its centroid and 64-bit dense attention is the result of every form at
@@ -41,7 +41,7 @@ def _close(got, want, what):
     got = got.double().cpu()
     finite = bool(torch.isfinite(got).all())
     assert finite, f"{what}: not finite"
-    # BF16 probabilities and outputs, rounded by at most 2^-9 each: 2^-8 together, and FP32 sums far below.
+    # BF16 probabilities and outputs, rounded by at most 2^-8 each and 2^-9 on average, and FP32 sums far below.
     rel = ((got - want).norm() / want.norm()).item()
     assert rel < 2 ** -8, f"{what}: relative error {rel:.4f}"
 
