@@ -1687,7 +1687,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
     den = den + w[g] * s_md[g][qh][1][lane];
   }
   den = pair_sum(den);
-  const float inv = __fdiv_rn(1.f, den);  // one division per row, as store_output
+  const float inv = __fdiv_rn(1.f, den);
   if (p.counts && tid == 0) p.counts[(int64_t(b) * p.NQB + qb) * p.H + h] = nsel;
   const int t = qb * kBlock + myq;
   if (t >= p.Tq) return;
@@ -1707,8 +1707,8 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
       for (int i = 0; i < 4; ++i) o[i] = o[i] + w[g] * x[i];
     }
     u32x2 v;
-    v[0] = pack_bf16x2(o[0] * inv, o[1] * inv);
-    v[1] = pack_bf16x2(o[2] * inv, o[3] * inv);
+    v[0] = pack_bf16x2(quotient(o[0], den, inv), quotient(o[1], den, inv));
+    v[1] = pack_bf16x2(quotient(o[2], den, inv), quotient(o[3], den, inv));
     *reinterpret_cast<u32x2*>(orow + (c / 4) * 32 + 8 * (c % 4) + 4 * hh) = v;
   }
 }

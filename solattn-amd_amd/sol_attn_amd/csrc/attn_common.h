@@ -622,6 +622,15 @@ struct FragLane {
 // interleave of matrix-core, LDS, DMA and VALU work below is kept.
 __device__ __forceinline__ void chunk_end() { __builtin_amdgcn_sched_barrier(0); }
 
+// x / den in FP32, correctly rounded, from inv = fl(1 / den): the product, its
+// remainder (exact in one fused step) added back, infinities and NaN as a
+// division gives them.  64 divisions per lane were 3,800 cycles of a workgroup,
+// 4% at 4,096 tokens; the product alone is up to one more rounding off.
+__device__ __forceinline__ float quotient(float x, float den, float inv) {
+  const float q = x * inv;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, den, x), inv, q), den, x);
+}
+
 template <int D>
 __device__ __forceinline__ void store_output(const AttnParams& p, int b, int h, int t, int hh,
                                              const State<D>& st) {
@@ -634,17 +643,14 @@ __device__ __forceinline__ void store_output(const AttnParams& p, int b, int h, 
     if (row < 0 || row >= p.out_rows) return;  // outside the output: not stored
   }
   uint16_t* orow = p.out + (row * p.H + h) * D;
-  // One division per query: 64 IEEE divisions per lane were 3,800 cycles of a
-  // workgroup, 4% at 4,096 tokens; the FP32 product differs from the quotient
-  // by at most 1 part in 2^23, before the rounding to BF16 (1 in 2^9).
   const float inv = __fdiv_rn(1.f, den);
 #pragma unroll
   for (int dt = 0; dt < S::DT; ++dt)
 #pragma unroll
     for (int k4 = 0; k4 < 4; ++k4) {
       u32x2 o;
-      o[0] = pack_bf16x2(st.acc[dt][4 * k4] * inv, st.acc[dt][4 * k4 + 1] * inv);
-      o[1] = pack_bf16x2(st.acc[dt][4 * k4 + 2] * inv, st.acc[dt][4 * k4 + 3] * inv);
+      o[0] = pack_bf16x2(quotient(st.acc[dt][4 * k4], den, inv), quotient(st.acc[dt][4 * k4 + 1], den, inv));
+      o[1] = pack_bf16x2(quotient(st.acc[dt][4 * k4 + 2], den, inv), quotient(st.acc[dt][4 * k4 + 3], den, inv));
       *reinterpret_cast<u32x2*>(orow + dt * 32 + 8 * k4 + 4 * hh) = o;
     }
 }

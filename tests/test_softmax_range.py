@@ -89,3 +89,37 @@ def test_first_half_below_the_fp32_range(d, monkeypatch):
     print(f"first half: D{d}", flush=True)
     levels = [-130.0 if t < 32 else -124.0 for t in range(64)] + [-130.0] * 64
     _all_forms(monkeypatch, levels, d, block_levels=False)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [3, 7, 14, 28, 56, 63])
+def test_outputs_are_rounded_quotients(n, d, monkeypatch):
+    # n equal keys whose values sum to n times a tie between two BF16 numbers: FP32 holds the sum and the quotient,
+    # so the output is the tie rounded to even.  (The sum times FP32's 1 / n rounds the other way for
+    # some ties at every n here but 3.)
+    print(f"quotients: Tk{n} D{d}", flush=True)
+    ties = (257 + 2 * torch.arange(d, dtype=torch.float64) % 254) / 256.0
+    total = n * ties
+    v = torch.zeros((1, n, 1, d), dtype=torch.float64)
+    for t in range(3):  # 9 bits times n: two or three BF16 terms
+        v[0, t, 0] = total.float().to(torch.bfloat16).double()
+        total = total - v[0, t, 0]
+    assert not total.any()
+    v = v.to(torch.bfloat16).cuda()
+    k = torch.ones((1, n, 1, d), dtype=torch.bfloat16, device="cuda")
+    q = torch.zeros((1, 70, 1, d), dtype=torch.bfloat16, device="cuda")
+    want = ties.float().to(torch.bfloat16).expand(1, 70, 1, d)   # round to nearest, ties to even
+    for got in (dense_attention(q, k, v), sol_attention(q, k, v), _form(monkeypatch, 1, q, k, v, 1.0)):
+        assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_infinite_values_stay_infinite(d):
+    print(f"infinite values: D{d}", flush=True)
+    q, k, v = (torch.randn((1, 100, 2, d), generator=torch.Generator().manual_seed(s)).to(torch.bfloat16)
+               for s in (4, 5, 6))
+    v[0, 3, 0, 5], v[0, 80, 1, 7] = math.inf, -math.inf
+    got = dense_attention(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    assert (got[0, :, 0, 5] == math.inf).all() and (got[0, :, 1, 7] == -math.inf).all()
+    got[0, :, 0, 5] = got[0, :, 1, 7] = 0.0
+    assert torch.isfinite(got).all()
