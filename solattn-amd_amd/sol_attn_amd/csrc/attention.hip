@@ -139,10 +139,12 @@ __device__ __forceinline__ void landed_barrier() {
 // only) is added once a half's products are done instead, which keeps it out
 // of the registers live across the score chain; the same values (x + 0 is x
 // for the nonzero-signed sums a chain from +0 gives, and -inf either way).
+// v_bits (SlotStep): 0 for a tile with every score at -inf, whose values then
+// count as 0: 0 times an infinite one would be NaN.
 template <int D, bool BIASED, typename Bias, typename Step, bool LATE = false, bool FULL = false>
 __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
                                             const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
-                                            Bias bias, const Step& step) {
+                                            Bias bias, const Step& step, uint32_t v_bits = ~0u) {
   constexpr bool EARLY = BIASED && !LATE;
   constexpr bool ONE = Step::kOneSlot;
   static_assert(ONE || !FULL, "a ring's tile stays in LDS");
@@ -209,9 +211,9 @@ __device__ __forceinline__ void tile_attend(State<D>& st, const uint16_t* buf,
 #pragma unroll
       for (int f = 2 * ks; f < 2 * ks + 2; ++f) {
         if (f < KT)
-          va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT);
+          va[f / DT][f % DT] = fl.v(vbase, 0, f / DT, f % DT) & v_bits;
         else
-          vb[(f - KT) / DT][f % DT] = fl.v(vbase, 1, (f - KT) / DT, f % DT);
+          vb[(f - KT) / DT][f % DT] = fl.v(vbase, 1, (f - KT) / DT, f % DT) & v_bits;
       }
     } else {
       if (ks >= KT / 2) {  // two of half 0's 2 DT = KT V^T fragments per chunk
@@ -291,7 +293,7 @@ __device__ __forceinline__ void tail_tile(State<D>& st, const uint16_t* buf, int
     }
     return bias;
   };
-  tile_attend<D, true, decltype(absent), Step, true, FULL>(st, buf, qf, col, hh, c, absent, step);
+  tile_attend<D, true, decltype(absent), Step, true, FULL>(st, buf, qf, col, hh, c, absent, step, any ? ~0u : 0u);
 }
 
 // Exact block j: a full block, or the partial last block.  Only a stream's
@@ -315,7 +317,8 @@ __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, in
 template <int D, bool FULL = false, typename Step>
 __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf, int ct, uint64_t approx,
                                               int tk, const bf16x8 (&qf)[Shape<D>::KT], int col, int hh,
-                                              float c, const Step& step, bool exact = false) {
+                                              float c, const Step& step, bool exact = false,
+                                              uint32_t v_bits = ~0u) {
   const float inv_c = 1.f / c;
   // Every block is whole but the sequence's last one: whole blocks share one
   // offset, log2(64) / c.  The approximated blocks are wave-uniform, so each
@@ -339,7 +342,7 @@ __device__ __forceinline__ void centroid_tile(State<D>& st, const uint16_t* buf,
     }
     return bias;
   };
-  tile_attend<D, true, decltype(lengths), Step, false, FULL>(st, buf, qf, col, hh, c, lengths, step);
+  tile_attend<D, true, decltype(lengths), Step, false, FULL>(st, buf, qf, col, hh, c, lengths, step, v_bits);
 }
 
 // The quantised-QK experiment's exact tile: S^T = K8 Q8^T on the INT8 matrix
@@ -1626,15 +1629,17 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
       }
       return ct < nct ? tile_approx(s_mask, ct, 0, nkb) : 0ull;
     };
+    auto attend = [&](int ct, uint64_t approx, const auto& step, bool exact) {
+      centroid_tile<D, true>(st, slot, ct, approx, tk, qf, col, hh, scale_log2, step, exact,
+                             __builtin_amdgcn_readfirstlane(exact || approx != 0ull ? ~0u : 0u));
+    };
     int ct = grp;
     for (; ct - grp + KS < nct; ct += KS)
-      centroid_tile<D, true>(st, slot, ct, approximated(ct), tk, qf, col, hh, scale_log2,
-                             slot_step<D>(crefill(min(ct + KS, nct - 1), slot_lds), NoFrag{}, k, slot));
+      attend(ct, approximated(ct), slot_step<D>(crefill(min(ct + KS, nct - 1), slot_lds), NoFrag{}, k, slot), false);
     const uint64_t approx = approximated(ct);
     const int steps = (cursor.all.count() + KS - 1) / KS;
     const int id = cursor();
-    centroid_tile<D, true>(st, slot, min(ct, nct - 1), approx, tk, qf, col, hh, scale_log2,
-                           slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot), early);
+    attend(min(ct, nct - 1), approx, slot_step<D>(make(id, slot_lds), NoFrag{}, k, slot), early);
     // 4. Exact pass: group grp's share of the other selected blocks, ascending.
     const auto kfrag = k_fragments<D, KT>(p, b, h, col, hh);
     slot_stream(
@@ -1646,7 +1651,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
           full_tile<D>(st, slot, qf, col, hh, scale_log2, slot_step<D>(refill, kfrag(tag >> 1), k, slot));
         },
         [&](int tag, const auto& refill) {
-          tail_tile<D, !KT, true>(st, slot, tag >> 1, tk, (tag & 1) != 0, qf, col, hh, scale_log2,
+          tail_tile<D, !KT, true>(st, slot, tag >> 1, tk, __builtin_amdgcn_readfirstlane(tag & 1) != 0, qf, col, hh, scale_log2,
                                   slot_step<D>(refill, NoFrag{}, k, slot));
         });
   }

@@ -114,12 +114,17 @@ def test_outputs_are_rounded_quotients(n, d, monkeypatch):
 
 
 @pytest.mark.parametrize("d", [64, 128])
-def test_infinite_values_stay_infinite(d):
-    print(f"infinite values: D{d}", flush=True)
-    q, k, v = (torch.randn((1, 100, 2, d), generator=torch.Generator().manual_seed(s)).to(torch.bfloat16)
-               for s in (4, 5, 6))
-    v[0, 3, 0, 5], v[0, 80, 1, 7] = math.inf, -math.inf
-    got = dense_attention(q.cuda(), k.cuda(), v.cuda()).float().cpu()
-    assert (got[0, :, 0, 5] == math.inf).all() and (got[0, :, 1, 7] == -math.inf).all()
-    got[0, :, 0, 5] = got[0, :, 1, 7] = 0.0
-    assert torch.isfinite(got).all()
+@pytest.mark.parametrize("tk,heads", [(100, 2), (700, 2), (2304, 2), (2304, 150)])   # four groups; two
+def test_infinite_values_stay_infinite(d, tk, heads):
+    # Every block exact: one infinite value per head, in the first block (which groups that have run out of tiles
+    # pass through again) and in the last.
+    print(f"infinite values: D{d} Tk{tk} H{heads}", flush=True)
+    q, k, v = (torch.randn((1, t, heads, d), generator=torch.Generator().manual_seed(s)).to(torch.bfloat16)
+               for t, s in ((100, 4), (tk, 5), (tk, 6)))
+    v[0, 3, ::2, 5], v[0, tk - 20, 1::2, 7] = math.inf, -math.inf
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    for got in (dense_attention(q, k, v), sol_attention(q, k, v, local_blocks=1 << 20)):
+        got = got.float().cpu()
+        assert (got[0, :, ::2, 5] == math.inf).all() and (got[0, :, 1::2, 7] == -math.inf).all()
+        got[0, :, ::2, 5] = got[0, :, 1::2, 7] = 0.0
+        assert torch.isfinite(got).all()
