@@ -77,12 +77,14 @@ def library():
                 f"SOL HIP library not built ({LIB_PATH} missing); "
                 "run `python -m sol_attn_amd._build` or __graft_entry__.build()")
         lib = ctypes.CDLL(LIB_PATH)
+        missing = [name for name in _SIGNATURES if not hasattr(lib, name)]
+        if missing or lib.sol_abi_version() != ABI_VERSION:
+            raise RuntimeError("libsol_attn_amd.so ABI version mismatch; rebuild it"
+                               + (f" (no {', '.join(missing)})" if missing else ""))
         for name, (args, res) in _SIGNATURES.items():
             fn = getattr(lib, name)
             fn.argtypes = args
             fn.restype = res
-        if lib.sol_abi_version() != ABI_VERSION:
-            raise RuntimeError("libsol_attn_amd.so ABI version mismatch; rebuild it")
         _lib = lib
     return _lib
 

@@ -4,6 +4,8 @@ import ctypes
 import math
 import os
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -156,6 +158,18 @@ def test_c_abi_library_exports_every_declared_symbol():
     assert native.sol_pair_workspace_size(1, 193, 2, 64) == 2 * 64 * (4 + 256) * 4
     assert native.sol_pair_workspace_size(1, 192, 2, 64) == 0
     assert native.sol_pair_workspace_size(1, 193, 2, 96) == 0
+
+
+def test_a_library_without_every_function_is_to_be_rebuilt(tmp_path, monkeypatch):
+    # Functions were added within one ABI version: a library built before them has the version and not the functions.
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not installed")
+    (tmp_path / "old.cpp").write_text('extern "C" int sol_abi_version() { return %d; }' % _native.ABI_VERSION)
+    subprocess.run(["g++", "-shared", "-fPIC", str(tmp_path / "old.cpp"), "-o", str(tmp_path / "old.so")], check=True)
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(_native, "LIB_PATH", str(tmp_path / "old.so"))
+    with pytest.raises(RuntimeError, match="rebuild it .*sol_attention_windows"):
+        _native.library()
 
 
 def test_c_abi_rejects_bad_arguments_without_launching():
