@@ -494,7 +494,8 @@ __device__ __forceinline__ auto kv_refills(const AttnParams& p, int b, int h, in
     const uint16_t* tiles = p.tiles + (int64_t(b) * p.H + h) * p.NKB * Shape<D>::TILE;
     if constexpr (WINDOWS) {
       const KvRows<D, NT> rows = kv_rows<D, NT>(p, b, h, wave * kWave + lane);
-      return [=, &p](int j, uint32_t lds) {
+      return [=, &p](int block, uint32_t lds) {
+        const int j = __builtin_amdgcn_readfirstlane(block);
         return WindowRefill<D, NT>(rows, tiles + int64_t(j) * Shape<D>::TILE, block_row(p, b, j), lds, wave, lane);
       };
     } else {
