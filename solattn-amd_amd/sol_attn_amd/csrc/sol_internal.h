@@ -208,10 +208,12 @@ inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_
 // hold up its group is kUnevenMax times the average.  A head costs at least 8
 // steps' time and its centroid tiles per query block, at most half the key
 // blocks more (the threshold is at least the mean); one such head among a
-// group's P and the launch's `heads`.  Over 72 inputs -- one dense head, a
+// group's P and the launch's `heads`.  Over 140 inputs -- one dense head, a
 // quarter, every fourth, random densities; 4,096 to 24,576 tokens, 8 to 32 heads
-// -- the launches took 0.61 to 0.99 of the two-block form's time there.
-constexpr double kUnevenMax = 1.7;
+// -- the launches took 0.61 to 1.05 of the two-block form's time there (1.05: one
+// dense head of 24 at 10,000 tokens and beta 2).  At 1.7 that call took 0.87, and 4,096
+// queries x 10,000 keys x 24 heads 182 instead of 164 us.
+constexpr double kUnevenMax = 1.75;
 inline int xcds_per_head(int64_t heads, int64_t nkb) {
   const double base = 8.0 + double(nkb) / kBlock, more = 0.5 * double(nkb) / base;
   for (int xcds = 1; xcds <= 4; xcds *= 2) {
