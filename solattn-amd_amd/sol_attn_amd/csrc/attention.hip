@@ -298,14 +298,14 @@ __device__ __forceinline__ void tail_tile(State<D>& st, const uint16_t* buf, int
 
 // Exact block j: a full block, or the partial last block.  Only a stream's
 // last exact tile can be that block.
-template <int D, bool SHIFTED, bool FULL = false, typename Step>
+template <int D, bool SHIFTED, typename Step>
 __device__ __forceinline__ void exact_tile(State<D>& st, const uint16_t* buf, int j, int tk,
                                            const bf16x8 (&qf)[Shape<D>::KT], int col, int hh, float c,
                                            const Step& step) {
   if ((j + 1) * kBlock <= tk) {
-    full_tile<D, FULL>(st, buf, qf, col, hh, c, step);
+    full_tile<D>(st, buf, qf, col, hh, c, step);
   } else {
-    tail_tile<D, SHIFTED, FULL>(st, buf, j, tk, true, qf, col, hh, c, step);
+    tail_tile<D, SHIFTED>(st, buf, j, tk, true, qf, col, hh, c, step);
   }
 }
 

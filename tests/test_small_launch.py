@@ -27,7 +27,7 @@ pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not HAS_GPU, reason="AMD ROCm 
 
 # (batch, query tokens, key tokens, heads, head_dim, inputs, query sink tokens)
 CASES = [(1, 1024, 1024, 8, 64, "smooth", 128),    # one launch, keys pooled inside (the 1,024-token case)
-         (1, 1024, 1024, 4, 128, "smooth", 128),   # D = 128, two key-split groups, pooling kernel first
+         (1, 1024, 1024, 4, 128, "smooth", 128),   # D = 128, pooling kernel first
          (2, 700, 1000, 3, 64, "random", 64),      # tails, 16 blocks pooled inside, two entries
          (1, 1500, 2000, 2, 128, "random", 128),   # 32 key blocks: centroid tiles from the pooling kernel
          (1, 600, 4000, 2, 64, "smooth", 0),       # 63 key blocks, 4 groups

@@ -87,7 +87,7 @@ def test_noalloc_leaves_sink_tiles_whole_where_their_split_does_not_fit():
 _FIRST_CALL = r"""
 import ctypes
 import torch
-from sol_attn_amd import _native, sol_attention
+from sol_attn_amd import _native
 from sol_testlib import block_smooth
 b, tq, tk, h, d = 1, 4096, 4096, 4, 128
 q = block_smooth(b, tq, h, d, seed=41, device="cuda")
