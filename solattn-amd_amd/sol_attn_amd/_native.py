@@ -217,7 +217,8 @@ def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, v
     sizes += [b * h * -(-nkb // 16) * 2 * d * 4, b * h * d * 4, b * h * d * 4] if moments else [0, 0, 0]
     if qk_int8:
         sizes += [b * h * nkb * BLOCK * d, b * h * nkb * 4]
-    windows = windows and indexed and max(k.stride(-3), v.stride(-3)) < (1 << 24)
+    ks, vs = _strides(k, indexed), _strides(v, indexed)
+    windows = windows and indexed and ks[1] < (1 << 24) and vs[1] < (1 << 24)
     if windows:
         sizes.append(b * nkb * 4)
     offsets, total = _carve(tuple(sizes))
@@ -226,7 +227,7 @@ def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, v
     ctiles, tiles = base + offsets[0], None if rows else base + offsets[1]
     sums, mean, var = (base + o for o in offsets[2:5]) if moments else (None, None, None)
     block_rows = base + offsets[-1] if windows else None
-    args = (k.data_ptr(), _strides(k, indexed), v.data_ptr(), _strides(v, indexed),
+    args = (k.data_ptr(), ks, v.data_ptr(), vs,
             _ptr(key_index), _ptr(key_lengths), k.shape[0] if indexed else 0,
             b, tk, h, d, ctiles, tiles, sums, mean, var)
     _check(lib.sol_pool_windows(*args, block_rows, stream) if windows else lib.sol_pool_kv(*args, stream))
@@ -234,7 +235,8 @@ def pool_kv(k, v, key_index=None, moments=True, key_lengths=None, stream=None, v
               "mean_ptr": mean, "var_ptr": var, "cov_ptr": None, "key_tokens": tk,
               "key_blocks": nkb, "key_lengths": key_lengths, "k8_ptr": None, "k8_scale_ptr": None,
               "block_rows_ptr": block_rows,
-              "k": k if rows or windows else None, "v": v if rows or windows else None}
+              "k": k if rows or windows else None, "v": v if rows or windows else None,
+              "k_strides": ks if rows or windows else None, "v_strides": vs if rows or windows else None}
     if qk_int8:
         k8, k8s = base + offsets[5], base + offsets[6]
         _check(lib.sol_quantize_keys(k.data_ptr(), _strides(k, indexed), _ptr(key_index), _ptr(key_lengths),
@@ -289,6 +291,7 @@ def _one_block(b, nq, nk, h, d, beta, int8, windows):
     return bool(library().sol_attention_one_block(b, nq, nk, h, d, beta, int8, windows))
 
 
+@functools.lru_cache(maxsize=256)
 def _one_block_keys(nk, d):
     """Key sequences whose launches may hold one query block per workgroup
     however many query blocks there are."""
@@ -308,8 +311,9 @@ def _windows(b, nq, nk, h, d, beta, int8):
     """Whether an indexed launch reads key blocks of consecutive rows from K
     and V (sol_pool_windows), which the one-block form does.  (A debug launch
     hands out every block's tiles instead.)"""
-    return _one_block_keys(nk, d) and (WORKGROUP_FORM == 1 or (
-        WORKGROUP_FORM == 0 and _one_block(b, nq, nk, h, d, beta, int8, True)))
+    if WORKGROUP_FORM == 2 or not _one_block_keys(nk, d):
+        return False
+    return WORKGROUP_FORM == 1 or _one_block(b, nq, nk, h, d, beta, int8, True)
 
 
 def _pair_buffers(q, rows, min_blocks):
@@ -497,8 +501,7 @@ def attend(q, pooled, scale, beta, local, kv_sink, q_sink, protection=None, rows
     _check((lib.sol_attention_windows if gathered else lib.sol_attention_fwd)(
         q.data_ptr(), _strides(q, indexed), _ptr(rows), q.shape[0] if indexed else 0,
         b, nq, nk, _ptr(pooled["key_lengths"]), h, d,
-        _ptr(kr), None if kr is None else _strides(kr, gathered), _ptr(vr),
-        None if vr is None else _strides(vr, gathered), *((block_rows,) if gathered else ()),
+        _ptr(kr), pooled["k_strides"], _ptr(vr), pooled["v_strides"], *((block_rows,) if gathered else ()),
         pooled["tiles_ptr"], pooled["ctiles_ptr"], pooled["mean_ptr"], pooled["var_ptr"], pooled["cov_ptr"],
         _ptr(prot), _ptr(strides), _ptr(split), _ptr(route), _ptr(query_means), float(scale), float(beta),
         int(local), int(kv_sink), int(q_sink),
@@ -558,7 +561,7 @@ def _self_pooled(k, v):
             "mean_ptr": None, "var_ptr": None, "cov_ptr": None, "key_tokens": nk,
             "key_blocks": -(-nk // BLOCK), "key_lengths": None, "k8_ptr": None, "k8_scale_ptr": None,
             "block_rows_ptr": None,
-            "k": k, "v": v}
+            "k": k, "v": v, "k_strides": _strides(k), "v_strides": _strides(v)}
 
 
 def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=None,
@@ -595,9 +598,11 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
              and ROUTE_PREPASS != "always")
     b, nq = rows.shape if rows is not None else q.shape[:2]
     nk = keys.shape[1] if keys is not None else k.shape[1]
+    h, d = q.shape[-2:]
     int8 = qk_precision == "int8"
     beta = float(beta)
-    pairs = _pairs(b, nq, nk, *q.shape[-2:], beta, int8, keys is not None)
+    pairs = (PAIRING and b * h * -(-nq // BLOCK) >= PAIR_MIN_QUERY_BLOCKS
+             and _pairs(b, nq, nk, h, d, beta, int8, keys is not None))
     if ALL_IN and plain and protection is None and out is None and SELF_POOLING and SPLIT_SINKS and not pairs:
         # No pairing pass: pooling and attention in one C-ABI call.
         return _all_in(q, k, v, float(scale), float(beta), int(local), int(kv_sink), int(q_sink), stats)
@@ -628,7 +633,7 @@ def launch_sol(q, k, v, scale, beta, local, kv_sink, q_sink, stats, protection=N
     try:
         pooled = pool_kv(k, v, key_index=keys, moments=not math.isinf(beta), key_lengths=key_lengths,
                          stream=stream, views=debug, qk_int8=int8,
-                         windows=keys is not None and not debug and _windows(b, nq, nk, *q.shape[-2:], beta, int8))
+                         windows=keys is not None and not debug and _windows(b, nq, nk, h, d, beta, int8))
         if threshold_estimator == "full_covariance" and not math.isinf(beta):
             key_covariance(pooled, stream)
     finally:

@@ -18,7 +18,8 @@ import math
 
 import torch
 
-from .attention import (SolStats, _key_length, _validate, _nonnegative_integer, _qk_precision,
+from . import _native
+from .attention import (SolStats, _key_length, _on, _validate, _nonnegative_integer, _qk_precision,
                         _threshold_estimator)
 
 BLOCK = 64
@@ -229,25 +230,24 @@ def sol_attention_indexed(q, k, v, plan, *, beta=1.0, scale=None, return_stats=F
         raise ValueError("beta must not be NaN")
     _threshold_estimator(threshold_estimator)
     _qk_precision(qk_precision)
-    from ._native import launch_dense, launch_sol
     if beta == -math.inf and qk_precision == "bf16" and plan.key_range is not None:
         # Every block exact over one contiguous key range: the dense kernel on
         # those K / V rows, queries gathered and (with out=) results scattered
         # inside it -- no pooling pass, no block tiles, no protection needed.
         start, count = plan.key_range
-        with torch.no_grad(), torch.cuda.device(q.device):
-            result = launch_dense(q, k[start:start + count], v[start:start + count], scale,
-                                  rows=plan.rows, out=out)
+        with _on(q.device):
+            result = _native.launch_dense(q, k[start:start + count], v[start:start + count], scale,
+                                          rows=plan.rows, out=out)
         if return_stats:
             nkb = (plan.keys.shape[1] + 63) // 64
             counts = torch.full((b, (nq + 63) // 64, q.shape[1]), nkb, device=q.device, dtype=torch.int32)
             return result, SolStats(counts, nkb)
         return result
-    with torch.no_grad(), torch.cuda.device(q.device):
-        result, counts = launch_sol(q, k, v, scale, beta, -1, 0, 0, return_stats,
-                                    plan.protected_blocks, rows=plan.rows, keys=plan.keys,
-                                    key_lengths=lengths, out=out,
-                                    threshold_estimator=threshold_estimator, qk_precision=qk_precision)
+    with _on(q.device):
+        result, counts = _native.launch_sol(q, k, v, scale, beta, -1, 0, 0, return_stats,
+                                            plan.protected_blocks, rows=plan.rows, keys=plan.keys,
+                                            key_lengths=lengths, out=out,
+                                            threshold_estimator=threshold_estimator, qk_precision=qk_precision)
     if return_stats:
         key_blocks = ((plan.keys.shape[1] + 63) // 64 if lengths is None
                       else (lengths.to(torch.int64) + 63) // 64)
