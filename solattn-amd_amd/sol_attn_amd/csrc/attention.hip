@@ -769,6 +769,24 @@ __device__ __forceinline__ float cutoff_value(const AttnParams& p, float lin0, f
   return (lin0 + lin1) + p.beta * sqrtf(p.cov ? fmaxf(quad, 0.f) : quad);
 }
 
+// Full covariance: feature f's element of cov Qc, in feature order.  cov is
+// symmetric bit for bit, so the threads read it by column (coalesced), 16 loads
+// in flight (one at a time they were 6 of 63 us: 3 x 143 tokens x 3 heads).
+template <int D>
+__device__ __forceinline__ float covariance_column(const AttnParams& p, int64_t head, int f, const float* qm) {
+  const float* col = p.cov + head * D * D + f;
+  float sq = 0.f;
+#pragma unroll 1
+  for (int e0 = 0; e0 < D; e0 += 16) {
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = col[(e0 + i) * D];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sq = fmaf(x[i], qm[e0 + i], sq);
+  }
+  return sq;
+}
+
 // The FP32 query mean of one feature as an exact sum of three BF16 terms (hi,
 // mid, lo: 8 significant bits each) in the routing operand rows qb [4][QB]:
 // row k the k-th term, row 3 zero.
@@ -989,12 +1007,7 @@ __global__ __launch_bounds__(256, D == 64 && !Q8 && !SEG ? 3 : 2) void sol_atten
       split_query_mean<D>(s_qb[qg], lt, qm);
       a = qm * km.mu;
       if (p.cov) {
-        // Full covariance: this feature's term of Qc^T cov Qc.  cov is
-        // symmetric bit for bit, so thread lt reads column lt (coalesced).
-        const float* col = p.cov + int64_t(head) * D * D + lt;
-        float sq = 0.f;
-        for (int e = 0; e < D; ++e) sq = fmaf(col[e * D], s_qm[qg][e], sq);
-        g = qm * sq;
+        g = qm * covariance_column<D>(p, head, lt, s_qm[qg]);
       } else {
         g = qm * qm * km.var;
       }
@@ -1533,10 +1546,7 @@ __global__ __launch_bounds__(128 * KS, 2) void sol_small_kernel(AttnParams p) {
       }
       a = qm * mu;
       if (p.cov) {
-        const float* col = p.cov + int64_t(head) * D * D + tid;  // symmetric: column tid
-        float sq = 0.f;
-        for (int e = 0; e < D; ++e) sq = fmaf(col[e * D], s_qm[e], sq);
-        g = qm * sq;
+        g = qm * covariance_column<D>(p, head, tid, s_qm);
       } else {
         g = qm * qm * (POOL ? s_mom[1][tid] : km.var);
       }
