@@ -155,8 +155,8 @@ int sol_key_covariance(const void* ctiles, const float* key_mean, const int32_t*
  * end: at fewer than 512 query-block pairs over all (entry, head) pairs; at
  * beta = +INFINITY up to 8,192 query blocks; at finite beta and at most 16 MB
  * of K and V per head when the chain is at least twice the steps a workgroup
- * slot has on average (launches with INT8 key tiles at head_dim 128 are not
- * split for that, whatever the workspace).  They split the key blocks of sink blocks [0, 2 floor(sink blocks / 2))
+ * slot has on average (launches with INT8 key tiles are not split for that,
+ * whatever the workspace).  They split the key blocks of sink blocks [0, 2 floor(sink blocks / 2))
  * over up to 8 workgroups each (parts of at least 16 blocks); a merge kernel
  * combines their partial softmax states.  Split launches pair adjacent query
  * blocks (pair_strides is ignored).

@@ -143,8 +143,7 @@ int sink_splits(int64_t bh, int64_t nqb, int64_t nkb, int64_t q_sink_blocks, int
                 int64_t head_dim, bool int8) {
   const bool few_groups = bh * ((nqb + 1) / 2) < sol::kSmallLaunchGroups ||
                           (force == 0 && sol::head_key_bytes(nkb, head_dim) <= kSplitKeyBytes &&
-                           !(int8 && head_dim == 128) &&
-                           sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2);
+                           !int8 && sink_chain_ratio(bh, nqb, nkb, q_sink_blocks, beta, head_dim) >= 2);
   // Launches of the small kernel split every query block's chain inside its
   // workgroup instead.
   if (sol::small_key_split(bh * nqb, nkb, q_sink_blocks, head_dim)) return 1;

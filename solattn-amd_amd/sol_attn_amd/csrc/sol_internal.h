@@ -182,9 +182,10 @@ inline double selected_share(int force, double beta) {
 // INT8 scores (the experiment) have no one-slot form: at head_dim 128 a
 // one-block workgroup holds a 64 KB ring too, so a CU has half the waves of the
 // two-block form.  us per call, one block -> two: 2 x 4,096 x 16 heads beta 1
-// 155 -> 130, beta 0 269 -> 207; 16,384 x 8 367 -> 307; 32,768 x 16 2417 ->
-// 2052; 21 x 4,032 windows x 24 10258 -> 8587.  (At 64 the ring is 32 KB: 2 x
-// 4,096 x 16 93 -> 83 the other way round.)
+// 155 -> 132, beta 0 269 -> 208; 16,384 x 8 367 -> 315; 32,768 x 16 2417 ->
+// 2058; 21 x 4,032 windows x 24 10258 -> 9304.  At 64, where the ring is 32 KB, it
+// is one way or the other: 2 x 4,096 x 16 beta 1 83 -> 93, beta -inf 215 -> 175;
+// 2 x 1,823 windows x 32 beta +inf 145 -> 138.
 constexpr int64_t kOneBlockKeyBytes = int64_t(12) << 20;
 constexpr double kOneBlockSelectedBytes = 5 << 20;
 constexpr int64_t kSmallLaunchGroups = 512;
@@ -192,7 +193,7 @@ inline bool one_block_launch(int64_t bh, int64_t nqb, int64_t nkb, int64_t head_
                              bool windows) {
   if (bh * ((nqb + 1) / 2) < kSmallLaunchGroups) return true;
   const int64_t bytes = head_key_bytes(nkb, head_dim);
-  if (bytes > kOneBlockKeyBytes || (int8 && head_dim == 128)) return false;
+  if (bytes > kOneBlockKeyBytes || int8) return false;
   if (windows) return share <= 0.7 || nkb <= 192;
   return share <= 0.5 && 2 * share * double(nkb) <= double(nqb) && share * double(bytes) <= kOneBlockSelectedBytes;
 }

@@ -14,10 +14,10 @@ pytestmark = pytest.mark.skipif(not os.path.exists(_native.LIB_PATH), reason="li
 
 
 @pytest.mark.parametrize("b,nq,nk,h,d,int8,one", [
-    # INT8 scores at head_dim 128 have a two-slot ring in either form: two blocks, as half the waves fit otherwise.
+    # INT8 scores have a two-slot ring in either form: two blocks, as half the waves fit otherwise.
     (2, 4096, 4096, 16, 128, False, True), (2, 4096, 4096, 16, 128, True, False),
     (1, 16384, 16384, 8, 128, True, False),
-    (2, 4096, 4096, 16, 64, True, True),
+    (2, 4096, 4096, 16, 64, True, False),
     (1, 4096, 4096, 4, 128, True, True),       # 128 pairs: two blocks would leave CUs idle
 ])
 def test_int8_launches(b, nq, nk, h, d, int8, one):
@@ -28,6 +28,8 @@ def test_int8_launches_pair_their_query_blocks():
     # 8,192 query blocks and more.
     assert _native._pairs(1, 32768, 24000, 24, 128, 1.0, True, False)
     assert not _native._windows(21, 4032, 8064, 24, 128, 1.0, True)
+    assert not _native._windows(2, 1823, 3646, 32, 64, 1.0, True) and _native._windows(2, 1823, 3646, 32, 64, 1.0, False)
+    assert _native._windows(8, 1000, 4000, 2, 64, 1.0, True)   # fewer than 512 pairs
 
 
 @pytest.mark.parametrize("b,nq,nk,h,d,beta,windows,one", [
