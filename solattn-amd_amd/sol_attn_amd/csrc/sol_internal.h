@@ -140,14 +140,16 @@ struct QuantParams {
 // takes sol_attention_kernel.  Small launches leave most SIMDs idle, so their
 // time is one workgroup's tile chain: KS groups of two waves split it KS ways,
 // four while a CU holds one workgroup (at most kSmallBlocks query blocks), two
-// while it holds two.  A query-sink block's chain is every key block: with two
+// while it holds two, or for one or two key blocks at head_dim 128 (2 x 121 x 63
+// keys x 32 heads 20.9 -> 18.8 us a call, 1,000 x 128 x 8 17.0 -> 15.0, 128 x 128 x 8
+// 14.6 -> 14.8; at 64 four groups may pool the keys too).  A query-sink block's chain is every key block: with two
 // or more of them, over keys of more than kSmallChain steps, the launch goes
 // to the one-block kernel, whose sink tiles split over workgroups instead (a
 // single sink block is not split there).
 constexpr int64_t kSmallBlocks = 256;
 constexpr int64_t kSmallChain = 8;  // at head_dim 128; twice that at 64
 inline int small_key_split(int64_t blocks, int64_t nkb, int64_t q_sink_blocks, int64_t head_dim) {
-  const int ks = blocks <= kSmallBlocks ? 4 : 2;
+  const int ks = blocks <= kSmallBlocks && !(head_dim == 128 && nkb <= 2) ? 4 : 2;
   if (blocks > 2 * kSmallBlocks || nkb > kMaxKeyBlocks) return 0;
   return q_sink_blocks < 2 || nkb <= kSmallChain * ks * (128 / head_dim) ? ks : 0;
 }

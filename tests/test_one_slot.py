@@ -75,6 +75,19 @@ def test_early_local_blocks_of_small_launches(d, tq, tk, heads, monkeypatch):
         assert_close(small.cpu(), one.cpu())
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("tq,tk,heads", [(121, 63, 3), (64, 64, 2), (75, 75, 3), (300, 128, 2), (300, 129, 2)])
+def test_small_launches_of_one_or_two_key_blocks(d, tq, tk, heads, monkeypatch):
+    # Two key-split groups at head_dim 128 up to two blocks, with fewer blocks than groups.
+    print(f"short keys: D{d} Tq{tq} Tk{tk}", flush=True)
+    q, k, v = tensors(tq, tk, d, 2, heads, device="cuda", seed=12)
+    for local, beta in ((0, 1.0), (1, 0.0), (-1, math.inf)):
+        small, c0 = _launch(q, k, v, 0, monkeypatch, beta, local=local)
+        one, c1 = _launch(q, k, v, 1, monkeypatch, beta, local=local)
+        assert torch.equal(c0, c1)
+        assert_close(small.cpu(), one.cpu())
+
+
 def _windows(kind, n):
     rows = torch.stack((torch.arange(0, 200), torch.arange(500, 700)))
     if kind == "runs":         # every whole block consecutive
