@@ -230,7 +230,8 @@ int64_t sol_route_workspace_size(int64_t batch, int64_t query_tokens, int64_t ke
  * workgroup_form: 0 picks the schedule by launch size: launches at finite
  * or +INFINITY beta of at most 512 query blocks (over all entries and
  * heads) run one query block per workgroup with its key tiles split over 4
- * (at most 256 query blocks) or 2 groups of two waves, merged in LDS (outputs
+ * (at most 256 query blocks) or 2 (also for at most two key blocks at
+ * head_dim 128) groups of two waves, merged in LDS (outputs
  * agree with the other forms to rounding; decisions and counts are the
  * same), unless two or more query-sink blocks meet long keys
  * (small_key_split in csrc/sol_internal.h); otherwise one query block per
